@@ -46,11 +46,32 @@ __device__ __forceinline__ int wrapi(int v, int n) { return v < 0 ? v + n : (v >
 // field a, scale s and spectrum s_hat (group 0: every load shares design 0).
 __host__ __device__ __forceinline__ int design_of(int l, int group) { return group > 0 ? l / group : 0; }
 
-// Sum over the 64 lanes of a wavefront with a fixed butterfly order; every lane gets the total.
+// One 32-bit half of a lane permutation inside a row of 16 lanes (CTRL: a DPP control word).
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp(int(b), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(int(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned>(lo));
+}
+
+__device__ __forceinline__ double read_lane(double v, int lane) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane(int(b), lane);
+  const int hi = __builtin_amdgcn_readlane(int(b >> 32), lane);
+  return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned>(lo));
+}
+
+// Sum over the 64 lanes of a wavefront with a fixed order; every lane gets the total. All 64 lanes take part.
+// The four steps inside a row of 16 lanes are DPP moves of the vector unit (lane ^ 1, lane ^ 2, then the mirrors
+// of 8 and 16, which meet equal partial sums as lane ^ 4 and lane ^ 8 would), the four row sums scalar reads: a
+// tenth of the latency of six shuffles through the LDS unit, which every small launch paid several times in a row.
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+  v += dpp_move<0xB1>(v);   // quad_perm [1, 0, 3, 2]
+  v += dpp_move<0x4E>(v);   // quad_perm [2, 3, 0, 1]
+  v += dpp_move<0x141>(v);  // row_half_mirror
+  v += dpp_move<0x140>(v);  // row_mirror
+  return (read_lane(v, 0) + read_lane(v, 16)) + (read_lane(v, 32) + read_lane(v, 48));
 }
 
 // Block-wide sum with fixed order (lanes, then waves in index order). `scratch`
