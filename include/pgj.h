@@ -134,11 +134,13 @@ int pgj_hex8_set_shape(const pgj_grid* g, int L, int es, int R, int W, int ZC, i
  * multiply, 2 inverse y/x; plan 0 takes radix-4 stages first (64 = 4 x 4 x 4),
  * plan 1 radix-8 stages first (64 = 8 x 8); for the z pass at 64^3, plan 2
  * keeps the transforms in registers (two radix-8 passes with one LDS transpose
- * each, LDS otherwise only for the 3x3 Green multiply). plan -1 restores the
- * default, plan 0. The
+ * each, LDS otherwise only for the 3x3 Green multiply). plan -1 leaves the pass
+ * to the library's choice for that length (radix 8 first from 24 on, except the z
+ * pass at 48). The
  * choice holds for every later launch of that pass on any n^3 grid of that
  * precision (a graph keeps the kernels of its capture; a solver reads the plan
- * when it sets up its launches). get_plan writes the three passes' plans.
+ * when it sets up its launches). get_plan writes the three passes' plans, 0
+ * where none is set.
  * Counterpart of the reference's variant sweep
  * (solver/src/hex8_modal/gpu_study.py:174-222) for the FFT radix schedule. */
 int pgj_fft_set_plan(const pgj_grid* g, int es, int pass, int plan);

@@ -40,7 +40,7 @@ std::map<PlanKey, int> g_plans;
 int fft_plan(int n, int es, int pass) {
   std::lock_guard<std::mutex> lock(g_plan_mutex);
   auto it = g_plans.find(PlanKey(n, es, pass));
-  return it == g_plans.end() ? 0 : it->second;
+  return it == g_plans.end() ? -1 : it->second;
 }
 
 bool tuned_shape(const pgj_grid& g, int L, int es, int* R, int* W, int* ZC, int* plane) {
@@ -90,7 +90,7 @@ extern "C" int pgj_fft_set_plan(const pgj_grid* g, int es, int pass, int plan) {
 
 extern "C" int pgj_fft_get_plan(const pgj_grid* g, int es, int* out3) {
   PGJ_REQUIRE(g && (es == 4 || es == 8) && out3, "invalid FFT plan query");
-  for (int pass = 0; pass < 3; ++pass) out3[pass] = pgj::fft_plan(g->nx, es, pass);
+  for (int pass = 0; pass < 3; ++pass) out3[pass] = std::max(0, pgj::fft_plan(g->nx, es, pass));
   return PGJ_OK;
 }
 

@@ -699,6 +699,7 @@ extern "C" int pgj_scale_spectrum(const pgj_grid* g, const void* plan, const dou
     A.spec = static_cast<double2*>(s_hat);
     A.pr = reinterpret_cast<double*>(static_cast<char*>(ws) + pl.pr);
     A.pg = reinterpret_cast<double*>(static_cast<char*>(ws) + pl.pg);
+    zpass_choose(A, *g, 1);
     hipStream_t st = as_stream(stream);
     if (int e = launch_fxy_static(A, 1, kFxyScale, st)) return e;
     return launch_fz_static(A, 1, kFzScale, st);
@@ -732,6 +733,7 @@ extern "C" int pgj_precond_apply(const pgj_grid* g, int L, const void* plan, con
     A.pg = reinterpret_cast<double*>(w + pl.pg);
     A.zout = z;
     A.soa = 0;
+    zpass_choose(A, *g, L);
     if (int e = launch_fxy_static(A, L, kFxyPre, st)) return e;
     if (int e = launch_fz_static(A, L, kFzPre, st)) return e;
     return launch_fxyi_static(A, L, st, kFxyiPre);

@@ -47,7 +47,7 @@ struct Cube {
 // zero in LDS and skipped). 128^3 takes 13 columns in FP32 (104-byte runs
 // instead of 40) but keeps 5 in FP64, where 13 would need 147 VGPRs at 2 blocks
 // per CU; 17 columns at 96^3 measured no faster than 7. KCX > 0 overrides the
-// chunk width (the wide 64^3 FP64 instance, kWideKC).
+// chunk width (ZWidths).
 template <int N, typename R, int KCX = 0>
 struct ZPass {
   static constexpr int NKX = N / 2 + 1;
@@ -70,30 +70,42 @@ struct ZPass {
   using ZCols = Lines<3 * KC, KC, N * KC, 1, KC, true>;  // z transforms on (component, column)
 };
 
-// Wide z chunks: at 64^3 in FP64 the default 11 columns give 3 chunks per ky row
-// in 34 KiB of LDS (4 blocks per CU), 17 columns give 2 chunks in 52 KiB (3 per
-// CU), and the symbol and s_hat are read by 2 blocks per ky row instead of 3. A
-// 6-load launch is 1152 blocks against 1024 slots of 256 CUs with the default, a
-// partial second round, and 768 blocks in exactly one round with the wide
-// chunks: the pass takes 31 us instead of 39 us. Launches of many rounds (a
-// batched set of 72 loads) gain from the fewer re-reads; launches that fit one
-// round with the default (up to 5 loads) keep it, since a wide block does more
-// work in that single round. zpass_wide decides.
+// The kx chunk widths a z pass can run with (FFTArgs::zkc picks one per workspace, zpass_choose):
+// - wide, 64^3 FP64 from 6 loads on 256 CUs (zpass_wide): 17 columns in 52 KiB of LDS (3 blocks per CU) instead
+//   of 11 in 34 KiB (4 per CU). A 6-load launch is 768 blocks, exactly one round, instead of 1152 on 1024 slots:
+//   27 us against 33 us. Launches of many rounds gain from reading the symbol and s_hat in fewer blocks.
+// - narrow, where the default chunks give at most 2.5 blocks per CU (few loads on a small grid): the blocks are
+//   what hides the pass's latency there. Graph-replayed launches, radix 8 first, default against narrow:
+//   32^3 FP64 1 / 3 / 6 loads 10.1 / 10.5 / 11.2 -> 6.5 / 7.6 / 9.5 us, 24^3 8.6 / 8.7 / 9.0 -> 6.4 / 6.7 / 7.6,
+//   16^3 6.4 -> 5.8 (6 loads 6.5 -> 6.3), 64^3 1 / 3 loads 13.2 / 19.8 -> 10.9 / 19.5; FP32 alike. Above that the
+//   default is faster (64^3 FP32, 6 loads, 4.5 blocks per CU: 22.7 against 25.5 us). 48^3 already runs 5 columns
+//   (3: 13.6 against 11.6 us at 3 loads).
 template <int N, typename R>
-constexpr int kWideKC = N == 64 && sizeof(R) == 8 ? 17 : 0;
+struct ZWidths {
+  static constexpr int def = ZPass<N, R>::KC;
+  static constexpr int narrow = N == 16 ? 3 : N == 24 ? 5 : N == 32 ? 4 : N == 64 ? 4 : def;
+  static constexpr int wide = N == 64 && sizeof(R) == 8 ? 17 : def;
+};
+
+// Radix plan of a pass whose plan is not set (pgj_fft_set_plan), and of the passes outside the PCG iteration:
+// radix 8 first, one LDS stage less at 32 and 64 and 128. Graph-replayed 3-load launches, radix 4 first against
+// radix 8 first, fxy / fz / fxyi: 64^3 FP64 22.8 / 21.3 / 23.5 -> 20.9 / 19.8 / 22.5 us, 32^3 7.1 / 12.2 / 6.8 ->
+// 6.9 / 10.5 / 6.4, 128^3 FP32 85.5 / 99.0 / 104.4 -> 81.2 / 96.2 / 99.4. Radix 4 first stays where it is no
+// slower: 16 (4 x 4 against 8 x 2: 4.4 / 6.4 / 4.1 against 4.5 / 6.6 / 4.2) and the z pass at 48 (11.1 against 11.6).
+template <int N>
+constexpr int default_plan(int pass) {
+  return N == 16 || (N == 48 && pass == 1) ? 0 : 1;
+}
+
+template <int N, typename R>
+int plan_of(int pass) {
+  const int plan = fft_plan(N, int(sizeof(R)), pass);
+  return plan < 0 ? default_plan<N>(pass) : plan;
+}
 
 // Register-resident z pass of the 64^3 cube (fz64_reg below): blocks per load, which lay out its partials:
 // 4 chunks of 8 kx columns per ky row, then 8 blocks for the Nyquist column kx = 32 (8 ky rows each).
 constexpr int kZRegBlocks = 4 * 64 + 8;
-
-// Per-load partial slots written by the z pass variant (FFTArgs::zwide: 0 default chunks, 1 wide chunks,
-// kZReg the register-resident pass); fxy and fxyi reduce exactly these.
-template <int N, typename R>
-__host__ __device__ constexpr int z_slots(int variant) {
-  if (N == 64 && variant == kZReg) return kZRegBlocks;
-  return (kWideKC<N, R> > 0 && variant == 1 ? ZPass<N, R, (kWideKC<N, R> > 0 ? kWideKC<N, R> : 1)>::NKB
-                                            : ZPass<N, R>::NKB) * N;
-}
 
 // Global -> LDS copy of COUNT values in two phases, so that independent work
 // can run while the loads are in flight: load() issues every load of a thread
@@ -194,7 +206,7 @@ void fxy_static(FFTArgsT<R> A) {
       double pq, rz;
       // per-load partials are laid out with the geometry's chunk count (slices of a set are offset by it)
       wave_reduce_partials_2(A.ppq + int64_t(l) * A.ppq_stride, A.ppq_count, 1, A.pg + int64_t(l) * A.f.nkb * N * 4,
-                             z_slots<N, R>(A.zwide), 4, pq, rz);
+                             A.zslots, 4, pq, rz);
       const bool valid = isfinite(pq) && pq > 0.0 && isfinite(rz) && rz > 0.0;
       alpha = valid ? rz / pq : 0.0;
       if (threadIdx.x == 0 && z == 0 && c == 0) {
@@ -659,7 +671,7 @@ void fxyi_static(FFTArgsT<R> A) {
   StageIn<N, T, X> twl;
   in.load(A.spec + ((int64_t(l) * 3 + c) * N + z) * int64_t(N) * C::NKX, [](int e) { return e; });
   twl.load(A.twy, [](int e) { return e; });
-  const int NSLOT = z_slots<N, R>(A.zwide);
+  const int NSLOT = A.zslots;
   // per-load partials are laid out with the geometry's chunk count (slices of a set are offset by it)
   const double* pgl = A.pg + int64_t(l) * A.f.nkb * N * 4;
   // the output is the next direction p = z + beta p (z alone right after init or without a direction input)
@@ -800,15 +812,15 @@ int fxy_static_n(FFTArgsT<R>& A, int L, int mode, hipStream_t s) {
   dim3 grid(N, 3, L), block(C::TXY);
   switch (mode) {
     case kFxyScale:
-      if (int e = allow_lds_static(fxy_static<N, kFxyScale, R>, lds)) return e;
-      hipLaunchKernelGGL((fxy_static<N, kFxyScale, R>), grid, block, lds, s, A);
+      if (int e = allow_lds_static((fxy_static<N, kFxyScale, R, default_plan<N>(0)>), lds)) return e;
+      hipLaunchKernelGGL((fxy_static<N, kFxyScale, R, default_plan<N>(0)>), grid, block, lds, s, A);
       break;
     case kFxyPre:
-      if (int e = allow_lds_static(fxy_static<N, kFxyPre, R>, lds)) return e;
-      hipLaunchKernelGGL((fxy_static<N, kFxyPre, R>), grid, block, lds, s, A);
+      if (int e = allow_lds_static((fxy_static<N, kFxyPre, R, default_plan<N>(0)>), lds)) return e;
+      hipLaunchKernelGGL((fxy_static<N, kFxyPre, R, default_plan<N>(0)>), grid, block, lds, s, A);
       break;
     default:
-      if (fft_plan(N, int(sizeof(R)), 0) == 1) {
+      if (plan_of<N, R>(0) == 1) {
         if (int e = allow_lds_static(fxy_static<N, kFxyPCG, R, 1>, lds)) return e;
         hipLaunchKernelGGL((fxy_static<N, kFxyPCG, R, 1>), grid, block, lds, s, A);
       } else {
@@ -829,19 +841,19 @@ int fz_static_kc(FFTArgsT<R>& A, int L, int mode, hipStream_t s) {
   dim3 grid(N, Z::NKB, L), block(Z::TZ);
   switch (mode) {
     case kFzScale:
-      if (int e = allow_lds_static(fz_static<N, kFzScale, R, KCX>, lds)) return e;
-      hipLaunchKernelGGL((fz_static<N, kFzScale, R, KCX>), grid, block, lds, s, A);
+      if (int e = allow_lds_static(fz_static<N, kFzScale, R, KCX, default_plan<N>(1)>, lds)) return e;
+      hipLaunchKernelGGL((fz_static<N, kFzScale, R, KCX, default_plan<N>(1)>), grid, block, lds, s, A);
       break;
     case kFzPre:
-      if (int e = allow_lds_static(fz_static<N, kFzPre, R, KCX>, lds)) return e;
-      hipLaunchKernelGGL((fz_static<N, kFzPre, R, KCX>), grid, block, lds, s, A);
+      if (int e = allow_lds_static(fz_static<N, kFzPre, R, KCX, default_plan<N>(1)>, lds)) return e;
+      hipLaunchKernelGGL((fz_static<N, kFzPre, R, KCX, default_plan<N>(1)>), grid, block, lds, s, A);
       break;
     case kFzInit:
-      if (int e = allow_lds_static(fz_static<N, kFzInit, R, KCX>, lds)) return e;
-      hipLaunchKernelGGL((fz_static<N, kFzInit, R, KCX>), grid, block, lds, s, A);
+      if (int e = allow_lds_static(fz_static<N, kFzInit, R, KCX, default_plan<N>(1)>, lds)) return e;
+      hipLaunchKernelGGL((fz_static<N, kFzInit, R, KCX, default_plan<N>(1)>), grid, block, lds, s, A);
       break;
     default:
-      if (fft_plan(N, int(sizeof(R)), 1) == 1) {
+      if (plan_of<N, R>(1) == 1) {
         if (int e = allow_lds_static(fz_static<N, kFzPCG, R, KCX, 1>, lds)) return e;
         hipLaunchKernelGGL((fz_static<N, kFzPCG, R, KCX, 1>), grid, block, lds, s, A);
       } else {
@@ -871,13 +883,17 @@ int fz64_reg_launch(FFTArgsT<R>& A, int L, int mode, hipStream_t s) {
 
 template <int N, typename R>
 int fz_static_n(FFTArgsT<R>& A, int L, int mode, hipStream_t s) {
+  using W = ZWidths<N, R>;
   if constexpr (N == 64) {
-    if (A.zwide == kZReg) return fz64_reg_launch<R>(A, L, mode, s);
+    if (A.zkc == 0) return fz64_reg_launch<R>(A, L, mode, s);
   }
-  if constexpr (kWideKC<N, R> > 0) {
-    if (A.zwide == 1) return fz_static_kc<N, R, kWideKC<N, R>>(A, L, mode, s);
+  if constexpr (W::wide != W::def) {
+    if (A.zkc == W::wide) return fz_static_kc<N, R, W::wide>(A, L, mode, s);
   }
-  return fz_static_kc<N, R, 0>(A, L, mode, s);
+  if constexpr (W::narrow != W::def) {
+    if (A.zkc == W::narrow) return fz_static_kc<N, R, W::narrow>(A, L, mode, s);
+  }
+  return fz_static_kc<N, R, W::def>(A, L, mode, s);
 }
 
 // CUs of the current device, cached per device; 0 if the query fails.
@@ -901,10 +917,36 @@ bool zpass_wide(const pgj_grid& g, int L, int es) {
   return cus > 0 && narrow > cus * Zn::per_cu;
 }
 
-int zpass_variant(const pgj_grid& g, int L, int es) {
-  if (static_cube(g) && g.nx == 64 && fft_plan(64, es, 1) == 2) return kZReg;
-  return zpass_wide(g, L, es) ? 1 : 0;
+template <int N, typename R>
+static int zkc_of(const pgj_grid& g, int L) {
+  using W = ZWidths<N, R>;
+  if (N == 64 && fft_plan(64, int(sizeof(R)), 1) == 2) return 0;
+  if (W::wide != W::def && zpass_wide(g, L, int(sizeof(R)))) return W::wide;
+  if (W::narrow != W::def && 2 * int64_t(ZPass<N, R>::NKB) * N * L <= 5 * int64_t(device_cus())) return W::narrow;
+  return W::def;
 }
+
+template <typename R>
+void zpass_choose(FFTArgsT<R>& A, const pgj_grid& g, int L) {
+  if (!static_cube(g)) {
+    A.zkc = A.f.kc;
+    A.zslots = A.f.nkb * g.ny;
+    return;
+  }
+  switch (g.nx) {
+    case 16: A.zkc = zkc_of<16, R>(g, L); break;
+    case 24: A.zkc = zkc_of<24, R>(g, L); break;
+    case 32: A.zkc = zkc_of<32, R>(g, L); break;
+    case 48: A.zkc = zkc_of<48, R>(g, L); break;
+    case 64: A.zkc = zkc_of<64, R>(g, L); break;
+    case 96: A.zkc = zkc_of<96, R>(g, L); break;
+    default: A.zkc = zkc_of<128, R>(g, L); break;
+  }
+  const int nkx = g.nx / 2 + 1;
+  A.zslots = A.zkc == 0 ? kZRegBlocks : ((nkx + A.zkc - 1) / A.zkc) * g.nx;
+}
+template void zpass_choose<double>(FFTArgsT<double>&, const pgj_grid&, int);
+template void zpass_choose<float>(FFTArgsT<float>&, const pgj_grid&, int);
 
 }  // namespace pgj
 
@@ -919,9 +961,9 @@ int fxyi_static_n(FFTArgsT<R>& A, int L, int mode, hipStream_t s) {
   using C = Cube<N>;
   const size_t lds = C::lds_xy(sizeof(cplx<R>));
   if (mode == kFxyiPre) {
-    if (int e = allow_lds_static(fxyi_static<N, kFxyiPre, R>, lds)) return e;
-    hipLaunchKernelGGL((fxyi_static<N, kFxyiPre, R>), dim3(N, 3, L), dim3(C::TXY), lds, s, A);
-  } else if (fft_plan(N, int(sizeof(R)), 2) == 1) {
+    if (int e = allow_lds_static(fxyi_static<N, kFxyiPre, R, default_plan<N>(2)>, lds)) return e;
+    hipLaunchKernelGGL((fxyi_static<N, kFxyiPre, R, default_plan<N>(2)>), dim3(N, 3, L), dim3(C::TXY), lds, s, A);
+  } else if (plan_of<N, R>(2) == 1) {
     if (int e = allow_lds_static(fxyi_static<N, kFxyiPCG, R, 1>, lds)) return e;
     hipLaunchKernelGGL((fxyi_static<N, kFxyiPCG, R, 1>), dim3(N, 3, L), dim3(C::TXY), lds, s, A);
   } else {

@@ -37,8 +37,8 @@ struct RowMarch {
 bool tuned_shape(const pgj_grid& g, int L, int es, int* R, int* W, int* ZC, int* plane);
 
 // Radix plan of the compile-time FFT pass `pass` (0 forward xy, 1 z with the Green multiply, 2 inverse xy) of
-// the PCG iteration on an n^3 cube in precision es: 0 (radix 4 first, the default) or 1 (radix 8 first); set by
-// pgj_fft_set_plan (the autotuner) and read at every launch of that pass.
+// the PCG iteration on an n^3 cube in precision es: 0 (radix 4 first), 1 (radix 8 first), -1 (not set: the
+// library's choice); set by pgj_fft_set_plan (the autotuner) and read at every launch of that pass.
 int fft_plan(int n, int es, int pass);
 
 // Shape preferences (R, W, ZC) for L loads per launch. ZC (planes marched by
@@ -188,15 +188,15 @@ inline FFTGeom fft_geom(const pgj_grid& g) {
   int kc = 1;
   while (kc < f.nkx && size_t(kc + 1) * col + 64 * 8 <= 56 * 1024) ++kc;
   if (g.nx == g.ny && g.ny == g.nz) {
-    // cubes: at least as many chunks as the compile-time kernels use (fft_static.hip, ZPass<N, R>::NKB; at 64^3
-    // 5 x 64 rows for the 264 blocks of the register-resident pass), so the per-block partials laid out with
-    // nkb below hold every kind of z pass
+    // cubes: as many chunks as the narrowest compile-time z pass uses (fft_static.hip, ZWidths; at 64^3 also more
+    // rows than the 264 blocks of the register-resident pass), so the per-block partials laid out with nkb below
+    // hold every kind of z pass
     switch (g.nx) {
-      case 16: kc = 9; break;
-      case 24: kc = 13; break;
-      case 32: kc = 17; break;
+      case 16: kc = 3; break;
+      case 24: kc = 5; break;
+      case 32: kc = 4; break;
       case 48: kc = 5; break;
-      case 64: kc = 7; break;
+      case 64: kc = 4; break;
       case 96: kc = 7; break;
       case 128: kc = 5; break;
       default: break;

@@ -131,6 +131,7 @@ extern "C" int pgj_precond_apply_mixed(const pgj_grid* g, int L, const void* pla
   A.pg = reinterpret_cast<double*>(w + pl.pg);
   A.zout64 = z;
   A.soa = 0;
+  zpass_choose(A, *g, L);
   hipStream_t st = as_stream(stream);
   if (int e = launch_fxy_static(A, L, kFxyPre, st)) return e;
   if (int e = launch_fz_static(A, L, kFzPre, st)) return e;

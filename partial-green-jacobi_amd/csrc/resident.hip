@@ -213,7 +213,7 @@ int resident_init_t(const pgj_grid* g, int L, int group, int l0, int nl, FFTArgs
   A.st = state_view(state, L, l0);
   A.soa = 1;
   A.group = group;
-  A.zwide = zpass_variant(*g, L, int(sizeof(T)));  // from the workspace's load count: every slice agrees
+  zpass_choose(A, *g, L);  // from the workspace's load count: every slice agrees
   if (int e = fxy(A, *g, nl, kFxyPre, s)) return e;
   if (int e = fz(A, *g, nl, kFzInit, s)) return e;
   return fxyi(A, *g, nl, s);
@@ -256,7 +256,7 @@ int resident_stage_t(const pgj_grid* g, int L, int group, int l0, int nl, FFTArg
   F.st = st;
   F.soa = 1;
   F.group = group;
-  F.zwide = zpass_variant(*g, L, int(sizeof(T)));
+  zpass_choose(F, *g, L);
   if (stage == 0) {
     if constexpr (sizeof(T) == 8) {
       if (c21) return launch_c21_pcg(*g, nl, c21->pool, c21->index, p + v, st.active, q + v, b.ppq, F.ppq_stride, s);
@@ -283,6 +283,7 @@ extern "C" int pgj_resident_scale(const pgj_grid* g, const void* plan, const dou
   if (int e = launch_scale(*g, a, alpha, nullptr, sc, b.pcert, 1, s)) return e;
   FFTArgs A = fft_args(*g, plan);
   A.s = sc; A.spec = static_cast<double2*>(s_hat); A.pr = b.pr; A.pg = b.pg; A.soa = 1;
+  zpass_choose(A, *g, 1);
   if (int e = fxy(A, *g, 1, kFxyScale, s)) return e;
   return fz(A, *g, 1, kFzScale, s);
 }
@@ -296,6 +297,7 @@ extern "C" int pgj_resident_scale_dev(const pgj_grid* g, const void* plan, const
   if (int e = launch_scale(*g, a, 0.0, nullptr, sc, b.pcert, 1, s, alpha)) return e;
   FFTArgs A = fft_args(*g, plan);
   A.s = sc; A.spec = static_cast<double2*>(s_hat); A.pr = b.pr; A.pg = b.pg; A.soa = 1;
+  zpass_choose(A, *g, 1);
   if (int e = fxy(A, *g, 1, kFxyScale, s)) return e;
   return fz(A, *g, 1, kFzScale, s);
 }
