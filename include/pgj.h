@@ -363,6 +363,27 @@ int pgj_cone_candidate(int n, const double* x, const double* ratio, const double
  * pgj_cone_project's ws) with relative stop 1e-4; bounds[3] counts steps.
  * Replaces `bisect` (outer.cu:35-39). */
 int pgj_cone_bisect(int n, const double* ws, double* bounds, double volume, void* stream);
+/* The same filter, projection, gradient and bisection as fused passes, for
+ * stencils whose offsets are at most `reach` in every direction, reach <=
+ * pgj_cone_max_reach(): a tile and its halo are staged in LDS once, and a
+ * bisection round is one launch. Same terms and order per sum.
+ * physical: t = filter(x), then ph, dp, a of its projection.
+ * gradient: g = filter(dp (3 (1-Emin) ph^2) e / hs) / n^3, dv = filter(dp / hs),
+ * ratio = -g/dv, root (2 n^3 doubles) = ratio^0.3 as unevaluated (hi, lo)
+ * sums, bounds = [0, 1e9, 1, 0].
+ * rounds: `rounds` bisection steps on `bounds` (none once bounds[2] == 0); y is
+ * the last candidate. ws: pgj_cone_rounds_ws_bytes(n) bytes. */
+int pgj_cone_max_reach(void);
+size_t pgj_cone_rounds_ws_bytes(int n);
+int pgj_cone_physical(int n, const double* x, const int32_t* offsets, const double* weights, int m, int reach,
+                      const double* hs, double beta, double eta, double emin, double* t, double* ph, double* dp,
+                      double* a, void* stream);
+int pgj_cone_gradient(int n, const double* dp, const double* ph, const double* energy, const double* hs,
+                      const int32_t* offsets, const double* weights, int m, int reach, double emin, double* g,
+                      double* dv, double* ratio, double* root, double* bounds, void* stream);
+int pgj_cone_rounds(int n, const double* x, const double* root, const int32_t* offsets, const double* weights,
+                    int m, int reach, const double* hs, double beta, double eta, double move, double volume,
+                    int rounds, double* y, double* bounds, double* ws, void* stream);
 /* out[0] = max |a - b| (the design change). */
 int pgj_absmax_diff(int n, const double* a, const double* b, double* ws, double* out, void* stream);
 
@@ -386,6 +407,16 @@ int pgj_gauss_candidate(int n, const double* x, const double* ratio, const doubl
                         void* stream);
 /* bisection on the mean of the projected candidate (outer.cu:30-33). */
 int pgj_gauss_bisect(int n, const double* ws, double* bounds, double volume, void* stream);
+/* `rounds` bisection steps on `bounds`, two launches each (candidate and z pass;
+ * y and x passes, projection and volume partials); y is the last candidate, tmp
+ * one field of scratch, ws pgj_gauss_rounds_ws_bytes(n) bytes. Grids and radii
+ * for which pgj_gauss_fused is 1 (the staged lines fit LDS: n up to about 128
+ * with the radius of the Study-I filter); others return PGJ_ERR_ARG. */
+int pgj_gauss_fused(int n, int radius);
+size_t pgj_gauss_rounds_ws_bytes(int n);
+int pgj_gauss_rounds(int n, const double* x, const double* ratio, const double* weights, int radius, double* tmp,
+                     double beta, double move, double volume, int rounds, double* y, double* bounds, double* ws,
+                     void* stream);
 
 /* --------------------------------------------- generic batched PCG vectors */
 /* Vector side of the operator-agnostic best-iterate PCG on B batches of n

@@ -114,6 +114,18 @@ SIGNATURES = {
     'pgj_gauss_ratio': (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     'pgj_gauss_candidate': (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_double, c_void_p, c_void_p]),
     'pgj_gauss_bisect': (c_int, [c_int, c_void_p, c_void_p, c_double, c_void_p]),
+    'pgj_cone_max_reach': (c_int, []),
+    'pgj_cone_rounds_ws_bytes': (c_size_t, [c_int]),
+    'pgj_cone_physical': (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_double, c_double,
+                                  c_double, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    'pgj_cone_gradient': (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int,
+                                  c_double, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    'pgj_cone_rounds': (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_double,
+                                c_double, c_double, c_double, c_int, c_void_p, c_void_p, c_void_p, c_void_p]),
+    'pgj_gauss_fused': (c_int, [c_int, c_int]),
+    'pgj_gauss_rounds_ws_bytes': (c_size_t, [c_int]),
+    'pgj_gauss_rounds': (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_double, c_double, c_double,
+                                 c_int, c_void_p, c_void_p, c_void_p, c_void_p]),
     'pgj_plan32_bytes': (c_size_t, [GP]),
     'pgj_plan32_init': (c_int, [GP, c_void_p, c_void_p, c_void_p]),
     'pgj_to_f32': (c_int, [c_int64, c_void_p, c_void_p, c_void_p]),

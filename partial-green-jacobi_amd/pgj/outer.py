@@ -68,6 +68,11 @@ class PaperOuter(_Fields):
         self._alloc(n, ['x', 'ph', 'dp', 'a', 'energy', 'new', 'g', 'dv', 'ratio', 't', 'hs', 'trial_ph',
                         'trial_dp', 'trial_a', 'tmp'], device)
         self.bounds = torch.zeros(4, dtype=torch.float64, device=device)
+        lib = _lib.lib()
+        self.reach = max(0, math.ceil(rmin) - 1)
+        self.fused = self.reach <= lib.pgj_cone_max_reach()   # wider stencils: one launch per filter, projection, ...
+        self.rounds_ws = torch.empty(lib.pgj_cone_rounds_ws_bytes(n) // 8, dtype=torch.float64, device=device)
+        self.root = torch.empty(2 * n ** 3 if self.fused else 0, dtype=torch.float64, device=device)
         self.raw_filter(torch.ones_like(self.x), self.hs)
         self.physical_graph = self.prepare_graph = self.bisect_graph = None
 
@@ -81,10 +86,23 @@ class PaperOuter(_Fields):
                   _lib.ptr(self.ws) if volume else None, _lib.stream())
 
     def physical(self):
+        if self.fused:
+            _lib.call('pgj_cone_physical', self.n, _lib.ptr(self.x), *self._stencil(), _lib.ptr(self.hs), self.beta,
+                      self.eta, self.emin, _lib.ptr(self.t), _lib.ptr(self.ph), _lib.ptr(self.dp), _lib.ptr(self.a),
+                      _lib.stream())
+            return
         self.raw_filter(self.x, self.t)
         self.project(self.t, self.ph, self.dp, self.a)
 
+    def _stencil(self):
+        return _lib.ptr(self.offsets), _lib.ptr(self.weights), len(self.weights), self.reach
+
     def _prepare(self):
+        if self.fused:
+            _lib.call('pgj_cone_gradient', self.n, _lib.ptr(self.dp), _lib.ptr(self.ph), _lib.ptr(self.energy),
+                      _lib.ptr(self.hs), *self._stencil(), self.emin, _lib.ptr(self.g), _lib.ptr(self.dv),
+                      _lib.ptr(self.ratio), _lib.ptr(self.root), _lib.ptr(self.bounds), _lib.stream())
+            return
         _lib.call('pgj_cone_sensitivity', self.n, _lib.ptr(self.dp), _lib.ptr(self.ph), _lib.ptr(self.energy),
                   _lib.ptr(self.hs), self.emin, _lib.ptr(self.tmp), _lib.ptr(self.new), _lib.stream())
         self.raw_filter(self.tmp, self.g)
@@ -93,6 +111,11 @@ class PaperOuter(_Fields):
                   _lib.ptr(self.bounds), _lib.stream())
 
     def _bisect_chunk(self):
+        if self.fused:
+            _lib.call('pgj_cone_rounds', self.n, _lib.ptr(self.x), _lib.ptr(self.root), *self._stencil(),
+                      _lib.ptr(self.hs), self.beta, self.eta, self.move, self.volume, self.chunk, _lib.ptr(self.new),
+                      _lib.ptr(self.bounds), _lib.ptr(self.rounds_ws), _lib.stream())
+            return
         for _ in range(self.chunk):
             _lib.call('pgj_cone_candidate', self.n, _lib.ptr(self.x), _lib.ptr(self.ratio), _lib.ptr(self.bounds),
                       self.move, _lib.ptr(self.new), _lib.stream())
@@ -165,6 +188,9 @@ class GaussianOuter(_Fields):
                         'trial_dp', 'trial_a', 'gin'], device)
         self.beta = 1.0
         self.bounds = torch.zeros(2, dtype=torch.float64, device=device)
+        lib = _lib.lib()
+        self.fused = bool(lib.pgj_gauss_fused(n, self.radius))
+        self.rounds_ws = torch.empty(lib.pgj_gauss_rounds_ws_bytes(n) // 8, dtype=torch.float64, device=device)
         self.physical_graph = self.update_graph = None
 
     def gaussian(self, x, out):
@@ -186,6 +212,12 @@ class GaussianOuter(_Fields):
         self.gaussian(self.dp, self.dv)
         _lib.call('pgj_gauss_ratio', self.n, _lib.ptr(self.g), _lib.ptr(self.dv), _lib.ptr(self.ratio),
                   _lib.ptr(self.ws), _lib.ptr(self.bounds), _lib.stream())
+        if self.fused and self.bisections > 0:
+            _lib.call('pgj_gauss_rounds', self.n, _lib.ptr(self.x), _lib.ptr(self.ratio), _lib.ptr(self.weights),
+                      self.radius, _lib.ptr(self.tmp1), float(beta), self.move, self.volume, self.bisections,
+                      _lib.ptr(self.new), _lib.ptr(self.bounds), _lib.ptr(self.rounds_ws), _lib.stream())
+            self._change()
+            return
         for _ in range(self.bisections):
             _lib.call('pgj_gauss_candidate', self.n, _lib.ptr(self.x), _lib.ptr(self.ratio), _lib.ptr(self.bounds),
                       self.move, _lib.ptr(self.new), _lib.stream())
