@@ -3,6 +3,7 @@
 // mean stress, nodal diagonal / partial Green-Jacobi scale and projection.
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 
 #include "hex8_kernels.h"
 
@@ -403,54 +404,126 @@ __global__ __launch_bounds__(MAXT) void hex8_rowmarch(RowArgsT<T> A) {
   }
 }
 
-template <bool CUBIC, bool CERT>
-__global__ __launch_bounds__(256) void hex8_reference(RefArgs A) {
+// The 24x24 element stiffness of C0 by its tensor-product form, independent of the modal form of the other kernels.
+// The integrals over the element factor into per-axis ones: stiffness (s s' / h), mass (h / 3 on equal, h / 6 on
+// different ends) and mixed (s / 2, whatever the other end), with s = -1 or +1 the node's end of the axis. So
+//   K_ii(n, m) = diag[i][n ^ m],  K_ij(n, m) = (lam s_i(n) s_j(m) + mu s_j(n) s_i(m)) off[k][bit k of n ^ m]
+// (i != j, k the third axis): 36 numbers, all held in scalar registers.
+struct RefStiffness {
+  double diag[3][8];
+  double off_sum[3][2], off_diff[3][2];   // (lam + mu) and (lam - mu) times the mixed integral
+};
+
+// Certification apply. A thread owns the column of nodes (x, y) over ZC planes and marches them: it loads each plane's
+// 3 x 3 neighbours once and adds their 3x3 blocks to the forces of the four elements of the layer below (as its top
+// corners) and of the layer above (as its bottom corners) on the layer's two nodes of the column: 576 FMAs and 31 loads
+// per node, with nine fixed offsets per thread. The form before evaluated eight whole elements per node for 3 of their
+// 24 forces each, 2700 flops and 192 loads: 64^3, six loads, 205 us against 75, 128^3 1590 against 430.
+// I: unsigned where the byte offsets of a vector fit 32 bits (uniform base + 32-bit offset), else int64_t.
+template <bool CERT, typename I>
+__global__ __launch_bounds__(256) void hex8_reference(RefArgs A, RefStiffness K, int ZC) {
   __shared__ double red[8];
   const int l = blockIdx.y;
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t base = int64_t(l) * 3 * A.N;
+  const int64_t P = int64_t(A.nx) * A.ny;
+  const int64_t id = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int z0 = int(id / P) * ZC, z1 = min(z0 + ZC, A.nz);
   double res2 = 0.0;
-  if (i < A.N) {
-    const int x = int(i % A.nx), y = int((i / A.nx) % A.ny), z = int(i / (int64_t(A.nx) * A.ny));
-    double acc[3] = {0.0, 0.0, 0.0};
-    // one element at a time (unrolling the eight elements spills); the node's
-    // local index in element o is o, selected with static register indices
+  if (z0 < A.nz) {
+    const int col = int(id % P), x = col % A.nx, y = col / A.nx;
+    const int xs[3] = {wrapi(x - 1, A.nx), x, wrapi(x + 1, A.nx)};
+    const int ys[3] = {wrapi(y - 1, A.ny), y, wrapi(y + 1, A.ny)};
+    const double* __restrict__ mat = A.a + int64_t(design_of(l, A.group)) * A.N;
+    const double* __restrict__ u = A.u + int64_t(l) * 3 * A.N;
+    const double* __restrict__ rhs = CERT ? A.rhs + int64_t(l) * 3 * A.N : nullptr;
+    double* __restrict__ out = A.out + int64_t(l) * 3 * A.N;
+    const I cs = A.soa ? I(A.N) : I(1), ns = A.soa ? I(1) : I(3);   // strides of components and nodes
+    double v[3][3][3];            // a plane's neighbours [y][x][component]
+    double bot[4][3], top[4][3];  // forces, for a = 1, of the layer's elements on its bottom and top node of the column
+    double carry[3] = {0.0, 0.0, 0.0};
+    // contributions of the plane at the layer's z corner ZM to the layer's node at z corner ZN
+    auto add = [&](auto zm, auto zn, double (&f)[4][3]) {
+      constexpr int ZM = decltype(zm)::value, ZN = decltype(zn)::value;
+#pragma unroll
+      for (int py = 0; py < 3; ++py)
+#pragma unroll
+        for (int px = 0; px < 3; ++px)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            // element e lies on the minus side of an axis where its bit is set; the node is its corner of those bits
+            const int ox = px - 1 + (e & 1), oy = py - 1 + (e >> 1);
+            if (ox < 0 || ox > 1 || oy < 0 || oy > 1) continue;
+            const int n = e | ZN << 2, m = ox | oy << 1 | ZM << 2, df = n ^ m;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) f[e][a] = fma(K.diag[a][df], v[py][px][a], f[e][a]);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+              // the two axes (a, b) other than k; K_ab = lam s_a(n) s_b(m) + mu s_b(n) s_a(m): equal signs or opposite
+              const int a = (k + 1) % 3, b = (k + 2) % 3, kb = (df >> k) & 1;
+              const bool p = ((n >> a) & 1) == ((m >> b) & 1), q = ((n >> b) & 1) == ((m >> a) & 1);
+              const double same = p ? K.off_sum[k][kb] : -K.off_sum[k][kb];
+              const double kab = p == q ? same : (p ? K.off_diff[k][kb] : -K.off_diff[k][kb]);
+              const double kba = p == q ? same : (q ? K.off_diff[k][kb] : -K.off_diff[k][kb]);
+              f[e][a] = fma(kab, v[py][px][b], f[e][a]);
+              f[e][b] = fma(kba, v[py][px][a], f[e][b]);
+            }
+          }
+    };
+    using Z0 = std::integral_constant<int, 0>;
+    using Z1 = std::integral_constant<int, 1>;
+    I at[3][3];
+#pragma unroll
+    for (int py = 0; py < 3; ++py)
+#pragma unroll
+      for (int px = 0; px < 3; ++px) at[py][px] = I(ys[py]) * I(A.nx) + I(xs[px]);
 #pragma unroll 1
-    for (int o = 0; o < 8; ++o) {
-      const int ex = wrapi(x - (o & 1), A.nx), ey = wrapi(y - ((o >> 1) & 1), A.ny),
-                ez = wrapi(z - ((o >> 2) & 1), A.nz);
-      double ue[24], fe[24];
+    for (int z = z0 - 1; z <= z1; ++z) {
+      const I plane = I(wrapi(z, A.nz)) * I(P), below = I(wrapi(z - 1, A.nz)) * I(P);
 #pragma unroll
-      for (int n = 0; n < 8; ++n) {
-        const int nxp = wrapi(ex + (n & 1), A.nx), nyp = wrapi(ey + ((n >> 1) & 1), A.ny),
-                  nzp = wrapi(ez + ((n >> 2) & 1), A.nz);
-        const int64_t node = (int64_t(nzp) * A.ny + nyp) * A.nx + nxp;
+      for (int py = 0; py < 3; ++py)
 #pragma unroll
-        for (int d = 0; d < 3; ++d) ue[3 * n + d] = A.u[A.soa ? (int64_t(l) * 3 + d) * A.N + node : base + 3 * node + d];
-      }
-      const double ae = A.a[int64_t(design_of(l, A.group)) * A.N + (int64_t(ez) * A.ny + ey) * A.nx + ex];
-      hex8_element<CUBIC>(ue, ae, A.coef, fe);
+        for (int px = 0; px < 3; ++px)
 #pragma unroll
-      for (int k = 0; k < 8; ++k)
-        if (k == o) {
+          for (int d = 0; d < 3; ++d) v[py][px][d] = u[ns * (plane + at[py][px]) + cs * I(d)];
+      if (z >= z0) {
+        double ae[4];
 #pragma unroll
-          for (int d = 0; d < 3; ++d) acc[d] += fe[3 * k + d];
+        for (int e = 0; e < 4; ++e) ae[e] = mat[below + at[1 - (e >> 1)][1 - (e & 1)]];
+        add(Z1{}, Z0{}, bot);
+        add(Z1{}, Z1{}, top);
+        if (z > z0) {
+#pragma unroll
+          for (int d = 0; d < 3; ++d) {
+            double acc = carry[d];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc = fma(ae[e], bot[e][d], acc);
+            const I idx = ns * (below + at[1][1]) + cs * I(d);
+            if (CERT) {
+              const double r = rhs[idx] - acc;
+              out[idx] = r;
+              res2 = fma(r, r, res2);
+            } else {
+              out[idx] = acc;
+            }
+          }
         }
-    }
-    for (int d = 0; d < 3; ++d) {
-      const int64_t idx = A.soa ? (int64_t(l) * 3 + d) * A.N + i : base + 3 * i + d;
-      if (CERT) {
-        const double r = A.rhs[idx] - acc[d];
-        A.out[idx] = r;
-        res2 = fma(r, r, res2);
-      } else {
-        A.out[idx] = acc[d];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          carry[d] = 0.0;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) carry[d] = fma(ae[e], top[e][d], carry[d]);
+        }
       }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) bot[e][d] = top[e][d] = 0.0;
+      add(Z0{}, Z0{}, bot);
+      add(Z0{}, Z1{}, top);
     }
   }
   if (CERT) {
     const double t = block_sum(res2, red);
-    if (threadIdx.x == 0) A.pres[(int64_t(l) * gridDim.x + blockIdx.x) * 4 + 3] = t;
+    if (threadIdx.x == 0) A.pres[(int64_t(l) * A.pres_rows + blockIdx.x) * 4 + 3] = t;
   }
 }
 
@@ -474,11 +547,15 @@ __global__ __launch_bounds__(256) void component_sums(const double* v, int64_t N
 
 // v -= mean per load/component (mean from component_sums partials; the first
 // wave reduces them in a fixed order and shares the result through LDS).
+// FINISHED: component_means has left the means in the load's first partial row.
+template <bool FINISHED>
 __global__ __launch_bounds__(256) void subtract_mean(double* v, int64_t N, const double* part, int nblk, int soa) {
   __shared__ double mean[3];
   const int l = blockIdx.y;
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (threadIdx.x < 64) {
+  if (FINISHED) {
+    if (threadIdx.x < 3) mean[threadIdx.x] = part[int64_t(l) * nblk * 4 + threadIdx.x];
+  } else if (threadIdx.x < 64) {
     const double* p = part + int64_t(l) * nblk * 4;
     for (int d = 0; d < 3; ++d) {
       const double s = wave_reduce_partials(p + d, nblk, 4);
@@ -488,6 +565,19 @@ __global__ __launch_bounds__(256) void subtract_mean(double* v, int64_t N, const
   __syncthreads();
   if (i < N)
     for (int d = 0; d < 3; ++d) v[lidx(soa, l, d, i, N)] -= mean[d];
+}
+
+// The three means of load blockIdx.x into slots 0..2 of its first partial row, which only this block reads.
+__global__ __launch_bounds__(256) void component_means(int64_t N, double* part, int nblk) {
+  __shared__ double red[12];
+  double* p = part + int64_t(blockIdx.x) * nblk * 4;
+  double s[3] = {0.0, 0.0, 0.0};
+#pragma unroll 4
+  for (int b = threadIdx.x; b < nblk; b += 256)
+    for (int d = 0; d < 3; ++d) s[d] += p[int64_t(b) * 4 + d];
+  block_sums<3>(s, red);
+  if (threadIdx.x == 0)
+    for (int d = 0; d < 3; ++d) p[d] = s[d] / double(N);
 }
 
 // AoS (L, N, 3) <-> SoA (L, 3, N)
@@ -579,54 +669,56 @@ __global__ __launch_bounds__(256) void hex8_energy_kernel(int nz, int ny, int nx
   out[int64_t(l) * N + e] = en / c.vol;
 }
 
-// C^H partials: per block the 21 upper-triangle sums of a_e (Ke v_i) . v_j / V.
+// C^H partials: per block the 21 upper-triangle sums of a_e (Ke v_i) . v_j / V over 256 elements, 32 at a time. Thread
+// (load i, element) gathers v_i, evaluates Ke v_i once and shares v_i through LDS; the pairs (i, i + 0..3 mod 6) are
+// its dot products (i + 3 for i < 3), which covers every pair once. One thread per element with all pairs gathered the
+// element's displacements 27 times (64^3: 88 us, 128^3 670 us).
+constexpr int kEffElements = 32, kEffThreads = 6 * kEffElements;
+
 template <bool CUBIC>
-__global__ __launch_bounds__(256) void effective_partials(int nz, int ny, int nx, ElementCoef c, const double* a,
-                                                          const double* u6, double* part) {
-  __shared__ double red[21][4];
+__global__ __launch_bounds__(kEffThreads) void effective_partials(int nz, int ny, int nx, ElementCoef c, const double* a,
+                                                                  const double* u6, double* part) {
+  __shared__ double v[6][24][kEffElements];
   const int64_t N = int64_t(nx) * ny * nz;
-  const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  double s[21];
+  const int i = threadIdx.x / kEffElements, k = threadIdx.x % kEffElements;
+  double m[6], s[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-  for (int k = 0; k < 21; ++k) s[k] = 0.0;
-  if (e < N) {
-    const int x = int(e % nx), y = int((e / nx) % ny), z = int(e / (int64_t(nx) * ny));
-    const double ae = a[e];
-    int idx = 0;
-    for (int i = 0; i < 6; ++i) {
-      double m[6] = {0, 0, 0, 0, 0, 0};
-      m[i] = 1.0;
-      double vi[24], fi[24], chi[24];
-      gather_element(u6 + int64_t(i) * 3 * N, nz, ny, nx, x, y, z, vi);
-      affine_local(m, c, chi);
+  for (int q = 0; q < 6; ++q) m[q] = q == i ? 1.0 : 0.0;
+  double chi[24];
+  affine_local(m, c, chi);
+  for (int g = 0; g < 256; g += kEffElements) {
+    const int64_t e = int64_t(blockIdx.x) * 256 + g + k;
+    const int64_t ec = e < N ? e : N - 1;
+    const int x = int(ec % nx), y = int((ec / nx) % ny), z = int(ec / (int64_t(nx) * ny));
+    const double ae = e < N ? a[ec] : 0.0;
+    double vi[24], fi[24];
+    gather_element(u6 + int64_t(i) * 3 * N, nz, ny, nx, x, y, z, vi);
 #pragma unroll
-      for (int k = 0; k < 24; ++k) vi[k] += chi[k];
-      hex8_element<CUBIC>(vi, 1.0, c, fi);
-      for (int j = i; j < 6; ++j, ++idx) {
-        double vj[24];
-        double mj[6] = {0, 0, 0, 0, 0, 0};
-        mj[j] = 1.0;
-        gather_element(u6 + int64_t(j) * 3 * N, nz, ny, nx, x, y, z, vj);
-        affine_local(mj, c, chi);
-        double t = 0.0;
+    for (int q = 0; q < 24; ++q) vi[q] += chi[q];
+    hex8_element<CUBIC>(vi, 1.0, c, fi);
+    __syncthreads();   // the previous group's values have been read
 #pragma unroll
-        for (int k = 0; k < 24; ++k) t = fma(fi[k], vj[k] + chi[k], t);
-        s[idx] = ae * t / c.vol;
-      }
+    for (int q = 0; q < 24; ++q) v[i][q][k] = vi[q];
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int j = i + p < 6 ? i + p : i + p - 6;
+      double t = 0.0;
+#pragma unroll
+      for (int q = 0; q < 24; ++q) t = fma(fi[q], v[j][q][k], t);
+      s[p] = e < N ? s[p] + ae * t / c.vol : s[p];
     }
   }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // sums over the 32 lanes of a load
 #pragma unroll
-  for (int k = 0; k < 21; ++k) {
-    const double t = wave_sum(s[k]);
-    if (lane == 0) red[k][wave] = t;
-  }
-  __syncthreads();
-  if (threadIdx.x < 21) {
-    double t = 0.0;
-    for (int w = 0; w < 4; ++w) t += red[threadIdx.x][w];
-    part[int64_t(blockIdx.x) * 21 + threadIdx.x] = t;
-  }
+  for (int p = 0; p < 4; ++p)
+#pragma unroll
+    for (int off = kEffElements / 2; off >= 1; off >>= 1) s[p] += __shfl_xor(s[p], off, 64);
+  if (k == 0)
+    for (int p = 0; p < (i < 3 ? 4 : 3); ++p) {
+      const int j = i + p < 6 ? i + p : i + p - 6, lo = min(i, j), hi = max(i, j);
+      part[int64_t(blockIdx.x) * 21 + lo * 6 - lo * (lo - 1) / 2 + (hi - lo)] = s[p];
+    }
 }
 
 __global__ void effective_finish(const double* part, int nblk, int64_t N, double* out) {
@@ -795,27 +887,77 @@ int launch_rowmarch(const pgj_grid& g, int L, int mode, RowArgsT<T>& A, hipStrea
 template int launch_rowmarch<double>(const pgj_grid&, int, int, RowArgsT<double>&, hipStream_t);
 template int launch_rowmarch<float>(const pgj_grid&, int, int, RowArgsT<float>&, hipStream_t);
 
-int launch_reference(const pgj_grid& g, int L, RefArgs& A, bool cert, hipStream_t s) {
-  A.nz = g.nz; A.ny = g.ny; A.nx = g.nx;
-  A.N = int64_t(g.nx) * g.ny * g.nz;
-  A.coef = coef_of(g);
-  dim3 grid(unsigned((A.N + 255) / 256), L), block(256);
-  const bool cb = cubic(g);
-  if (cert) {
-    if (cb) hipLaunchKernelGGL((hex8_reference<true, true>), grid, block, 0, s, A);
-    else hipLaunchKernelGGL((hex8_reference<false, true>), grid, block, 0, s, A);
-  } else {
-    if (cb) hipLaunchKernelGGL((hex8_reference<true, false>), grid, block, 0, s, A);
-    else hipLaunchKernelGGL((hex8_reference<false, false>), grid, block, 0, s, A);
+// 36 numbers of the element stiffness (RefStiffness).
+static RefStiffness ref_stiffness(const pgj_grid& g) {
+  RefStiffness K{};
+  const double h[3] = {g.hx, g.hy, g.hz};
+  auto mass = [&](int axis, int differ) { return differ ? h[axis] / 6 : h[axis] / 3; };
+  for (int df = 0; df < 8; ++df) {
+    double grad[3];   // integral of the product of the two nodes' derivatives along one axis
+    for (int j = 0; j < 3; ++j) {
+      grad[j] = ((df >> j) & 1 ? -1.0 : 1.0) / h[j];
+      for (int k = 0; k < 3; ++k)
+        if (k != j) grad[j] *= mass(k, (df >> k) & 1);
+    }
+    for (int i = 0; i < 3; ++i) {
+      K.diag[i][df] = g.lam * grad[i];
+      for (int j = 0; j < 3; ++j) K.diag[i][df] += g.mu * (i == j ? 2.0 : 1.0) * grad[j];
+    }
   }
+  for (int k = 0; k < 3; ++k)
+    for (int differ = 0; differ < 2; ++differ) {
+      K.off_sum[k][differ] = (g.lam + g.mu) * 0.25 * mass(k, differ);
+      K.off_diff[k][differ] = (g.lam - g.mu) * 0.25 * mass(k, differ);
+    }
+  return K;
+}
+
+// Planes per thread: the longest march that leaves 96k threads (six waves per CU), so that one layer in ZC + 1 is
+// redundant; at least 2.
+static int reference_zc(const pgj_grid& g, int L) {
+  const int64_t N = int64_t(g.nx) * g.ny * g.nz;
+  int zc = 16;
+  while (zc > 2 && N * L / zc < 98304) zc /= 2;
+  return zc;
+}
+
+int reference_blocks(const pgj_grid& g, int L) {
+  const int zc = reference_zc(g, L);
+  return int((int64_t(g.nx) * g.ny * ((g.nz + zc - 1) / zc) + 255) / 256);
+}
+
+template <bool CERT>
+static int launch_reference_t(const pgj_grid& g, int L, RefArgs& A, hipStream_t s) {
+  const dim3 grid(unsigned(reference_blocks(g, L)), L), block(256);
+  const RefStiffness K = ref_stiffness(g);
+  const int zc = reference_zc(g, L);
+  if (A.N < (int64_t(1) << 32) / 24)
+    hipLaunchKernelGGL((hex8_reference<CERT, unsigned>), grid, block, 0, s, A, K, zc);
+  else
+    hipLaunchKernelGGL((hex8_reference<CERT, int64_t>), grid, block, 0, s, A, K, zc);
   PGJ_LAUNCHED("hex8_reference");
   return PGJ_OK;
 }
 
-int launch_subtract_mean(const pgj_grid& g, int L, double* v, const double* part, int soa, hipStream_t s) {
+int launch_reference(const pgj_grid& g, int L, RefArgs& A, bool cert, hipStream_t s) {
+  A.nz = g.nz; A.ny = g.ny; A.nx = g.nx;
+  A.N = int64_t(g.nx) * g.ny * g.nz;
+  return cert ? launch_reference_t<true>(g, L, A, s) : launch_reference_t<false>(g, L, A, s);
+}
+
+// Above 256 partial rows per load (more than 40^3 nodes) the means are reduced once per load instead of once per
+// block: 128^3, six loads, 1071 us of which all but 110 were the blocks' own reductions of 8192 rows; 64^3 22.9 us.
+// Below, the second launch costs more than it saves.
+int launch_subtract_mean(const pgj_grid& g, int L, double* v, double* part, int soa, hipStream_t s) {
   const int64_t N = int64_t(g.nx) * g.ny * g.nz;
   const int nblk = int((N + 255) / 256);
-  hipLaunchKernelGGL(subtract_mean, dim3(nblk, L), dim3(256), 0, s, v, N, part, nblk, soa);
+  if (nblk > 256) {
+    hipLaunchKernelGGL(component_means, dim3(L), dim3(256), 0, s, N, part, nblk);
+    PGJ_LAUNCHED("component_means");
+    hipLaunchKernelGGL(subtract_mean<true>, dim3(nblk, L), dim3(256), 0, s, v, N, part, nblk, soa);
+  } else {
+    hipLaunchKernelGGL(subtract_mean<false>, dim3(nblk, L), dim3(256), 0, s, v, N, part, nblk, soa);
+  }
   PGJ_LAUNCHED("subtract_mean");
   return PGJ_OK;
 }
@@ -931,9 +1073,9 @@ extern "C" int pgj_effective_tensor(const pgj_grid* g, const double* a, const do
   const int nblk = int((N + 255) / 256);
   hipStream_t s = as_stream(stream);
   if (cubic(*g))
-    hipLaunchKernelGGL(effective_partials<true>, dim3(nblk), dim3(256), 0, s, g->nz, g->ny, g->nx, coef_of(*g), a, u6, ws);
+    hipLaunchKernelGGL(effective_partials<true>, dim3(nblk), dim3(kEffThreads), 0, s, g->nz, g->ny, g->nx, coef_of(*g), a, u6, ws);
   else
-    hipLaunchKernelGGL(effective_partials<false>, dim3(nblk), dim3(256), 0, s, g->nz, g->ny, g->nx, coef_of(*g), a, u6,
+    hipLaunchKernelGGL(effective_partials<false>, dim3(nblk), dim3(kEffThreads), 0, s, g->nz, g->ny, g->nx, coef_of(*g), a, u6,
                        ws);
   PGJ_LAUNCHED("effective_partials");
   hipLaunchKernelGGL(effective_finish, dim3(21), dim3(64), 0, s, ws, nblk, N, out36);
@@ -997,10 +1139,10 @@ extern "C" int pgj_effective_tensor_noalloc(const pgj_grid* g, const double* a, 
   const int nblk = int((N + 255) / 256);
   hipStream_t s = as_stream(stream);
   if (cubic(*g))
-    hipLaunchKernelGGL(effective_partials<true>, dim3(nblk), dim3(256), 0, s, g->nz, g->ny, g->nx, coef_of(*g), a,
+    hipLaunchKernelGGL(effective_partials<true>, dim3(nblk), dim3(kEffThreads), 0, s, g->nz, g->ny, g->nx, coef_of(*g), a,
                        u6, part);
   else
-    hipLaunchKernelGGL(effective_partials<false>, dim3(nblk), dim3(256), 0, s, g->nz, g->ny, g->nx, coef_of(*g), a,
+    hipLaunchKernelGGL(effective_partials<false>, dim3(nblk), dim3(kEffThreads), 0, s, g->nz, g->ny, g->nx, coef_of(*g), a,
                        u6, part);
   PGJ_LAUNCHED("effective_partials");
   hipLaunchKernelGGL(effective_finish, dim3(21), dim3(64), 0, s, part, nblk, N, out36);

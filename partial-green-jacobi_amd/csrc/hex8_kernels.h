@@ -26,20 +26,19 @@ struct RowArgsT {
 };
 using RowArgs = RowArgsT<double>;
 
-// Independent reference apply: one thread per node gathers the rows of its
-// eight elements; optionally fused with the certification residual.
+// Independent reference apply: one thread per node, by another form of the
+// element stiffness; optionally fused with the certification residual.
 struct RefArgs {
   int nz, ny, nx;
   int64_t N;
-  ElementCoef coef;
-  bool cubic;
   const double* a;
   const double* u;
   double* out;
   // certification residual: out = rhs - K u, per-block |r|^2 into slot 3 of
-  // 4-wide partial rows [l][block][4]
+  // 4-wide partial rows [l][block][4], pres_rows rows per load
   const double* rhs;
   double* pres;
+  int pres_rows;
   int soa;               // vectors are SoA (L, 3, N) instead of AoS (L, N, 3)
   int group;             // loads per design (a is (designs, N)); 0: one shared a
 };
@@ -51,8 +50,10 @@ int check_grid(const pgj_grid* g);
 template <typename T>
 int launch_rowmarch(const pgj_grid& g, int L, int mode, RowArgsT<T>& A, hipStream_t s);
 int launch_reference(const pgj_grid& g, int L, RefArgs& A, bool cert, hipStream_t s);
+// Blocks per load of launch_reference over L loads (at most one per 256 nodes).
+int reference_blocks(const pgj_grid& g, int L);
 int launch_component_sums(const pgj_grid& g, int L, const double* v, double* part, int soa, hipStream_t s);
-int launch_subtract_mean(const pgj_grid& g, int L, double* v, const double* part, int soa, hipStream_t s);
+int launch_subtract_mean(const pgj_grid& g, int L, double* v, double* part, int soa, hipStream_t s);
 int launch_rhs(const pgj_grid& g, const double* a, const double* macro, double* out, int soa, hipStream_t s);
 // alpha_dev (nullable): read alpha from device memory instead of `alpha`
 int launch_scale(const pgj_grid& g, const double* a, double alpha, double* d, double* s_out, double* ws, int soa,

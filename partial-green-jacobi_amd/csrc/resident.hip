@@ -49,9 +49,10 @@ __global__ void setup_finish(const double* part, int nblk, double rtol, double a
   }
 }
 
-__global__ void certify_finish(const double* part, int nblk, StateView st) {
+// Sum of slot 3 of the first nblk of a load's `rows` partial rows.
+__global__ void certify_finish(const double* part, int rows, int nblk, StateView st) {
   const int l = blockIdx.x;
-  const double s = wave_reduce_partials(part + int64_t(l) * nblk * 4 + 3, nblk, 4);
+  const double s = wave_reduce_partials(part + int64_t(l) * rows * 4 + 3, nblk, 4);
   if (threadIdx.x == 0) st.absolute[l] = sqrt(s);
 }
 
@@ -163,9 +164,11 @@ extern "C" int pgj_resident_certify(const pgj_grid* g, int L, int group, int l0,
   if (int e = launch_subtract_mean(*g, nl, us, b.pcert, 1, s)) return e;
   RefArgs A{};
   A.a = a + sl.design() * sl.N; A.u = us; A.out = r + sl.vec(); A.rhs = rhs + sl.vec(); A.pres = b.pcert;
+  A.pres_rows = b.lay.nblk_cert;
   A.soa = 1; A.group = group;
   if (int e = launch_reference(*g, nl, A, true, s)) return e;
-  hipLaunchKernelGGL(certify_finish, dim3(nl), dim3(64), 0, s, b.pcert, b.lay.nblk_cert, state_view(state, L, l0));
+  hipLaunchKernelGGL(certify_finish, dim3(nl), dim3(64), 0, s, b.pcert, b.lay.nblk_cert, reference_blocks(*g, nl),
+                     state_view(state, L, l0));
   PGJ_LAUNCHED("certify_finish");
   return PGJ_OK;
 }
@@ -377,7 +380,8 @@ extern "C" int pgj_hybrid_resident_certify(const pgj_grid* g, int L, int l0, int
   if (int e = launch_component_sums(*g, nl, us, b.pcert, 1, s)) return e;
   if (int e = launch_subtract_mean(*g, nl, us, b.pcert, 1, s)) return e;
   if (int e = launch_c21_certify(*g, nl, pool, index, us, rhs + sl.vec(), r + sl.vec(), b.pcert, s)) return e;
-  hipLaunchKernelGGL(certify_finish, dim3(nl), dim3(64), 0, s, b.pcert, b.lay.nblk_cert, state_view(state, L, l0));
+  hipLaunchKernelGGL(certify_finish, dim3(nl), dim3(64), 0, s, b.pcert, b.lay.nblk_cert, b.lay.nblk_cert,
+                     state_view(state, L, l0));
   PGJ_LAUNCHED("certify_finish");
   return PGJ_OK;
 }
