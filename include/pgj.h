@@ -133,10 +133,9 @@ int pgj_hex8_set_shape(const pgj_grid* g, int L, int es, int R, int W, int ZC, i
  * precision es (8: FP64, 4: FP32): pass 0 forward x/y, 1 z with the Green
  * multiply, 2 inverse y/x; plan 0 takes radix-4 stages first (64 = 4 x 4 x 4),
  * plan 1 radix-8 stages first (64 = 8 x 8); for the z pass at 64^3, plan 2
- * keeps the transforms in registers (two radix-8 passes with one LDS transpose
- * each, LDS otherwise only for the 3x3 Green multiply). plan -1 leaves the pass
- * to the library's choice for that length (radix 8 first from 24 on, except the z
- * pass at 48). The
+ * keeps the transforms and the Green multiply in registers (one LDS exchange per
+ * transform). plan -1 leaves the pass to the library's choice for that length
+ * (radix 8 first from 24 on; the z pass in registers where 16 divides n). The
  * choice holds for every later launch of that pass on any n^3 grid of that
  * precision (a graph keeps the kernels of its capture; a solver reads the plan
  * when it sets up its launches). get_plan writes the three passes' plans, 0
@@ -257,9 +256,9 @@ int pgj_alpha_select(const pgj_grid* g, int method, const double* params, const 
  * passes' block shapes, and so the layout of the partial sums one pass leaves
  * for the next, follow it. */
 
-/* 1 if the z pass of a resident set of L loads (its workspace's load count) with
- * elements of es bytes runs on the wide kx chunks on the current device (64^3
- * FP64 where the default chunks need more than one round of blocks), else 0. */
+/* 1 if the LDS z pass of a resident set of L loads (its workspace's load count)
+ * with elements of es bytes runs on the wide kx chunks on the current device
+ * (64^3 FP64 where these give more than one round of blocks), else 0. */
 int pgj_zpass_wide(const pgj_grid* g, int L, int es);
 
 /* rhs_l for the L macro strains (host L*6), norms, targets

@@ -60,9 +60,8 @@ int launch_fz_mode(FFTArgs& A, int L, int mode, hipStream_t s);
 int launch_fxyi_mode(FFTArgs& A, int L, int mode, hipStream_t s);
 // Compile-time-shaped SoA kernels for cubic grids (n in 16, 24, 32, 48, 64, 96, 128).
 bool static_fft(const pgj_grid& g);
-// Whether the z pass of a solve with L loads in all (its workspace's load count) and elements of es bytes
-// takes the wide kx chunks: where the default chunks need more than one round of blocks on the device
-// (64^3 FP64 from 6 loads on 256 CUs).
+// Whether the LDS z pass of a solve with L loads in all (its workspace's load count) and elements of es bytes
+// takes the wide kx chunks: where these fill the device with more than one round of blocks (64^3 FP64).
 bool zpass_wide(const pgj_grid& g, int L, int es);
 // Sets A.zkc and A.zslots for a workspace of L loads (FFTArgsT).
 template <typename T> void zpass_choose(FFTArgsT<T>& A, const pgj_grid& g, int L);

@@ -25,6 +25,9 @@ struct Cube {
   static constexpr int PLANE = N * N;         // nodes per z-plane
   static constexpr int64_t NF = int64_t(N) * N * NKX;
   static constexpr int TXY = N >= 96 ? 512 : 256;
+  // Partial sums of the other passes are added up by the whole block where there are many of them (128^3: 1040 rows of
+  // the z pass per load), else by every wave for itself, which needs no barrier.
+  static constexpr bool SHARED_SUMS = N >= 96;
   // LDS bytes for complex values of ES bytes: the data, the twiddle table W_N^j
   // (j < N; the same table serves x, y and z on a cube) and a reduction tail
   // of 4 values x 8 waves
@@ -41,71 +44,62 @@ struct Cube {
   static constexpr bool EXACT = HALF % TXY == 0;
 };
 
-// z pass of a cube in precision R: KC kx columns of all three components per
-// block; a row of KC complex values is the contiguous run a block reads per
-// (c, kz). A last chunk narrower than KC is supported (columns past NKX are
-// zero in LDS and skipped). 128^3 takes 13 columns in FP32 (104-byte runs
-// instead of 40) but keeps 5 in FP64, where 13 would need 147 VGPRs at 2 blocks
-// per CU; 17 columns at 96^3 measured no faster than 7. KCX > 0 overrides the
-// chunk width (ZWidths).
-template <int N, typename R, int KCX = 0>
-struct ZPass {
-  static constexpr int NKX = N / 2 + 1;
-  static constexpr int KC = KCX > 0    ? KCX
-                            : N == 16  ? 9
-                            : N == 24  ? 13
-                            : N == 32  ? 17
-                            : N == 48  ? 5
-                            : N == 64  ? 11
-                            : N == 96  ? 7
-                            : sizeof(R) == 8 ? 5 : 13;
-  static constexpr int TZ = KC >= 13 && N >= 96 ? 512 : 256;
-  static constexpr int NKB = (NKX + KC - 1) / KC;
-  static constexpr bool KFULL = NKX % KC == 0;
-  // columns and the twiddle table; the reduction reuses the column storage once
-  // the columns are written back (2 blocks of the 128^3 FP32 pass fit one CU)
-  static constexpr size_t lds = (size_t(3) * N * KC + N) * 2 * sizeof(R);
-  static constexpr int occ = lds_occupancy(lds, TZ);
-  static constexpr int per_cu = occ * 4 / (TZ / 64) > 0 ? occ * 4 / (TZ / 64) : 1;  // resident blocks per CU
-  using ZCols = Lines<3 * KC, KC, N * KC, 1, KC, true>;  // z transforms on (component, column)
+// Layout of a load's half spectrum between the passes: the columns kx < N/2 as [c][kz][ky][kx], then the Nyquist
+// columns kx = N/2 as [c][kz][ky]. A row of the first part is N/2 complex values, so a chunk of 8 (FP64) or 16 (FP32)
+// columns is one aligned 128-byte line that one block of the z pass reads and writes whole. In rows of N/2 + 1 values
+// every run straddled lines that its neighbours fetched again (128^3 FP32, three loads: 430 MB fetched for 77 MB of
+// spectrum and 51 MB of symbol and scale spectrum).
+template <int N>
+struct Spec {
+  static constexpr int M = N / 2;
+  static constexpr int64_t MAIN = int64_t(3) * N * N * M;
 };
 
-// The kx chunk widths a z pass can run with (FFTArgs::zkc picks one per workspace, zpass_choose):
-// - wide, 64^3 FP64 from 6 loads on 256 CUs (zpass_wide): 17 columns in 52 KiB of LDS (3 blocks per CU) instead
-//   of 11 in 34 KiB (4 per CU). A 6-load launch is 768 blocks, exactly one round, instead of 1152 on 1024 slots:
-//   27 us against 33 us. Launches of many rounds gain from reading the symbol and s_hat in fewer blocks.
-// - narrow, where the default chunks give at most 2.5 blocks per CU (few loads on a small grid): the blocks are
-//   what hides the pass's latency there. Graph-replayed launches, radix 8 first, default against narrow:
-//   32^3 FP64 1 / 3 / 6 loads 10.1 / 10.5 / 11.2 -> 6.5 / 7.6 / 9.5 us, 24^3 8.6 / 8.7 / 9.0 -> 6.4 / 6.7 / 7.6,
-//   16^3 6.4 -> 5.8 (6 loads 6.5 -> 6.3), 64^3 1 / 3 loads 13.2 / 19.8 -> 10.9 / 19.5; FP32 alike. Above that the
-//   default is faster (64^3 FP32, 6 loads, 4.5 blocks per CU: 22.7 against 25.5 us). 48^3 already runs 5 columns
-//   (3: 13.6 against 11.6 us at 3 loads).
+// z pass of a cube in precision R on KC columns of all three components per block: N/2 / KC chunks per ky row, then
+// blocks of the Nyquist column, KC ky values each.
+template <int N, typename R, int KC>
+struct ZPass {
+  static_assert((N / 2) % KC == 0 && N % KC == 0, "chunks cover the columns exactly");
+  static constexpr int NCH = N / 2 / KC;
+  static constexpr int BLOCKS = NCH * N + N / KC;
+  static constexpr int TZ = 3 * N * KC >= 4096 ? 512 : 256;
+  // columns in LDS: rows of KC + 1 values and components KC values further apart than their N rows, so that the lines
+  // of a transform (a power of two apart otherwise) fall on different banks
+  static constexpr int KS = KC + 1, CS = N * KS + KC;
+  // columns and the twiddle table; the reduction reuses the column storage once the columns are written back
+  static constexpr int COLS = 3 * CS;
+  static constexpr size_t lds = (size_t(COLS) + N) * 2 * sizeof(R);
+  __host__ __device__ static constexpr int slot(int cz, int k) { return cz * KS + cz / N * KC + k; }
+  static constexpr int occ = lds_occupancy(lds, TZ);
+  static constexpr int per_cu = occ * 4 / (TZ / 64) > 0 ? occ * 4 / (TZ / 64) : 1;  // resident blocks per CU
+  using ZCols = Lines<3 * KC, KC, CS, 1, KS, true>;  // z transforms on (component, column)
+};
+
+// Chunk widths of the LDS z pass (fz_static), the best of the widths that divide N/2 on launches of one, three and six
+// loads: 96^3 FP64 6 columns 31.7 / 68.6 / 127 us (8: 34.0 / 73.6 / 136, 12: 35.9 / 75.8 / 132), 96^3 FP32 8 columns
+// 23.7 / 43 / 73 (6: 25.4 / 46 / 82), 64^3 FP64 4 columns 11.9 / 20.4 / 32.2 (8: 13.6 / 20.5 / 30.7: `wide`, six loads).
 template <int N, typename R>
 struct ZWidths {
-  static constexpr int def = ZPass<N, R>::KC;
-  static constexpr int narrow = N == 16 ? 3 : N == 24 ? 5 : N == 32 ? 4 : N == 64 ? 4 : def;
-  static constexpr int wide = N == 64 && sizeof(R) == 8 ? 17 : def;
+  static constexpr bool d = sizeof(R) == 8;
+  static constexpr int def = N <= 64 ? 4 : N == 96 ? (d ? 6 : 8) : d ? 8 : 16;
+  static constexpr int wide = N == 64 && d ? 8 : def;
 };
 
 // Radix plan of a pass whose plan is not set (pgj_fft_set_plan), and of the passes outside the PCG iteration:
 // radix 8 first, one LDS stage less at 32 and 64 and 128. Graph-replayed 3-load launches, radix 4 first against
-// radix 8 first, fxy / fz / fxyi: 64^3 FP64 22.8 / 21.3 / 23.5 -> 20.9 / 19.8 / 22.5 us, 32^3 7.1 / 12.2 / 6.8 ->
-// 6.9 / 10.5 / 6.4, 128^3 FP32 85.5 / 99.0 / 104.4 -> 81.2 / 96.2 / 99.4. Radix 4 first stays where it is no
-// slower: 16 (4 x 4 against 8 x 2: 4.4 / 6.4 / 4.1 against 4.5 / 6.6 / 4.2) and the z pass at 48 (11.1 against 11.6).
+// radix 8 first, fxy / fxyi: 64^3 FP64 23.2 / 23.6 -> 21.6 / 22.4 us, 48^3 12.3 / 13.1 -> 11.7 / 12.5, 32^3 7.2 / 6.7 ->
+// 6.9 / 6.3, 128^3 FP32 72.3 / 101.7 -> 67.8 / 98.4. Radix 4 first stays where it is no slower: 16 (4 x 4 against 8 x 2:
+// 4.4 / 4.3 against 4.5 / 4.4).
 template <int N>
-constexpr int default_plan(int pass) {
-  return N == 16 || (N == 48 && pass == 1) ? 0 : 1;
+constexpr int default_plan() {
+  return N == 16 ? 0 : 1;
 }
 
 template <int N, typename R>
 int plan_of(int pass) {
   const int plan = fft_plan(N, int(sizeof(R)), pass);
-  return plan < 0 ? default_plan<N>(pass) : plan;
+  return plan < 0 ? default_plan<N>() : plan;
 }
-
-// Register-resident z pass of the 64^3 cube (fz64_reg below): blocks per load, which lay out its partials:
-// 4 chunks of 8 kx columns per ky row, then 8 blocks for the Nyquist column kx = 32 (8 ky rows each).
-constexpr int kZRegBlocks = 4 * 64 + 8;
 
 // Global -> LDS copy of COUNT values in two phases, so that independent work
 // can run while the loads are in flight: load() issues every load of a thread
@@ -123,12 +117,16 @@ struct StageIn {
       v[k] = src[map(e)];
     }
   }
-  __device__ inline void store(X* lds) const {
+  template <typename Slot>
+  __device__ inline void store(X* lds, Slot slot) const {
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
       const int e = int(threadIdx.x) + k * T;
-      if (COUNT % T == 0 || e < COUNT) lds[e] = v[k];
+      if (COUNT % T == 0 || e < COUNT) lds[slot(e)] = v[k];
     }
+  }
+  __device__ inline void store(X* lds) const {
+    store(lds, [](int e) { return e; });
   }
 };
 
@@ -205,8 +203,18 @@ void fxy_static(FFTArgsT<R> A) {
     if (MODE == kFxyPCG && i0 == 0) {
       double pq, rz;
       // per-load partials are laid out with the geometry's chunk count (slices of a set are offset by it)
-      wave_reduce_partials_2(A.ppq + int64_t(l) * A.ppq_stride, A.ppq_count, 1, A.pg + int64_t(l) * A.f.nkb * N * 4,
-                             A.zslots, 4, pq, rz);
+      const double* ppq = A.ppq + int64_t(l) * A.ppq_stride;
+      const double* pg = A.pg + int64_t(l) * A.f.nkb * N * 4;
+      if (C::SHARED_SUMS) {
+        double t[2] = {0.0, 0.0};
+        for (int k = threadIdx.x; k < A.ppq_count; k += T) t[0] += ppq[k];
+        for (int k = threadIdx.x; k < A.zslots; k += T) t[1] += pg[4 * k];
+        block_sums<2>(t, red);
+        pq = t[0];
+        rz = t[1];
+      } else {
+        wave_reduce_partials_2(ppq, A.ppq_count, 1, pg, A.zslots, 4, pq, rz);
+      }
       const bool valid = isfinite(pq) && pq > 0.0 && isfinite(rz) && rz > 0.0;
       alpha = valid ? rz / pq : 0.0;
       if (threadIdx.x == 0 && z == 0 && c == 0) {
@@ -270,29 +278,38 @@ void fxy_static(FFTArgsT<R> A) {
   }
   __syncthreads();
   sfft<false, N, typename C::Cols, T, PLAN>(plane, tw, 1);
-  X* out = A.spec + ((int64_t(l) * 3 + c) * N + z) * int64_t(N) * C::NKX;
-  for (int e = threadIdx.x; e < N * C::NKX; e += T) out[e] = plane[e];
+  if (MODE == kFxyScale) {
+    // the caller's s_hat: rows of N/2 + 1 values
+    X* out = A.spec + ((int64_t(l) * 3 + c) * N + z) * int64_t(N) * C::NKX;
+    for (int e = threadIdx.x; e < N * C::NKX; e += T) out[e] = plane[e];
+  } else {
+    X* out = A.spec + int64_t(l) * 3 * C::NF;
+    X* row = out + (int64_t(c) * N + z) * (N * C::M);
+    for (int e = threadIdx.x; e < N * C::M; e += T) row[e] = plane[e / C::M * C::RS + e % C::M];
+    X* nyq = out + Spec<N>::MAIN + (int64_t(c) * N + z) * N;
+    for (int y = threadIdx.x; y < N; y += T) nyq[y] = plane[y * C::RS + C::M];
+  }
 }
 
 // ---------------------------------------------------------------- z + Green
-template <int N, int MODE, typename R, int KCX = 0, int PLAN = 0>
-__global__ __launch_bounds__((ZPass<N, R, KCX>::TZ)) __attribute__((amdgpu_waves_per_eu((ZPass<N, R, KCX>::occ))))
+template <int N, int MODE, typename R, int KC, int PLAN = 0>
+__global__ __launch_bounds__((ZPass<N, R, KC>::TZ)) __attribute__((amdgpu_waves_per_eu((ZPass<N, R, KC>::occ))))
 void fz_static(FFTArgsT<R> A) {
   using C = Cube<N>;
   using X = cplx<R>;
-  using Z = ZPass<N, R, KCX>;
-  constexpr int T = Z::TZ, KC = Z::KC, NKX = C::NKX;
+  using Z = ZPass<N, R, KC>;
+  constexpr int T = Z::TZ, NKX = C::NKX;
   extern __shared__ __align__(16) unsigned char smem[];
   X* cols = reinterpret_cast<X*>(smem);
-  X* tw = cols + 3 * N * KC;
+  X* tw = cols + Z::COLS;
   double* red = reinterpret_cast<double*>(cols);  // used only after the columns are written back
-  // ky is the fastest grid index: the kx chunks of one ky row (which share
-  // cache lines) get block ids N apart, a multiple of 8 for every supported N,
-  // and so run on the same XCD / L2.
-  const int y = blockIdx.x, kb = blockIdx.y, l = blockIdx.z;
-  const int kx0 = kb * KC;
-  const int blk = y * Z::NKB + kb;
-  const bool lead = threadIdx.x == 0 && kb == 0 && y == 0;
+  // ky is the fastest index: the kx chunks of one ky row (which share lines of the symbol and s_hat) get block ids N
+  // apart, a multiple of 8 for every supported N, and so run on the same XCD / L2.
+  const int blk = blockIdx.x, l = blockIdx.z;
+  const bool nyq = blk >= Z::NCH * N;                       // blocks of the Nyquist column
+  const int y = nyq ? (blk - Z::NCH * N) * KC : blk % N;    // ky of column 0
+  const int kx0 = nyq ? N / 2 : blk / N * KC;               // kx of column 0
+  const bool lead = threadIdx.x == 0 && blk == 0;
   const int64_t NN = int64_t(N) * N * N;
   // the spectrum columns are loaded first (for every load that may continue)
   // and stay in flight through the convergence test and the mean reduction
@@ -306,22 +323,21 @@ void fz_static(FFTArgsT<R> A) {
     }
     return;
   }
-  // the spectrum columns and the twiddle table go to LDS first (LDS slot
-  // e = cz * KC + kcol with cz = c * N + zz); they are read after the test below
-  X* S = A.spec + int64_t(l) * 3 * C::NF;
-  // columns of this chunk (the last chunk may hold fewer than KC; its missing columns are zero in LDS)
-  const int kcn = Z::KFULL ? KC : min(KC, NKX - kx0);
+  // the spectrum columns and the twiddle table go to LDS first; they are read after the test below
+  // frequency (cz, column) in the rows of N/2 + 1 values of the symbol and s_hat, and in the spectrum (the scale pass
+  // transforms s_hat in place)
+  const int fcol = nyq ? NKX : 1;
+  const int f0 = y * NKX + kx0;
+  const bool packed = MODE != kFzScale;
+  const int scol = packed ? 1 : fcol;
+  const int sstep = !packed ? N * NKX : nyq ? N : N * (N / 2);
+  X* S = A.spec + int64_t(l) * 3 * C::NF + (!packed ? int64_t(f0) : nyq ? Spec<N>::MAIN + y : int64_t(y) * (N / 2) + kx0);
   {
     StageIn<3 * N * KC, T, X> in;
-    in.load(S, [&](int e) { return (int64_t(e / KC) * N + y) * NKX + kx0 + min(e % KC, kcn - 1); });
-    if (!Z::KFULL) {
-#pragma unroll
-      for (int k = 0; k < in.PER; ++k)
-        if ((int(threadIdx.x) + k * T) % KC >= kcn) in.v[k] = c2(R(0), R(0));
-    }
+    in.load(S, [&](int e) { return e / KC * sstep + e % KC * scol; });
     StageIn<N, T, X> twl;
     twl.load(A.twz, [](int e) { return e; });
-    in.store(cols);
+    in.store(cols, [](int e) { return Z::slot(e / KC, e % KC); });
     twl.store(tw);
   }
   double mean[3] = {0.0, 0.0, 0.0};
@@ -368,25 +384,23 @@ void fz_static(FFTArgsT<R> A) {
       mean[c] = wave_reduce_partials(A.pr + (int64_t(l) * N * 3 + c) * 2 + 1, N, 6) / double(NN);
   }
   // a fixed number of frequency slots per thread, in groups of GS slots whose
-  // symbol and s_hat loads are all issued before the first is used. In FP32 one
-  // group holds every slot and is issued before the forward transform, so the
-  // loads stay in flight while it runs; FP64, and FP32 with more than 3 slots,
-  // lack the registers for that and issue their groups after it (the scaling
-  // pass needs none).
+  // symbol and s_hat loads are all issued before the first is used. Where one
+  // group of them fits 64 registers it holds every slot and is issued before the
+  // forward transform, so the loads stay in flight while it runs.
   constexpr int EPT = (N * KC + T - 1) / T;
-  constexpr bool EARLY = sizeof(R) == 4 && EPT <= 3;
+  constexpr bool EARLY = EPT * sizeof(R) <= 16;
   constexpr int GS = (EARLY || EPT <= 3) ? EPT : 2;
   constexpr bool FULL = (N * KC) % T == 0;
-  const X* __restrict__ shat_d = A.shat ? A.shat + int64_t(design_of(l, A.group)) * 3 * C::NF : nullptr;
-  const R* __restrict__ sym = A.sym;
+  const X* __restrict__ shat_d = A.shat ? A.shat + int64_t(design_of(l, A.group)) * 3 * C::NF + f0 : nullptr;
+  const R* __restrict__ sym = A.sym + f0;
   auto slot = [&](int k) { return FULL ? int(threadIdx.x) + k * T : min(int(threadIdx.x) + k * T, N * KC - 1); };
-  auto freq = [&](int e) { return (int64_t(e / KC) * N + y) * NKX + kx0 + min(e % KC, kcn - 1); };
+  auto freq = [&](int e) { return e / KC * (N * NKX) + e % KC * fcol; };
   R g[GS][6];
   X sh[GS][3];
   auto load_group = [&](int k0) {
 #pragma unroll
     for (int i = 0; i < GS; ++i) {
-      const int64_t fidx = freq(slot(k0 + i < EPT ? k0 + i : EPT - 1));
+      const int fidx = freq(slot(k0 + i < EPT ? k0 + i : EPT - 1));
 #pragma unroll
       for (int j = 0; j < 6; ++j) g[i][j] = sym[j * C::NF + fidx];
 #pragma unroll
@@ -395,7 +409,7 @@ void fz_static(FFTArgsT<R> A) {
     if (shat_d) {
 #pragma unroll
       for (int i = 0; i < GS; ++i) {
-        const int64_t fidx = freq(slot(k0 + i < EPT ? k0 + i : EPT - 1));
+        const int fidx = freq(slot(k0 + i < EPT ? k0 + i : EPT - 1));
 #pragma unroll
         for (int c = 0; c < 3; ++c) sh[i][c] = shat_d[int64_t(c) * C::NF + fidx];
       }
@@ -405,10 +419,7 @@ void fz_static(FFTArgsT<R> A) {
   __syncthreads();
   sfft<false, N, typename Z::ZCols, T, PLAN>(cols, tw, 1);
   if (MODE == kFzScale) {
-    for (int e = threadIdx.x; e < 3 * N * KC; e += T) {
-      const int kcol = e % KC, cz = e / KC;
-      if (Z::KFULL || kcol < kcn) S[(int64_t(cz) * N + y) * NKX + kx0 + kcol] = cols[e];
-    }
+    for (int e = threadIdx.x; e < 3 * N * KC; e += T) S[e / KC * sstep + e % KC * scol] = cols[Z::slot(e / KC, e % KC)];
     return;
   }
   double rz = 0.0, sw[3] = {0.0, 0.0, 0.0};
@@ -421,11 +432,9 @@ void fz_static(FFTArgsT<R> A) {
       const int e = threadIdx.x + k * T;
       if (k >= EPT || (!FULL && e >= N * KC)) continue;
       const int kcol = e % KC, zz = e / KC;
-      if (!Z::KFULL && kcol >= kcn) continue;
-      const int kx = kx0 + kcol;
       X v[3];
 #pragma unroll
-      for (int c = 0; c < 3; ++c) v[c] = cols[(c * N + zz) * KC + kcol];
+      for (int c = 0; c < 3; ++c) v[c] = cols[Z::slot(c * N + zz, kcol)];
       if (shat_d) {
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
@@ -438,7 +447,7 @@ void fz_static(FFTArgsT<R> A) {
       w[0] = c2(g0 * v[0].x + g3 * v[1].x + g4 * v[2].x, g0 * v[0].y + g3 * v[1].y + g4 * v[2].y);
       w[1] = c2(g3 * v[0].x + g1 * v[1].x + g5 * v[2].x, g3 * v[0].y + g1 * v[1].y + g5 * v[2].y);
       w[2] = c2(g4 * v[0].x + g5 * v[1].x + g2 * v[2].x, g4 * v[0].y + g5 * v[1].y + g2 * v[2].y);
-      const double wgt = (kx == 0 || kx == N / 2) ? 1.0 : 2.0;
+      const double wgt = (nyq || kx0 + kcol == 0) ? 1.0 : 2.0;
       double t = 0.0;
 #pragma unroll
       for (int c = 0; c < 3; ++c) t += double(v[c].x) * double(w[c].x) + double(v[c].y) * double(w[c].y);
@@ -449,15 +458,12 @@ void fz_static(FFTArgsT<R> A) {
           sw[c] = fma(wgt, double(sh[i][c].x) * double(w[c].x) + double(sh[i][c].y) * double(w[c].y), sw[c]);
       }
 #pragma unroll
-      for (int c = 0; c < 3; ++c) cols[(c * N + zz) * KC + kcol] = w[c];
+      for (int c = 0; c < 3; ++c) cols[Z::slot(c * N + zz, kcol)] = w[c];
     }
   }
   __syncthreads();
   sfft<true, N, typename Z::ZCols, T, PLAN>(cols, tw, 1);
-  for (int e = threadIdx.x; e < 3 * N * KC; e += T) {
-    const int kcol = e % KC, cz = e / KC;
-    if (Z::KFULL || kcol < kcn) S[(int64_t(cz) * N + y) * NKX + kx0 + kcol] = cols[e];
-  }
+  for (int e = threadIdx.x; e < 3 * N * KC; e += T) S[e / KC * sstep + e % KC * scol] = cols[Z::slot(e / KC, e % KC)];
   double t[4] = {rz, sw[0], sw[1], sw[2]};
   block_sums<4>(t, red);
   if (threadIdx.x == 0) {
@@ -470,32 +476,54 @@ void fz_static(FFTArgsT<R> A) {
   }
 }
 
-// ------------------------------------------------------- z + Green, in registers (n = 64)
-// The z pass of the 64^3 cube with its transforms in registers. A block is three waves, wave c holding
-// component c of 8 kx columns of one ky row (the Nyquist blocks: column kx = 32 of 8 ky rows); lane
-// (kcol = lane % 8, j = lane / 8) holds the points kz = j + 8 r (r < 8) of its column. The 64-point
-// transform is two radix-8 Stockham passes: pass 1 is a DFT over the lane's own points, an 8 x 8 transpose
-// among the 8 lanes of a column goes through LDS, and pass 2 (twiddles W^(j r)) leaves the lane with the
-// frequencies kz = j + 8 r: the same points the first inverse pass reads. LDS carries the two transposes of
-// each transform and the exchange of the three components for the 3x3 Green multiply; the default pass
-// stages every point through LDS for each of its radix stages. Semantics are those of fz_static.
-template <int MODE, typename R>
-__global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void fz64_reg(FFTArgsT<R> A) {
-  // LDS rows of one column, padded so that the 16 lanes (8 columns x 2 j) of a transposed or exchange read
-  // of 16-byte values fall on distinct banks
-  constexpr int N = 64, NKX = N / 2 + 1, RS = N + 2;
-  constexpr int64_t NF = int64_t(N) * N * NKX;
+// ------------------------------------------------------------- z + Green, in registers
+// The z pass of a cube n = 8 P with its transforms in registers and no barrier between its phases. A wave holds 8
+// columns of one ky row (the Nyquist blocks: 8 ky of kx = n/2), all three components; lane (col, j) the points
+// kz = j + 8 r (r < P) of its column. With k = P a + b,
+//   X[P a + b] = sum_j W_8^(j a) [ W_n^(j b) sum_r W_P^(r b) x[j + 8 r] ]:
+// a P-point transform in the lane, a twiddle, one exchange among the 8 lanes of the column through LDS, and 8-point
+// transforms for b = j + 8 q that leave the lane every component of its frequencies, so the Green multiply needs no
+// exchange either (where P is no multiple of 8 the last group leaves lanes idle); the inverse mirrors it. LDS carries
+// each point four times instead of the 16 of the staged pass (fz_static), and a wave's 24 (64^3) or 48 loads are all in
+// flight at once. Bound by memory from three loads on: 128^3 FP64, three loads, 140 us for 450 MB of spectrum, symbol
+// and scale spectrum; by its own chain of loads, exchanges and stores on fewer (zkc_of has the times on both sides).
+
+// Cubes whose columns divide into whole waves of the register-resident z pass.
+template <int N>
+constexpr bool zreg() { return N % 16 == 0; }
+
+template <int N>
+struct ZReg {
+  static constexpr int P = N / 8, Q = (P + 7) / 8;
+  static constexpr int BS = 8 * 8 + 8;      // row of one b: [j][col], padded by half the banks
+  template <typename R>
+  static constexpr size_t lds() { return size_t(8 * Q) * BS * 2 * sizeof(R); }
+  // Blocks of one wave: blocks of four with one row of partials each measured slower (128^3 FP32, three loads: 104 us
+  // against 78 us), their 260 blocks per load leave CUs one block longer than others.
+  static constexpr int BLOCKS = N / 16 * N + N / 8;
+};
+
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int N, int MODE, typename R, int EU, bool SCALED>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(EU))) void fz_reg(FFTArgsT<R> A) {
   using X = cplx<R>;
+  using Z = ZReg<N>;
+  constexpr int P = Z::P, NKX = N / 2 + 1, Q = Z::Q;
+  constexpr bool ALL = P % 8 == 0;   // else the last group of frequencies b = j + 8 q leaves lanes with b >= P idle
+  constexpr int64_t NF = int64_t(N) * N * NKX;
   extern __shared__ __align__(16) unsigned char smem[];
-  X* buf = reinterpret_cast<X*>(smem);                       // [component][kcol][RS]
-  X* twl = buf + 3 * 8 * RS;                                  // W_64^k, k < 64
-  double* red = reinterpret_cast<double*>(twl + N);           // block sums: 4 values x 3 waves
-  const int c = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
-  const int lane = int(threadIdx.x) & 63, kcol = lane & 7, j = lane >> 3;
-  const int b = int(blockIdx.x), l = int(blockIdx.z);
-  const int ky = b < 256 ? b % 64 : 8 * (b - 256) + kcol;
-  const int kx = b < 256 ? 8 * (b / 64) + kcol : N / 2;
-  const bool lead = threadIdx.x == 0 && b == 0;
+  X* buf = reinterpret_cast<X*>(smem);
+  const int lane = threadIdx.x, col = lane & 7, j = lane >> 3;
+  const int blk = blockIdx.x, l = blockIdx.z;
+  const bool nyq = blk >= N / 16 * N;
+  const int y = nyq ? (blk - N / 16 * N) * 8 : blk % N;     // ky of column 0
+  const int kx0 = nyq ? N / 2 : blk / N * 8;                // kx of column 0
+  const bool lead = lane == 0 && blk == 0;
   const int64_t NN = int64_t(N) * N * N;
   if (MODE == kFzPCG && !A.st.active[l]) {
     if (lead) {
@@ -506,128 +534,202 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void f
     }
     return;
   }
-  X* S = A.spec + int64_t(l) * 3 * NF;
-  auto fidx = [&](int kz) { return (int64_t(kz) * N + ky) * NKX + kx; };
-  // the column's points and the twiddle table are in flight through the convergence test
-  X v[8];
+  // frequency (kz, column) in the rows of N/2 + 1 values of the symbol and s_hat, and in the spectrum (the scale pass
+  // transforms s_hat in place)
+  const int fcol = nyq ? NKX : 1;
+  const bool packed = MODE != kFzScale;
+  const int sstep = !packed ? N * NKX : nyq ? N : N * (N / 2);
+  // uniform base and row offsets, one 32-bit offset per lane
+  X* S = A.spec + int64_t(l) * 3 * NF +
+         (!packed ? int64_t(y * NKX + kx0) : nyq ? Spec<N>::MAIN + y : int64_t(y) * (N / 2) + kx0);
+  const unsigned so = unsigned(j * sstep + col * (packed ? 1 : fcol));
+  int bq[Q];   // b of the lane's groups, in range also for the idle lanes
+  bool on[Q];
 #pragma unroll
-  for (int r = 0; r < 8; ++r) v[r] = S[int64_t(c) * NF + fidx(j + 8 * r)];
-  const X twv = A.twz[lane];
-  // s_hat_c at the lane's frequencies, in flight through the convergence test and the forward transform
-  const X* __restrict__ shat_d = A.shat ? A.shat + int64_t(design_of(l, A.group)) * 3 * NF : nullptr;
-  X sh[8];
-  if (MODE != kFzScale) {
-#pragma unroll
-    for (int r = 0; r < 8; ++r) sh[r] = shat_d ? shat_d[int64_t(c) * NF + fidx(j + 8 * r)] : c2(R(0), R(0));
+  for (int q = 0; q < Q; ++q) {
+    on[q] = ALL || j + 8 * q < P;
+    bq[q] = on[q] ? j + 8 * q : P - 1;
   }
-  double mean_c = 0.0;
-  if (MODE == kFzInit || MODE == kFzPCG) {
-    double res2 = 0.0, vm = 0.0;
-    {
-      double t = 0.0, m = 0.0;
-      for (int i = lane; i < N; i += 64) {
-        const double* p = A.pr + (int64_t(l) * N + i) * 6;
-        t += (p[0] + p[2]) + p[4];
-        m += p[2 * c + 1];
-      }
-      res2 = wave_sum(t);
-      vm = wave_sum(m);
+  unsigned fo[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) fo[q] = unsigned(bq[q] * (N * NKX) + col * fcol);
+  X v[3][P > 8 * Q ? P : 8 * Q];
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+#pragma unroll
+    for (int r = 0; r < P; ++r) v[c][r] = (S + (c * N + 8 * r) * sstep)[so];
+  __builtin_amdgcn_sched_barrier(0);
+  X tw[P];   // W_n^(j b)
+#pragma unroll
+  for (int b = 1; b < P; ++b) tw[b] = A.twz[j * b];
+  __builtin_amdgcn_sched_barrier(0);
+  double mean[3] = {0.0, 0.0, 0.0};
+  if (MODE != kFzScale) {
+    double ss = 0.0, vm[3] = {0.0, 0.0, 0.0};
+    for (int i = lane; i < N; i += 64) {
+      const double* p = A.pr + (int64_t(l) * N + i) * 6;
+      ss += (p[0] + p[2]) + p[4];
+      vm[0] += p[1];
+      vm[1] += p[3];
+      vm[2] += p[5];
     }
-    if (A.shat) mean_c = vm / double(NN);
-    bool act;
-    if (MODE == kFzInit) {
-      act = res2 > A.st.target2[l] && A.st.it[l] < A.st.cap[l] && !A.st.bad[l];
-      if (lead) {
-        A.st.active_next[l] = act;
-        A.st.it_next[l] = A.st.it[l];
-        A.st.bad_next[l] = A.st.bad[l];
-        A.st.first[l] = 1;
-        A.st.stopped[l] = 0;
-      }
-    } else {
-      const bool active = A.st.active[l] != 0;
-      const bool valid = A.st.valid[l] != 0;
-      const bool finite = isfinite(res2);
-      const int64_t it = A.st.it[l] + (active ? 1 : 0);
-      act = active && valid && finite && res2 > A.st.target2[l] && it < A.st.cap[l];
+    if (SCALED)
+      for (int c = 0; c < 3; ++c) mean[c] = wave_sum(vm[c]) / double(NN);
+    if (MODE != kFzPre) {
+      const double res2 = wave_sum(ss);
+      const int64_t it0 = A.st.it[l];
+      const bool bad = A.st.bad[l] != 0;
+      // the initialization's test, or the iteration's (the active mask was tested above; `valid` was set by the forward
+      // pass of this iteration)
+      const bool valid = MODE == kFzInit || A.st.valid[l] != 0, finite = isfinite(res2);
+      const int64_t it = it0 + (MODE == kFzPCG ? 1 : 0);
+      const bool act = valid && res2 > A.st.target2[l] && it < A.st.cap[l] && (MODE == kFzInit ? !bad : finite);
       if (lead) {
         A.st.active_next[l] = act;
         A.st.it_next[l] = it;
-        A.st.bad_next[l] = A.st.bad[l] || (active && !valid) || (active && !finite);
-        A.st.stopped[l] = active && !act;
+        A.st.bad_next[l] = bad || (MODE == kFzPCG && !(valid && finite));
+        A.st.stopped[l] = MODE == kFzPCG && !act;
+        if (MODE == kFzInit) A.st.first[l] = 1;
+      }
+      if (!act) return;
+    }
+  }
+  // symbol and s_hat of the lane's frequencies, fetched GS at a time: the first group before the transforms, each later
+  // one before the group in hand is used (when needed where P > 8 leaves no registers for that). The scheduling
+  // barriers keep it so: moved further up the loads would take the registers of the transforms, further down nothing
+  // would cover them.
+  constexpr int GS = 2;
+  const X* __restrict__ shat_d = SCALED ? A.shat + int64_t(design_of(l, A.group)) * 3 * NF + y * NKX + kx0 : nullptr;
+  const R* __restrict__ sym = A.sym + y * NKX + kx0;
+  R g[2][GS][6];
+  X sh[2][GS][3];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < GS; ++i) {
+      const int k = k0 + i, f = P * (k & 7) * (N * NKX);
+#pragma unroll
+      for (int m = 0; m < 6; ++m) g[k0 / GS & 1][i][m] = (sym + (m * NF + f))[fo[k >> 3]];
+      if (SCALED) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) sh[k0 / GS & 1][i][c] = (shat_d + (c * NF + f))[fo[k >> 3]];
       }
     }
-    if (!act) return;
-  } else if (MODE != kFzScale && A.shat) {
-    mean_c = wave_reduce_partials(A.pr + (int64_t(l) * N * 3 + c) * 2 + 1, N, 6) / double(NN);
-  }
-  if (c == 0) twl[lane] = twv;
-  X* row = buf + (c * 8 + kcol) * RS;
+  };
+  constexpr bool AHEAD = P <= 8;
+  __builtin_amdgcn_sched_barrier(0);
+  if (MODE != kFzScale && AHEAD) fetch(0);
   const X* none = nullptr;
-  // forward: pass 1 over x[j + 8 r] -> y[8 j + r], transpose, pass 2 (twiddles W^(j r)) -> Y[j + 8 r]
-  dft<8, false>(v, none, N, 1);
 #pragma unroll
-  for (int r = 0; r < 8; ++r) row[8 * j + r] = v[r];
-  // this wave's row of the symbol (G_c0, G_c1, G_c2 of [G00, G11, G22, G01, G02, G12]), in flight through
-  // the transpose, the second pass and the component exchange
-  R g[8][3];
-  if (MODE != kFzScale) {
+  for (int c = 0; c < 3; ++c) {
+    __builtin_amdgcn_sched_barrier(0);
+    X u[P];
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      const int64_t f = fidx(j + 8 * r);
+    for (int r = 0; r < P; ++r) u[r] = v[c][r];
+    dft<P, false>(u, none, N, 1);
 #pragma unroll
-      for (int d = 0; d < 3; ++d) g[r][d] = A.sym[(d == c ? c : c + d + 2) * NF + f];
+    for (int b = 0; b < P; ++b) buf[b * Z::BS + j * 8 + col] = b == 0 ? u[0] : cmul(u[b], tw[b]);
+    wave_lds_fence();
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      X w[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) w[i] = buf[bq[q] * Z::BS + i * 8 + col];
+      dft<8, false>(w, none, N, 1);
+#pragma unroll
+      for (int a = 0; a < 8; ++a) v[c][8 * q + a] = w[a];   // frequency kz = P a + b
     }
+    wave_lds_fence();
   }
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < 8; ++r) v[r] = r == 0 ? row[j] : cmul(row[j + 8 * r], twl[(j * r) & (N - 1)]);
-  dft<8, false>(v, none, N, 1);
   if (MODE == kFzScale) {
 #pragma unroll
-    for (int r = 0; r < 8; ++r) S[int64_t(c) * NF + fidx(j + 8 * r)] = v[r];
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        if (on[q]) {
+#pragma unroll
+          for (int a = 0; a < 8; ++a)
+            (S + (c * N + P * a) * sstep)[unsigned(bq[q] * sstep + col * (packed ? 1 : fcol))] = v[c][8 * q + a];
+        }
     return;
   }
-  // projection mean correction, then the three components meet in LDS for the Green multiply
-  if (shat_d) {
-    const R mc = R(mean_c);
+  const double wgt = (nyq || kx0 + col == 0) ? 1.0 : 2.0;
+  double rz = 0.0, sw[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-    for (int r = 0; r < 8; ++r) v[r] = c2(fma(-mc, sh[r].x, v[r].x), fma(-mc, sh[r].y, v[r].y));
+  for (int k0 = 0; k0 < 8 * Q; k0 += GS) {
+    __builtin_amdgcn_sched_barrier(0);
+    if (!AHEAD) fetch(k0);
+    else if (k0 + GS < 8 * Q) fetch(k0 + GS);
+    const int bf = k0 / GS & 1;
+#pragma unroll
+    for (int i = 0; i < GS; ++i) {
+      __builtin_amdgcn_sched_barrier(0);
+      X x[3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const R mc = R(mean[c]);
+        x[c] = v[c][k0 + i];
+        if (SCALED) x[c] = c2(fma(-mc, sh[bf][i][c].x, x[c].x), fma(-mc, sh[bf][i][c].y, x[c].y));
+      }
+      const R g0 = g[bf][i][0], g1 = g[bf][i][1], g2 = g[bf][i][2], g3 = g[bf][i][3], g4 = g[bf][i][4],
+              g5 = g[bf][i][5];
+      X w[3];
+      w[0] = c2(g0 * x[0].x + g3 * x[1].x + g4 * x[2].x, g0 * x[0].y + g3 * x[1].y + g4 * x[2].y);
+      w[1] = c2(g3 * x[0].x + g1 * x[1].x + g5 * x[2].x, g3 * x[0].y + g1 * x[1].y + g5 * x[2].y);
+      w[2] = c2(g4 * x[0].x + g5 * x[1].x + g2 * x[2].x, g4 * x[0].y + g5 * x[1].y + g2 * x[2].y);
+      double t = 0.0;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) t += double(x[c].x) * double(w[c].x) + double(x[c].y) * double(w[c].y);
+      const double wk = on[(k0 + i) >> 3] ? wgt : 0.0;
+      rz = fma(wk, t, rz);
+      if (SCALED) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+          sw[c] = fma(wk, double(sh[bf][i][c].x) * double(w[c].x) + double(sh[bf][i][c].y) * double(w[c].y), sw[c]);
+      }
+#pragma unroll
+      for (int c = 0; c < 3; ++c) v[c][k0 + i] = w[c];
+    }
   }
-  // a lane writes back exactly the slots it read after the transpose: no other lane reads them again
+  __builtin_amdgcn_sched_barrier(0);
+  // the twiddles are read again and the rows' offsets formed again (an opaque copy of what they derive from): held
+  // through the multiply they would cost its registers
+  const X* twz = A.twz;
+  unsigned so2 = so;
+  asm volatile("" : "+s"(twz), "+v"(so2));
 #pragma unroll
-  for (int r = 0; r < 8; ++r) row[j + 8 * r] = v[r];
-  __syncthreads();
-  const double wgt = (kx == 0 || kx == N / 2) ? 1.0 : 2.0;
-  double rz = 0.0, sw = 0.0;
-  X w[8];
+  for (int b = 1; b < P; ++b) tw[b] = twz[j * b];
 #pragma unroll
-  for (int r = 0; r < 8; ++r) {
-    const int kz = j + 8 * r;
-    const X v0 = buf[(0 * 8 + kcol) * RS + kz], v1 = buf[(1 * 8 + kcol) * RS + kz], v2 = buf[(2 * 8 + kcol) * RS + kz];
-    w[r] = c2(g[r][0] * v0.x + g[r][1] * v1.x + g[r][2] * v2.x, g[r][0] * v0.y + g[r][1] * v1.y + g[r][2] * v2.y);
-    rz = fma(wgt, double(v[r].x) * double(w[r].x) + double(v[r].y) * double(w[r].y), rz);
-    if (shat_d) sw = fma(wgt, double(sh[r].x) * double(w[r].x) + double(sh[r].y) * double(w[r].y), sw);
+  for (int c = 0; c < 3; ++c) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      X w[8];
+#pragma unroll
+      for (int a = 0; a < 8; ++a) w[a] = v[c][8 * q + a];
+      dft<8, true>(w, none, N, 1);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) buf[(j + 8 * q) * Z::BS + i * 8 + col] = w[i];   // rows b >= P are not read
+    }
+    wave_lds_fence();
+    X u[P];
+#pragma unroll
+    for (int b = 0; b < P; ++b) {
+      const X x = buf[b * Z::BS + j * 8 + col];
+      u[b] = b == 0 ? x : cmul(x, conjd(tw[b]));
+    }
+    wave_lds_fence();
+    dft<P, true>(u, none, N, 1);
+#pragma unroll
+    for (int r = 0; r < P; ++r) (S + (c * N + 8 * r) * sstep)[so2] = u[r];
   }
-  __syncthreads();  // the exchange rows are read before the inverse transposes overwrite them
-  // inverse: pass 1 over W[j + 8 r] -> 8 j + r, transpose, pass 2 with conjugate twiddles -> z = j + 8 r
-  dft<8, true>(w, none, N, 1);
+  rz = wave_sum(rz);
 #pragma unroll
-  for (int r = 0; r < 8; ++r) row[8 * j + r] = w[r];
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < 8; ++r) w[r] = r == 0 ? row[j] : cmul(row[j + 8 * r], conjd(twl[(j * r) & (N - 1)]));
-  dft<8, true>(w, none, N, 1);
-#pragma unroll
-  for (int r = 0; r < 8; ++r) S[int64_t(c) * NF + fidx(j + 8 * r)] = w[r];
-  double t[4] = {rz, c == 0 ? sw : 0.0, c == 1 ? sw : 0.0, c == 2 ? sw : 0.0};
-  block_sums<4>(t, red);
-  if (threadIdx.x == 0) {
-    double* pg = A.pg + (int64_t(l) * A.f.nkb * N + b) * 4;
-    pg[0] = t[0];
-    pg[1] = t[1];
-    pg[2] = t[2];
-    pg[3] = t[3];
+  for (int c = 0; c < 3; ++c) sw[c] = wave_sum(sw[c]);
+  if (lane == 0) {
+    // per-load partials are laid out with the geometry's chunk count (slices of a set are offset by it)
+    double* pg = A.pg + (int64_t(l) * A.f.nkb * N + blk) * 4;
+    pg[0] = rz;
+    for (int c = 0; c < 3; ++c) pg[1 + c] = sw[c];
   }
 }
 
@@ -667,9 +769,11 @@ void fxyi_static(FFTArgsT<R> A) {
     return;
   }
   // the half spectrum of the plane stays in flight through the mean and beta reductions
-  StageIn<N * C::NKX, T, X> in;
-  StageIn<N, T, X> twl;
-  in.load(A.spec + ((int64_t(l) * 3 + c) * N + z) * int64_t(N) * C::NKX, [](int e) { return e; });
+  StageIn<N * C::M, T, X> in;
+  StageIn<N, T, X> nyq, twl;
+  const X* __restrict__ spec = A.spec + int64_t(l) * 3 * C::NF;
+  in.load(spec + (int64_t(c) * N + z) * (N * C::M), [](int e) { return e; });
+  nyq.load(spec + Spec<N>::MAIN + (int64_t(c) * N + z) * N, [](int e) { return e; });
   twl.load(A.twy, [](int e) { return e; });
   const int NSLOT = A.zslots;
   // per-load partials are laid out with the geometry's chunk count (slices of a set are offset by it)
@@ -680,15 +784,25 @@ void fxyi_static(FFTArgsT<R> A) {
   if (A.shat || update) {
     // one pass: r.z (offset 0) and this component's s.w (offset 1 + c) partials
     const int off[2] = {0, 1 + c};
-    double sums[2];
-    wave_reduce_partials_n<2>(pgl, off, NSLOT, 4, sums);
+    double sums[2] = {0.0, 0.0};
+    // (FP64 holds too many of its loads in registers here to share the sums: 128^3 three loads 249 against 208 us)
+    if (C::SHARED_SUMS && sizeof(R) == 4) {
+      for (int k = threadIdx.x; k < NSLOT; k += T) {
+        sums[0] += pgl[4 * k];
+        sums[1] += pgl[4 * k + 1 + c];
+      }
+      block_sums<2>(sums, reinterpret_cast<double*>(tw + N));
+    } else {
+      wave_reduce_partials_n<2>(pgl, off, NSLOT, 4, sums);
+    }
     if (A.shat) mean = sums[1] / double(NN);
     if (update) {
       const double rz = A.st.rz[l];
       beta = sums[0] / (rz != 0.0 ? rz : 1.0);
     }
   }
-  in.store(plane);
+  in.store(plane, [](int e) { return e / C::M * C::RS + e % C::M; });
+  nyq.store(plane, [](int y) { return y * C::RS + C::M; });
   twl.store(tw);
   // output streams: every load of a chunk is issued before the first use; in
   // FP32 the first chunk is issued before the inverse transforms and stays in
@@ -812,12 +926,12 @@ int fxy_static_n(FFTArgsT<R>& A, int L, int mode, hipStream_t s) {
   dim3 grid(N, 3, L), block(C::TXY);
   switch (mode) {
     case kFxyScale:
-      if (int e = allow_lds_static((fxy_static<N, kFxyScale, R, default_plan<N>(0)>), lds)) return e;
-      hipLaunchKernelGGL((fxy_static<N, kFxyScale, R, default_plan<N>(0)>), grid, block, lds, s, A);
+      if (int e = allow_lds_static((fxy_static<N, kFxyScale, R, default_plan<N>()>), lds)) return e;
+      hipLaunchKernelGGL((fxy_static<N, kFxyScale, R, default_plan<N>()>), grid, block, lds, s, A);
       break;
     case kFxyPre:
-      if (int e = allow_lds_static((fxy_static<N, kFxyPre, R, default_plan<N>(0)>), lds)) return e;
-      hipLaunchKernelGGL((fxy_static<N, kFxyPre, R, default_plan<N>(0)>), grid, block, lds, s, A);
+      if (int e = allow_lds_static((fxy_static<N, kFxyPre, R, default_plan<N>()>), lds)) return e;
+      hipLaunchKernelGGL((fxy_static<N, kFxyPre, R, default_plan<N>()>), grid, block, lds, s, A);
       break;
     default:
       if (plan_of<N, R>(0) == 1) {
@@ -832,66 +946,65 @@ int fxy_static_n(FFTArgsT<R>& A, int L, int mode, hipStream_t s) {
   return PGJ_OK;
 }
 
-template <int N, typename R, int KCX>
+template <int N, typename R, int KC>
 int fz_static_kc(FFTArgsT<R>& A, int L, int mode, hipStream_t s) {
-  using Z = ZPass<N, R, KCX>;
+  using Z = ZPass<N, R, KC>;
   const size_t lds = Z::lds;
   // the per-block partials are laid out for the geometry's chunk count
-  PGJ_REQUIRE(Z::NKB <= A.f.nkb, "z pass chunks (%d) exceed the partial layout (%d)", Z::NKB, A.f.nkb);
-  dim3 grid(N, Z::NKB, L), block(Z::TZ);
+  PGJ_REQUIRE(Z::BLOCKS <= A.f.nkb * N, "z pass blocks (%d) exceed the partial layout (%d)", Z::BLOCKS, A.f.nkb * N);
+  dim3 grid(Z::BLOCKS, 1, L), block(Z::TZ);
   switch (mode) {
     case kFzScale:
-      if (int e = allow_lds_static(fz_static<N, kFzScale, R, KCX, default_plan<N>(1)>, lds)) return e;
-      hipLaunchKernelGGL((fz_static<N, kFzScale, R, KCX, default_plan<N>(1)>), grid, block, lds, s, A);
+      if (int e = allow_lds_static(fz_static<N, kFzScale, R, KC, default_plan<N>()>, lds)) return e;
+      hipLaunchKernelGGL((fz_static<N, kFzScale, R, KC, default_plan<N>()>), grid, block, lds, s, A);
       break;
     case kFzPre:
-      if (int e = allow_lds_static(fz_static<N, kFzPre, R, KCX, default_plan<N>(1)>, lds)) return e;
-      hipLaunchKernelGGL((fz_static<N, kFzPre, R, KCX, default_plan<N>(1)>), grid, block, lds, s, A);
+      if (int e = allow_lds_static(fz_static<N, kFzPre, R, KC, default_plan<N>()>, lds)) return e;
+      hipLaunchKernelGGL((fz_static<N, kFzPre, R, KC, default_plan<N>()>), grid, block, lds, s, A);
       break;
     case kFzInit:
-      if (int e = allow_lds_static(fz_static<N, kFzInit, R, KCX, default_plan<N>(1)>, lds)) return e;
-      hipLaunchKernelGGL((fz_static<N, kFzInit, R, KCX, default_plan<N>(1)>), grid, block, lds, s, A);
+      if (int e = allow_lds_static(fz_static<N, kFzInit, R, KC, default_plan<N>()>, lds)) return e;
+      hipLaunchKernelGGL((fz_static<N, kFzInit, R, KC, default_plan<N>()>), grid, block, lds, s, A);
       break;
     default:
       if (plan_of<N, R>(1) == 1) {
-        if (int e = allow_lds_static(fz_static<N, kFzPCG, R, KCX, 1>, lds)) return e;
-        hipLaunchKernelGGL((fz_static<N, kFzPCG, R, KCX, 1>), grid, block, lds, s, A);
+        if (int e = allow_lds_static(fz_static<N, kFzPCG, R, KC, 1>, lds)) return e;
+        hipLaunchKernelGGL((fz_static<N, kFzPCG, R, KC, 1>), grid, block, lds, s, A);
       } else {
-        if (int e = allow_lds_static(fz_static<N, kFzPCG, R, KCX>, lds)) return e;
-        hipLaunchKernelGGL((fz_static<N, kFzPCG, R, KCX>), grid, block, lds, s, A);
+        if (int e = allow_lds_static(fz_static<N, kFzPCG, R, KC>, lds)) return e;
+        hipLaunchKernelGGL((fz_static<N, kFzPCG, R, KC>), grid, block, lds, s, A);
       }
   }
   PGJ_LAUNCHED("fz_static");
   return PGJ_OK;
 }
 
-template <typename R>
-int fz64_reg_launch(FFTArgsT<R>& A, int L, int mode, hipStream_t s) {
-  constexpr size_t lds = (size_t(3) * 8 * 66 + 64) * sizeof(cplx<R>) + 4 * 8 * sizeof(double);
-  PGJ_REQUIRE(kZRegBlocks <= A.f.nkb * 64, "z pass blocks (%d) exceed the partial layout (%d)", kZRegBlocks,
-              A.f.nkb * 64);
-  const dim3 grid(kZRegBlocks, 1, L), block(192);
+template <int N, typename R, int EU, bool SCALED>
+int fz_reg_launch(FFTArgsT<R>& A, int L, int mode, hipStream_t s) {
+  constexpr size_t lds = ZReg<N>::template lds<R>();
+  PGJ_REQUIRE(ZReg<N>::BLOCKS <= A.f.nkb * N, "z pass blocks (%d) exceed the partial layout (%d)", ZReg<N>::BLOCKS,
+              A.f.nkb * N);
+  const dim3 grid(ZReg<N>::BLOCKS, 1, L), block(64);
   switch (mode) {
-    case kFzScale: hipLaunchKernelGGL((fz64_reg<kFzScale, R>), grid, block, lds, s, A); break;
-    case kFzPre: hipLaunchKernelGGL((fz64_reg<kFzPre, R>), grid, block, lds, s, A); break;
-    case kFzInit: hipLaunchKernelGGL((fz64_reg<kFzInit, R>), grid, block, lds, s, A); break;
-    default: hipLaunchKernelGGL((fz64_reg<kFzPCG, R>), grid, block, lds, s, A);
+    case kFzScale: hipLaunchKernelGGL((fz_reg<N, kFzScale, R, EU, false>), grid, block, lds, s, A); break;
+    case kFzPre: hipLaunchKernelGGL((fz_reg<N, kFzPre, R, EU, SCALED>), grid, block, lds, s, A); break;
+    case kFzInit: hipLaunchKernelGGL((fz_reg<N, kFzInit, R, EU, SCALED>), grid, block, lds, s, A); break;
+    default: hipLaunchKernelGGL((fz_reg<N, kFzPCG, R, EU, SCALED>), grid, block, lds, s, A);
   }
-  PGJ_LAUNCHED("fz64_reg");
+  PGJ_LAUNCHED("fz_reg");
   return PGJ_OK;
 }
 
 template <int N, typename R>
 int fz_static_n(FFTArgsT<R>& A, int L, int mode, hipStream_t s) {
   using W = ZWidths<N, R>;
-  if constexpr (N == 64) {
-    if (A.zkc == 0) return fz64_reg_launch<R>(A, L, mode, s);
+  if constexpr (zreg<N>()) {
+    constexpr int waves = sizeof(R) == 8 ? (N > 64 ? 1 : 2) : N > 64 ? 2 : 3;
+    if (A.zkc == 0)
+      return A.shat ? fz_reg_launch<N, R, waves, true>(A, L, mode, s) : fz_reg_launch<N, R, waves, false>(A, L, mode, s);
   }
   if constexpr (W::wide != W::def) {
     if (A.zkc == W::wide) return fz_static_kc<N, R, W::wide>(A, L, mode, s);
-  }
-  if constexpr (W::narrow != W::def) {
-    if (A.zkc == W::narrow) return fz_static_kc<N, R, W::narrow>(A, L, mode, s);
   }
   return fz_static_kc<N, R, W::def>(A, L, mode, s);
 }
@@ -912,18 +1025,23 @@ static int device_cus() {
 bool zpass_wide(const pgj_grid& g, int L, int es) {
   if (es != 8 || !static_cube(g) || g.nx != 64 || L < 1) return false;
   const int64_t cus = device_cus();
-  using Zn = ZPass<64, double>;
-  const int64_t narrow = int64_t(Zn::NKB) * 64 * L;  // blocks of the default pass
-  return cus > 0 && narrow > cus * Zn::per_cu;
+  using Zn = ZPass<64, double, ZWidths<64, double>::wide>;
+  return cus > 0 && int64_t(Zn::BLOCKS) * L > cus * Zn::per_cu;
 }
 
+// The z pass of a workspace: 0 = in registers (fz_reg), else the chunk width of the LDS pass. In registers by default
+// wherever the columns divide into its waves; the LDS pass by an explicit radix plan, for the ragged cube, and for one
+// FP64 load at 64^3, whose 264 waves leave most SIMDs idle on a long chain of their own. Graph-replayed launches of one,
+// three and six loads, LDS -> registers (us): 32^3 FP64 6.2 / 7.2 / 9.2 -> 6.4 / 6.5 / 7.0, 48^3 FP64 8.4 / 12.9 / 18.8 ->
+// 7.4 / 11.7 / 16.1, 64^3 FP64 11.9 / 20.5 / 30.6 -> 13.3 / 18.7 / 26.1, 64^3 FP32 9.5 / 15.4 / 23.8 -> 8.8 / 12.8 / 18.4,
+// 96^3 FP64 31.7 / 68.6 / 127 -> 28.2 / 60.9 / 114, 96^3 FP32 23.7 / 43 / 73 -> 23.3 / 34.4 / 63.8, 128^3 FP64
+// 61 / 151 / 295 -> 58 / 140 / 275, 128^3 FP32 49 / 99 / 175 -> 38 / 79 / 163.
 template <int N, typename R>
 static int zkc_of(const pgj_grid& g, int L) {
   using W = ZWidths<N, R>;
-  if (N == 64 && fft_plan(64, int(sizeof(R)), 1) == 2) return 0;
-  if (W::wide != W::def && zpass_wide(g, L, int(sizeof(R)))) return W::wide;
-  if (W::narrow != W::def && 2 * int64_t(ZPass<N, R>::NKB) * N * L <= 5 * int64_t(device_cus())) return W::narrow;
-  return W::def;
+  const int plan = fft_plan(N, int(sizeof(R)), 1);
+  if (zreg<N>() && (plan == 2 || (plan < 0 && !(N == 64 && sizeof(R) == 8 && L == 1)))) return 0;
+  return W::wide != W::def && zpass_wide(g, L, int(sizeof(R))) ? W::wide : W::def;
 }
 
 template <typename R>
@@ -942,8 +1060,7 @@ void zpass_choose(FFTArgsT<R>& A, const pgj_grid& g, int L) {
     case 96: A.zkc = zkc_of<96, R>(g, L); break;
     default: A.zkc = zkc_of<128, R>(g, L); break;
   }
-  const int nkx = g.nx / 2 + 1;
-  A.zslots = A.zkc == 0 ? kZRegBlocks : ((nkx + A.zkc - 1) / A.zkc) * g.nx;
+  A.zslots = A.zkc == 0 ? g.nx / 16 * g.nx + g.nx / 8 : g.nx / 2 / A.zkc * g.nx + g.nx / A.zkc;
 }
 template void zpass_choose<double>(FFTArgsT<double>&, const pgj_grid&, int);
 template void zpass_choose<float>(FFTArgsT<float>&, const pgj_grid&, int);
@@ -961,8 +1078,8 @@ int fxyi_static_n(FFTArgsT<R>& A, int L, int mode, hipStream_t s) {
   using C = Cube<N>;
   const size_t lds = C::lds_xy(sizeof(cplx<R>));
   if (mode == kFxyiPre) {
-    if (int e = allow_lds_static(fxyi_static<N, kFxyiPre, R, default_plan<N>(2)>, lds)) return e;
-    hipLaunchKernelGGL((fxyi_static<N, kFxyiPre, R, default_plan<N>(2)>), dim3(N, 3, L), dim3(C::TXY), lds, s, A);
+    if (int e = allow_lds_static(fxyi_static<N, kFxyiPre, R, default_plan<N>()>, lds)) return e;
+    hipLaunchKernelGGL((fxyi_static<N, kFxyiPre, R, default_plan<N>()>), dim3(N, 3, L), dim3(C::TXY), lds, s, A);
   } else if (plan_of<N, R>(2) == 1) {
     if (int e = allow_lds_static(fxyi_static<N, kFxyiPCG, R, 1>, lds)) return e;
     hipLaunchKernelGGL((fxyi_static<N, kFxyiPCG, R, 1>), dim3(N, 3, L), dim3(C::TXY), lds, s, A);

@@ -188,16 +188,15 @@ inline FFTGeom fft_geom(const pgj_grid& g) {
   int kc = 1;
   while (kc < f.nkx && size_t(kc + 1) * col + 64 * 8 <= 56 * 1024) ++kc;
   if (g.nx == g.ny && g.ny == g.nz) {
-    // cubes: as many chunks as the narrowest compile-time z pass uses (fft_static.hip, ZWidths; at 64^3 also more
-    // rows than the 264 blocks of the register-resident pass), so the per-block partials laid out with nkb below
-    // hold every kind of z pass
+    // cubes: at least as many rows of per-block partials (nkb n) as any of the compile-time z passes has blocks
+    // (fft_static.hip, ZWidths and ZReg)
     switch (g.nx) {
       case 16: kc = 3; break;
-      case 24: kc = 5; break;
+      case 24: kc = 4; break;
       case 32: kc = 4; break;
-      case 48: kc = 5; break;
+      case 48: kc = 4; break;
       case 64: kc = 4; break;
-      case 96: kc = 7; break;
+      case 96: kc = 6; break;
       case 128: kc = 5; break;
       default: break;
     }

@@ -61,6 +61,62 @@ __device__ __forceinline__ void dft(C (&v)[R], const C* tw, int n, int step) {
       v[2 * m] = a[m];
       v[2 * m + 1] = b[m];
     }
+  } else if constexpr (R == 16) {
+    // 4 x 4: x_j, x_{j+4}, x_{j+8}, x_{j+12} for each j, twiddles W_16^(j p), then across j
+    constexpr T c1 = T(0.92387953251128675613), s1 = T(0.38268343236508977173);  // cos, sin of pi/8
+    constexpr T h = T(0.70710678118654752440);
+    C b[4][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+      for (int p = 0; p < 4; ++p) b[j][p] = v[j + 4 * p];
+      dft<4, INV>(b[j], tw, n, step);
+    }
+    // W_16^1, ^2, ^3, ^4, ^6, ^9 (conjugate for the inverse)
+    auto rot = [](C x, auto c, auto s) -> C { return cmul(x, C(c2(c, INV ? s : -s))); };  // x (c -+ i s)
+    b[1][1] = rot(b[1][1], c1, s1);
+    b[1][2] = rot(b[1][2], h, h);
+    b[1][3] = rot(b[1][3], s1, c1);
+    b[2][1] = rot(b[2][1], h, h);
+    b[2][2] = INV ? c2(-b[2][2].y, b[2][2].x) : c2(b[2][2].y, -b[2][2].x);
+    b[2][3] = rot(b[2][3], -h, h);
+    b[3][1] = rot(b[3][1], s1, c1);
+    b[3][2] = rot(b[3][2], -h, h);
+    b[3][3] = rot(b[3][3], -c1, -s1);
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      C a[4] = {b[0][p], b[1][p], b[2][p], b[3][p]};
+      dft<4, INV>(a, tw, n, step);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[p + 4 * q] = a[q];
+    }
+  } else if constexpr (R == 6 || R == 12) {
+    // R = 3 H: 3-point transforms over x_{j + H r}, twiddles W_R^(j p), then H-point transforms over j
+    constexpr int H = R / 3;
+    constexpr T cs[7] = {T(1), T(0.86602540378443864676), T(0.5), T(0), T(-0.5), T(-0.86602540378443864676), T(-1)};
+    C b[H][3];
+#pragma unroll
+    for (int j = 0; j < H; ++j) {
+#pragma unroll
+      for (int p = 0; p < 3; ++p) b[j][p] = v[j + H * p];
+      dft<3, INV>(b[j], tw, n, step);
+#pragma unroll
+      for (int p = 1; p < 3; ++p) {
+        const int k = j * p * (12 / R);   // W_12^k, k <= 6: cos(k pi / 6), sin = cos of 3 - k
+        if (k == 0) continue;
+        const T c = cs[k], sn = cs[k <= 3 ? 3 - k : k - 3];
+        b[j][p] = cmul(b[j][p], C(c2(c, INV ? sn : -sn)));
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      C a[H];
+#pragma unroll
+      for (int j = 0; j < H; ++j) a[j] = b[j][p];
+      dft<H, INV>(a, tw, n, step);
+#pragma unroll
+      for (int q = 0; q < H; ++q) v[p + 3 * q] = a[q];
+    }
   } else if constexpr (R == 3) {
     constexpr T h = T(0.86602540378443864676);  // sqrt(3)/2
     const C s = cadd(v[1], v[2]), d = csub(v[1], v[2]);
