@@ -7,7 +7,26 @@ so the device never idles while the host decides. A chunk enqueued after every
 load stopped is a no-op: inactive loads exit at once and keep their state, so
 results and iteration counts equal those of the one-chunk-at-a-time loop.
 """
+import contextlib
+import gc
+
 import torch
+
+
+@contextlib.contextmanager
+def capturing(graph):
+    """``torch.cuda.graph(graph)`` with the cyclic garbage collector held off. A solver that was dropped earlier lives
+    in a reference cycle until the collector runs; if that happens between two launches of a capture, the destructors
+    of its graphs and events call into the runtime, which an open capture refuses, and the exception they raise ends
+    the process (seen as an abort with the collector on top of the stack of a capturing thread)."""
+    enabled = gc.isenabled()
+    gc.disable()
+    try:
+        with torch.cuda.graph(graph):
+            yield
+    finally:
+        if enabled:
+            gc.enable()
 
 
 class MaskPipeline:

@@ -18,7 +18,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from ._chunks import Fork, MaskPipeline
+from ._chunks import Fork, MaskPipeline, capturing
 from .certify import CAP, MAX_RESTARTS, fail, infos as make_infos, outcome
 from .operator import LAMBDA_STUDY2, MU_STUDY2, Operator
 
@@ -230,7 +230,7 @@ class BatchedDesigns:
         for name, fn in (('init_graph', self._each('initialize')), ('iter_graph', self._concurrent('iteration')),
                          ('cert_graph', self._each('certify'))):
             graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(graph):
+            with capturing(graph):
                 fn()
             setattr(self, name, graph)
         torch.cuda.synchronize()

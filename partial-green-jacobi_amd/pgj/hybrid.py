@@ -16,6 +16,7 @@ import numpy as np
 import torch
 
 from . import _lib
+from ._chunks import capturing
 from .materials import PAIRS
 
 
@@ -337,7 +338,7 @@ class HybridResident:
         for name, fn in (('init_graph', self.initialize), ('iter_graph', self.iteration),
                          ('cert_graph', self.certify)):
             graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(graph):
+            with capturing(graph):
                 fn()
             setattr(self, name, graph)
         torch.cuda.synchronize()

@@ -15,7 +15,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from ._chunks import MaskPipeline, StreamSplit
+from ._chunks import MaskPipeline, StreamSplit, capturing
 from .certify import CAP, CertificationError
 from .operator import LAMBDA_STUDY2, MU_STUDY2, Operator
 
@@ -196,7 +196,7 @@ class MixedResident:
         self.graphs = {}
         for name in ('begin', 'iteration', 'end_and_certify'):
             graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(graph):
+            with capturing(graph):
                 getattr(self, name)()
             self.graphs[name] = graph
         torch.cuda.synchronize()

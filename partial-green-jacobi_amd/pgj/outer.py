@@ -14,6 +14,7 @@ import numpy as np
 import torch
 
 from . import _lib
+from ._chunks import capturing
 
 
 def cone_stencil(rmin):
@@ -155,7 +156,7 @@ class PaperOuter(_Fields):
         for name, fn in (('physical_graph', self.physical), ('prepare_graph', self._prepare),
                          ('bisect_graph', self._bisect_chunk)):
             g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g):
+            with capturing(g):
                 fn()
             setattr(self, name, g)
         torch.cuda.synchronize()

@@ -16,7 +16,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from ._chunks import MaskPipeline, StreamSplit
+from ._chunks import MaskPipeline, StreamSplit, capturing
 from .certify import CAP, MAX_RESTARTS, fail, infos as make_infos, outcome
 from .backend import lame
 from .operator import LAMBDA_STUDY2, MU_STUDY2, Operator
@@ -236,7 +236,7 @@ class Resident:
         for name, fn in (('init_graph', self.initialize), ('iter_graph', self.iteration),
                          ('cert_graph', self.certify)):
             g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g):
+            with capturing(g):
                 fn()
             setattr(self, name, g)
         torch.cuda.synchronize()

@@ -31,6 +31,7 @@ import numpy as np
 import torch
 
 from . import _lib
+from ._chunks import capturing
 from .batched import DesignGroup
 from .certify import CAP, MAX_RESTARTS, CertificationError, outcome
 from .density import filtered_noise
@@ -129,7 +130,7 @@ class Server:
             g.iteration()
             torch.cuda.synchronize()
             graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(graph):
+            with capturing(graph):
                 g.iteration()
             self.graphs[n] = graph
             torch.cuda.synchronize()
