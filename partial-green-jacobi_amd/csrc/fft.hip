@@ -1,14 +1,21 @@
-// Hand-written FP64 3-D R2C/C2R FFT (LDS Stockham, radices 4/2/3/5/7) with
-// the FI Green symbol fused into the z pass, and the pre/post scaling,
-// projection and PCG vector updates fused into the xy passes.
+// Hand-written FP64 3-D R2C/C2R FFT for runtime shapes (LDS Stockham, radices
+// 2..10) with the FI Green symbol fused into the z pass, and the pre/post
+// scaling, projection and PCG vector updates fused into the xy passes.
 //
 // Data path per load (spectrum layout S[l][c][kz][ky][kx], kx < nx/2+1):
-//   fxy  : per z-plane, v = s*r (PCG: r -= alpha q first);
+//   fxy  : per z-plane and component, v = s*r (PCG: r -= alpha q first);
 //          x-R2C (two reals per complex line + split), y-FFT; write S.
-//   fz   : per (ky, kx-chunk), z-FFT, v^ -= mean(r) s^ (projection P),
+//   fz   : per chunk of (ky, kx) columns, z-FFT, v^ -= mean(r) s^ (projection P),
 //          w^ = G v^, Parseval partials of v.w and s.w, inverse z-FFT.
-//   fxyi : per z-plane, inverse y-FFT, x-C2R, z = s*w - mean(s*w)
+//   fxyi : per z-plane and component, inverse y-FFT, x-C2R, z = s*w - mean(s*w)
 //          (PCG: written as the next direction z + beta p; u += alpha p).
+//
+// What bounds these passes on small and middle grids is the chain of dependent steps in a block, not bytes: with
+// block-wide stages (2 barriers each, radices 4/2/3/5/7), run-time divisions in every index (64-bit ones in the loops)
+// and twiddles from global memory the three launches at 40^3, three loads, took 48 + 33 + 47 us (now 14.6 + 15.3 + 14.1), and
+// the preconditioner of 45x60x50, three loads, 153 us (now 47). Here a wavefront
+// carries whole lines through all stages without a barrier (AxisPlan: 2 stages for nearly every length up to 100), the
+// divisions are multiplications by constants of the plan, and the twiddles are in LDS.
 #include <cmath>
 
 #include "fft_kernels.h"
@@ -16,78 +23,101 @@
 
 namespace pgj {
 
-constexpr int kMaxV = kStageValues;
+// LDS reads and writes of one wavefront, in program order for all its lanes.
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
-// Placement of the lines of a batched transform in LDS: line l starts at
-// (l / per) * outer + (l % per) * inner and its elements are es apart.
-struct LineMap {
-  int nlines, per, outer, inner, es;
-  bool line_fast;  // consecutive threads take consecutive lines (else consecutive butterflies)
-  __device__ __forceinline__ int base(int l) const { return (l / per) * outer + (l % per) * inner; }
-};
-
-// One in-place Stockham stage over the lines of `map`, each of length n.
-// All threads of the block take part; two barriers separate the read and
-// write phases, so every value of the stage is held in registers between them.
+// One in-place Stockham stage of the line at `L` (elements es apart), by the lanes j0 of its group.
 template <int R, bool INV>
-__device__ void lds_stage(double2* buf, const LineMap& map, int n, int Ns, const double2* tw, int step) {
-  const int nlines = map.nlines, es = map.es;
-  const bool line_fast = map.line_fast;
-  constexpr int NB = kMaxV / R;
+__device__ __forceinline__ void line_stage(double2* L, int es, bool on, int j0, int G, const AxisPlan::Stage& st,
+                                           const double2* tw, int step) {
+  constexpr int NB = R == 3 ? 2 : 1;  // only n / 3 can pass the 64 lanes of a group (n = 243)
   double2 v[NB][R];
-  const int nb = n / R, count = nlines * nb, m = n / (Ns * R);
+  int out[NB];
+  const int Ns = st.Ns, rd = st.nb * es;
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
-    const int b = threadIdx.x + i * blockDim.x;
-    if (b < count) {
-      const int line = line_fast ? b % nlines : b / nb;
-      const int j = line_fast ? b / nlines : b % nb;
-      const int k = j % Ns;
-      const double2* L = buf + map.base(line);
+    const int j = j0 + i * G;
+    out[i] = -1;
+    if (on && j < st.nb) {
+      const int q = int((unsigned(j) * st.mNs) >> 16), k = j - q * Ns;
+      out[i] = (q * Ns * R + k) * es;
+      const double2* p = L + j * es;
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const double2 x = L[(j + r * nb) * es];
-        v[i][r] = r == 0 ? x : cmul(x, twiddle<INV>(tw, (k * r * m) % n, step));
+      for (int r = 0; r < R; ++r) v[i][r] = p[r * rd];
+      if (Ns > 1) {
+        const int t = k * st.tws * step;
+#pragma unroll
+        for (int r = 1; r < R; ++r) v[i][r] = cmul(v[i][r], twiddle<INV>(tw, r * t, 1));
       }
     }
   }
-  __syncthreads();
+  wave_fence();
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
-    const int b = threadIdx.x + i * blockDim.x;
-    if (b < count) {
-      const int line = line_fast ? b % nlines : b / nb;
-      const int j = line_fast ? b / nlines : b % nb;
-      const int k = j % Ns;
-      dft<R, INV>(v[i], tw, n, step);
-      double2* L = buf + map.base(line);
-      const int idx = (j / Ns) * Ns * R + k;
+    if (out[i] >= 0) {
+      dft<R, INV>(v[i], tw, 0, 0);
+      double2* p = L + out[i];
 #pragma unroll
-      for (int r = 0; r < R; ++r) L[(idx + r * Ns) * es] = v[i][r];
+      for (int r = 0; r < R; ++r) p[r * Ns * es] = v[i][r];
     }
   }
-  __syncthreads();
+  wave_fence();
 }
 
+// All stages of one line per group of lanes.
 template <bool INV>
-__device__ void lds_fft(double2* buf, const LineMap& map, const Factors& f, const double2* tw, int step) {
-  int Ns = 1;
-  for (int s = 0; s < f.count; ++s) {
-    const int R = f.r[s];
-    switch (R) {
-      case 4: lds_stage<4, INV>(buf, map, f.n, Ns, tw, step); break;
-      case 2: lds_stage<2, INV>(buf, map, f.n, Ns, tw, step); break;
-      case 3: lds_stage<3, INV>(buf, map, f.n, Ns, tw, step); break;
-      case 5: lds_stage<5, INV>(buf, map, f.n, Ns, tw, step); break;
-      default: lds_stage<7, INV>(buf, map, f.n, Ns, tw, step); break;
+__device__ __forceinline__ void line_fft(double2* L, int es, bool on, int j0, const AxisPlan& a, const double2* tw,
+                                         int step) {
+#pragma unroll 1
+  for (int s = 0; s < a.count; ++s) {
+    const AxisPlan::Stage& st = a.st[s];
+    switch (st.R) {
+      case 2: line_stage<2, INV>(L, es, on, j0, a.G, st, tw, step); break;
+      case 3: line_stage<3, INV>(L, es, on, j0, a.G, st, tw, step); break;
+      case 4: line_stage<4, INV>(L, es, on, j0, a.G, st, tw, step); break;
+      case 5: line_stage<5, INV>(L, es, on, j0, a.G, st, tw, step); break;
+      case 6: line_stage<6, INV>(L, es, on, j0, a.G, st, tw, step); break;
+      case 7: line_stage<7, INV>(L, es, on, j0, a.G, st, tw, step); break;
+      case 8: line_stage<8, INV>(L, es, on, j0, a.G, st, tw, step); break;
+      case 9: line_stage<9, INV>(L, es, on, j0, a.G, st, tw, step); break;
+      default: line_stage<10, INV>(L, es, on, j0, a.G, st, tw, step); break;
     }
-    Ns *= R;
   }
 }
 
-__device__ __forceinline__ LineMap rows_map(int rows, int rs) { return LineMap{rows, rows, 0, rs, 1, false}; }
-__device__ __forceinline__ LineMap cols_map(int comps, int ny, int nkx, int rs) {
-  return LineMap{comps * nkx, nkx, ny * rs, 1, rs, true};
+// Place of a lane in its wavefront's group of lines: line `line` of the group (on: it carries one) and lane j0 of that
+// line. FAST: consecutive lanes take consecutive lines (columns in LDS), else consecutive elements (rows).
+template <bool FAST>
+struct LanePlace {
+  int line, j0;
+  bool on;
+  __device__ __forceinline__ explicit LanePlace(const AxisPlan& a) {
+    const unsigned lane = threadIdx.x & 63;
+    if (FAST) {
+      j0 = int((lane * a.mL) >> 16);
+      line = int(lane) - j0 * a.lpw;
+      on = j0 < a.G;
+    } else {
+      line = int((lane * a.mG) >> 16);
+      j0 = int(lane) - line * a.G;
+      on = line < a.lpw;
+    }
+  }
+};
+
+// Transforms of the columns 0..ncol of a plane in LDS (rows rs apart).
+template <bool INV>
+__device__ __forceinline__ void column_ffts(double2* plane, int ncol, int rs, const AxisPlan& a, const double2* tw) {
+  const LanePlace<true> at(a);
+  const int wave = threadIdx.x >> 6, step = (blockDim.x >> 6) * a.lpw;
+  for (int l0 = wave * a.lpw; l0 < ncol; l0 += step) {
+    const int line = l0 + at.line;
+    line_fft<INV>(plane + line, rs, at.on && line < ncol, at.j0, a, tw, 1);
+  }
 }
 
 __device__ __forceinline__ double reduce_pr_sum(const FFTArgs& A, int l, int c) {
@@ -95,131 +125,178 @@ __device__ __forceinline__ double reduce_pr_sum(const FFTArgs& A, int l, int c) 
   return wave_reduce_partials(A.pr + (int64_t(l) * A.nz * 3 + c) * 2 + 1, A.nz, 6);
 }
 
+// Plane z and component c of a block of the xy passes. The three components of a plane run on one XCD (block ids 8
+// apart), because in the node-interleaved layout they share every line of r, s and z.
+__device__ __forceinline__ bool plane_of_block(int nz, int& z, int& c) {
+  const int id = blockIdx.x, group = id / 24, rem = id % 24;
+  c = rem / 8;
+  z = group * 8 + rem % 8;
+  return z < nz;
+}
+
+// Copies the twiddle tables of the xy passes to LDS, x before y.
+__device__ __forceinline__ void plane_twiddles(const FFTArgs& A, double2* lds) {
+  for (int i = threadIdx.x; i < A.nx; i += blockDim.x) lds[i] = A.twx[i];
+  for (int i = threadIdx.x; i < A.ny; i += blockDim.x) lds[A.nx + i] = A.twy[i];
+}
+
+constexpr int kRedDoubles = 32;  // LDS scratch of the block sums, ahead of the plane
+constexpr int kPlaneUnroll = 4;  // values of a plane a thread loads before it uses the first
+
 // --------------------------------------------------------------- forward xy
 template <int MODE>
 __global__ __launch_bounds__(512) void fxy_kernel(FFTArgs A) {
-  extern __shared__ double2 plane[];
+  extern __shared__ double smem[];
   const FFTGeom& f = A.f;
-  const int z = blockIdx.x;
-  const int comps = f.comps;
-  const int c0 = comps == 3 ? 0 : blockIdx.y;
-  const int l = blockIdx.z;
-  const int nx = A.nx, ny = A.ny;
-  const int64_t plane_nodes = int64_t(nx) * ny;
-  double* red = reinterpret_cast<double*>(plane + size_t(comps) * ny * f.rs);
-
-  double alpha = 0.0;
-  if (MODE == kFxyPCG) {
-    if (!A.st.active[l]) return;
-    double pq, rz;
-    wave_reduce_partials_2(A.ppq + int64_t(l) * A.ppq_stride, A.ppq_count, 1, A.pg + int64_t(l) * f.nkb * ny * 4,
-                           f.nkb * ny, 4, pq, rz);
-    const bool valid = isfinite(pq) && pq > 0.0 && isfinite(rz) && rz > 0.0;
-    alpha = valid ? rz / pq : 0.0;
-    if (threadIdx.x == 0 && z == 0 && blockIdx.y == 0) {
-      A.st.rz[l] = rz;
-      A.st.alpha[l] = alpha;
-      A.st.valid[l] = valid;
-      A.st.first[l] = 0;
-    }
-  }
+  int z, c;
+  if (!plane_of_block(A.nz, z, c)) return;
+  const int l = blockIdx.z, T = blockDim.x;
+  if (MODE == kFxyPCG && !A.st.active[l]) return;
+  const int nx = A.nx, ny = A.ny, pn = nx * ny, rs = f.rs;
+  double* red = smem;
+  double2* plane = reinterpret_cast<double2*>(smem + kRedDoubles);
+  double2 *twx = plane + ny * rs, *twy = twx + nx;
+  plane_twiddles(A, twx);
 
   // 1. load (and update) the plane; pack reals two per complex along x.
-  double sq[3] = {0.0, 0.0, 0.0}, sm[3] = {0.0, 0.0, 0.0};
+  const int ns = A.soa ? 1 : 3;
+  const int dl = design_of(l, A.group);
+  const int64_t p0 = int64_t(z) * pn;
+  const int64_t off = A.soa ? (int64_t(l) * 3 + c) * A.N + p0 : (int64_t(l) * A.N + p0) * 3 + c;
+  const int64_t soff = A.soa ? (int64_t(dl) * 3 + c) * A.N + p0 : (int64_t(dl) * A.N + p0) * 3 + c;
+  const double* sp = A.s ? A.s + soff : nullptr;
+  const double* in = MODE == kFxyPCG ? A.r + off : A.rin + off;
+  const double* qp = A.q + off;
+  double* rp = A.r + off;
+  const unsigned mx = f.mnx;
   const bool even = (nx % 2) == 0;
-  const int64_t count = comps == 3 ? 3 * plane_nodes : plane_nodes;
-  for (int64_t e = threadIdx.x; e < count; e += blockDim.x) {
-    const int64_t node = comps == 3 ? e / 3 : e;
-    const int c = comps == 3 ? int(e % 3) : c0;
-    const int64_t gnode = int64_t(z) * plane_nodes + node;
-    const int64_t idx = vindex(A, l, c, gnode);
-    const int64_t sidx = vindex(A, design_of(l, A.group), c, gnode);
-    double val;
-    if (MODE == kFxyScale) {
-      val = A.s[sidx];
-    } else if (MODE == kFxyPre) {
-      const double rv = A.rin[idx];
-      sq[c] = fma(rv, rv, sq[c]);
-      sm[c] += rv;
-      val = A.s ? A.s[sidx] * rv : rv;
-    } else {
-      const double rn = fma(-alpha, A.q[idx], A.r[idx]);
-      A.r[idx] = rn;
-      sq[c] = fma(rn, rn, sq[c]);
-      sm[c] += rn;
-      val = A.s ? A.s[sidx] * rn : rn;
+  double alpha = 0.0, sums[2] = {0.0, 0.0};
+  for (int e0 = 0; e0 < pn; e0 += kPlaneUnroll * T) {
+    double vr[kPlaneUnroll], vq[kPlaneUnroll], vs[kPlaneUnroll];
+#pragma unroll
+    for (int i = 0; i < kPlaneUnroll; ++i) {
+      const int e = min(e0 + i * T + int(threadIdx.x), pn - 1) * ns;
+      if (MODE != kFxyScale) vr[i] = in[e];
+      if (MODE == kFxyPCG) vq[i] = qp[e];
+      vs[i] = sp ? sp[e] : 1.0;
     }
-    const int x = int(node % nx), y = int(node / nx);
-    double2* row = plane + (size_t(comps == 3 ? c : 0) * ny + y) * f.rs;
-    if (even) reinterpret_cast<double*>(row)[x] = val;
-    else row[x] = c2(val, 0.0);
+    if (MODE == kFxyPCG && e0 == 0) {
+      // the step length is reduced while the first loads are in flight
+      double pq, rz;
+      wave_reduce_partials_2(A.ppq + int64_t(l) * A.ppq_stride, A.ppq_count, 1, A.pg + int64_t(l) * f.nkb * ny * 4,
+                             A.zslots, 4, pq, rz);
+      const bool valid = isfinite(pq) && pq > 0.0 && isfinite(rz) && rz > 0.0;
+      alpha = valid ? rz / pq : 0.0;
+      if (threadIdx.x == 0 && blockIdx.x == 0) {
+        A.st.rz[l] = rz;
+        A.st.alpha[l] = alpha;
+        A.st.valid[l] = valid;
+        A.st.first[l] = 0;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kPlaneUnroll; ++i) {
+      const int e = e0 + i * T + int(threadIdx.x);
+      if (e < pn) {
+        double val = vs[i];
+        if (MODE != kFxyScale) {
+          double rn = vr[i];
+          if (MODE == kFxyPCG) {
+            rn = fma(-alpha, vq[i], rn);
+            rp[e * ns] = rn;
+          }
+          sums[0] = fma(rn, rn, sums[0]);
+          sums[1] += rn;
+          val = sp ? val * rn : rn;
+        }
+        const int y = int(__umulhi(unsigned(e), mx)), x = e - y * nx;
+        double2* row = plane + y * rs;
+        if (even) reinterpret_cast<double*>(row)[x] = val;
+        else row[x] = c2(val, 0.0);
+      }
+    }
   }
   if (MODE != kFxyScale) {
-    for (int c = 0; c < 3; ++c) {
-      if (comps == 1 && c != c0) continue;
-      const double tq = block_sum(sq[c], red), tm = block_sum(sm[c], red);
-      if (threadIdx.x == 0) {
-        double* p = A.pr + ((int64_t(l) * A.nz + z) * 3 + c) * 2;
-        p[0] = tq;
-        p[1] = tm;
+    block_sums<2>(sums, red);
+    if (threadIdx.x == 0) {
+      double* p = A.pr + ((int64_t(l) * A.nz + z) * 3 + c) * 2;
+      p[0] = sums[0];
+      p[1] = sums[1];
+    }
+  }
+  __syncthreads();
+  // 2. x transform of every row (complex length M) and the split of the packed spectrum into the half spectrum of the
+  // real row, by the row's own lanes
+  {
+    const AxisPlan& a = f.px;
+    const LanePlace<false> at(a);
+    const int M = f.M, half = M / 2, step = (T >> 6) * a.lpw, wstep = even ? 2 : 1;
+    for (int l0 = (threadIdx.x >> 6) * a.lpw; l0 < ny; l0 += step) {
+      const int row = l0 + at.line;
+      const bool on = at.on && row < ny;
+      double2* L = plane + row * rs;
+      line_fft<false>(L, 1, on, at.j0, a, twx, wstep);
+      if (even && on) {
+        for (int k = at.j0; k <= half; k += a.G) {
+          const double2 zk = L[k], zm = L[k == 0 ? 0 : M - k];
+          const double2 E = c2(0.5 * (zk.x + zm.x), 0.5 * (zk.y - zm.y));
+          const double2 O = c2(0.5 * (zk.y + zm.y), -0.5 * (zk.x - zm.x));
+          const double2 wo = cmul(twx[k], O);
+          L[k] = cadd(E, wo);
+          if (M - k != k) L[M - k] = conjd(csub(E, wo));
+        }
       }
     }
   }
   __syncthreads();
-  // 2. x transform on every row (complex length M).
-  const int rows = comps * ny;
-  lds_fft<false>(plane, rows_map(rows, f.rs), f.fx, A.twx, nx / f.M);
-  // 3. split the packed spectrum into the half spectrum of each real row.
-  if (even) {
-    const int M = f.M, half = M / 2;
-    const int pairs = rows * (half + 1);
-    for (int b = threadIdx.x; b < pairs; b += blockDim.x) {
-      const int row = b / (half + 1), k = b % (half + 1);
-      double2* L = plane + size_t(row) * f.rs;
-      const double2 zk = L[k % M], zm = L[(M - k) % M];
-      const double2 E = c2(0.5 * (zk.x + zm.x), 0.5 * (zk.y - zm.y));
-      const double2 O = c2(0.5 * (zk.y + zm.y), -0.5 * (zk.x - zm.x));
-      const double2 w = A.twx[k];
-      const double2 wo = cmul(w, O);
-      L[k] = cadd(E, wo);
-      if (M - k != k) L[M - k] = conjd(csub(E, wo));
-    }
-    __syncthreads();
-  }
-  // 4. y transform on every kx column.
-  lds_fft<false>(plane, cols_map(comps, ny, f.nkx, f.rs), f.fy, A.twy, 1);
-  // 5. write the half spectrum.
-  double2* out = A.spec + ((int64_t(l) * 3 + c0) * A.nz + z) * int64_t(ny) * f.nkx;
-  const int64_t total = int64_t(comps) * ny * f.nkx;
-  for (int64_t e = threadIdx.x; e < total; e += blockDim.x) {
-    const int c = int(e / (int64_t(ny) * f.nkx));
-    const int rem = int(e % (int64_t(ny) * f.nkx));
-    const int y = rem / f.nkx, kx = rem % f.nkx;
-    out[int64_t(c) * A.nz * ny * f.nkx + rem] = plane[(size_t(c) * ny + y) * f.rs + kx];
-  }
+  // 3. y transform of every kx column.
+  column_ffts<false>(plane, f.nkx, rs, f.py, twy);
+  __syncthreads();
+  // 4. write the half spectrum.
+  double2* out = A.spec + ((int64_t(l) * 3 + c) * A.nz + z) * (ny * f.nkx);
+  const unsigned mk = f.mnkx;
+  const int total = ny * f.nkx, pad = rs - f.nkx;
+  for (int e = threadIdx.x; e < total; e += T) out[e] = plane[e + (pad ? int(__umulhi(unsigned(e), mk)) * pad : 0)];
 }
 
 // ---------------------------------------------------------------- z + Green
-template <int MODE>
-__global__ __launch_bounds__(256) void fz_kernel(FFTArgs A) {
-  extern __shared__ double2 cols[];
+// A block transforms C consecutive columns (ky, kx) of the three components, all in LDS [c][z][column]. C = 16 fills
+// two lines of every row it reads; 8 and 4 spread small grids over the CUs (runtime_chunk).
+template <int MODE, int C>
+__global__ __launch_bounds__(512) void fz_kernel(FFTArgs A) {
+  extern __shared__ double smem[];
   const FFTGeom& f = A.f;
-  const int kb = blockIdx.x, y = blockIdx.y, l = blockIdx.z;
-  const int nz = A.nz, ny = A.ny, nkx = f.nkx, kc = f.kc;
-  const int kx0 = kb * kc;
-  const int kcn = min(kc, nkx - kx0);
-  const int blk = y * f.nkb + kb;
-  const bool lead = threadIdx.x == 0 && kb == 0 && y == 0;
-  double* red = reinterpret_cast<double*>(cols + size_t(kc) * 3 * nz);
-  double* pg = A.pg + (int64_t(l) * f.nkb * ny + blk) * 4;
-
+  const int l = blockIdx.z, T = blockDim.x;
+  const int nz = A.nz, nzc = nz * C, pl = A.ny * f.nkx;
+  const int f0 = blockIdx.x * C, ncol = min(C, pl - f0);
+  const bool lead = threadIdx.x == 0 && blockIdx.x == 0;
+  double* red = smem;
+  double2* cols = reinterpret_cast<double2*>(smem + kRedDoubles);
+  double2* tw = cols + 3 * nzc;
+  double2* S = A.spec + int64_t(l) * 3 * f.nf + f0;
+  if (MODE == kFzPCG && !A.st.active[l]) {
+    // an inactive load stays inactive: the test below with active = false
+    if (lead) {
+      A.st.active_next[l] = 0;
+      A.st.it_next[l] = A.st.it[l];
+      A.st.bad_next[l] = A.st.bad[l];
+      A.st.stopped[l] = 0;
+    }
+    return;
+  }
+  // the columns and twiddles go to LDS first; the test below runs while they are in flight
+  for (int e = threadIdx.x; e < 3 * nzc; e += T) {
+    const int col = e % C, row = e / C;
+    cols[e] = col < ncol ? S[int64_t(row) * pl + col] : c2(0.0, 0.0);
+  }
+  for (int i = threadIdx.x; i < nz; i += T) tw[i] = A.twz[i];
   double mean[3] = {0.0, 0.0, 0.0};
   if (MODE == kFzInit || MODE == kFzPCG) {
     // one pass over the per-plane partials (|r|^2 and the component sums of r)
     const int lane = threadIdx.x & 63;
     double v = 0.0, vm[3] = {0.0, 0.0, 0.0};
-    for (int i = lane; i < A.nz; i += 64) {
-      const double* p = A.pr + (int64_t(l) * A.nz + i) * 6;
+    for (int i = lane; i < nz; i += 64) {
+      const double* p = A.pr + (int64_t(l) * nz + i) * 6;
       v += (p[0] + p[2]) + p[4];
       vm[0] += p[1];
       vm[1] += p[3];
@@ -239,203 +316,205 @@ __global__ __launch_bounds__(256) void fz_kernel(FFTArgs A) {
         A.st.stopped[l] = 0;
       }
     } else {
-      const bool active = A.st.active[l] != 0;
       const bool valid = A.st.valid[l] != 0;  // set by the forward pass of this iteration
       const bool finite = isfinite(res2);
-      const int64_t it = A.st.it[l] + (active ? 1 : 0);
-      act = active && valid && finite && res2 > A.st.target2[l] && it < A.st.cap[l];
+      const int64_t it = A.st.it[l] + 1;
+      act = valid && finite && res2 > A.st.target2[l] && it < A.st.cap[l];
       if (lead) {
         A.st.active_next[l] = act;
         A.st.it_next[l] = it;
-        A.st.bad_next[l] = A.st.bad[l] || (active && !valid) || (active && !finite);
-        A.st.stopped[l] = active && !act;
+        A.st.bad_next[l] = A.st.bad[l] || !valid || !finite;
+        A.st.stopped[l] = !act;
       }
     }
     if (!act) return;
   } else if (MODE != kFzScale && A.shat) {
     for (int c = 0; c < 3; ++c) mean[c] = reduce_pr_sum(A, l, c) / double(A.N);
   }
-  // load the columns (c, z, kcol) of this (ky, kx-chunk)
-  double2* S = A.spec + int64_t(l) * 3 * f.nf;
-  const int total = 3 * nz * kcn;
-  for (int e = threadIdx.x; e < total; e += blockDim.x) {
-    const int kcol = e % kcn, cz = e / kcn;
-    const int c = cz / nz, zz = cz % nz;
-    cols[(size_t(c) * nz + zz) * kc + kcol] = S[((int64_t(c) * nz + zz) * ny + y) * nkx + kx0 + kcol];
+  __syncthreads();
+  const AxisPlan& a = f.pz;
+  const LanePlace<true> at(a);
+  const int wave0 = (threadIdx.x >> 6) * a.lpw, step = (T >> 6) * a.lpw;
+  for (int l0 = wave0; l0 < 3 * C; l0 += step) {
+    const int line = l0 + at.line;
+    line_fft<false>(cols + line / C * nzc + line % C, C, at.on && line < 3 * C, at.j0, a, tw, 1);
   }
   __syncthreads();
-  const LineMap zmap{3 * kcn, kcn, nz * kc, 1, kc, true};
-  lds_fft<false>(cols, zmap, f.fz, A.twz, 1);
-  if (MODE == kFzScale) {
-    for (int e = threadIdx.x; e < total; e += blockDim.x) {
-      const int kcol = e % kcn, cz = e / kcn;
-      const int c = cz / nz, zz = cz % nz;
-      S[((int64_t(c) * nz + zz) * ny + y) * nkx + kx0 + kcol] = cols[(size_t(c) * nz + zz) * kc + kcol];
-    }
-    return;
-  }
-  // per frequency: projection correction, Green multiply, Parseval partials
-  double rz = 0.0, sw[3] = {0.0, 0.0, 0.0};
-  for (int e = threadIdx.x; e < nz * kcn; e += blockDim.x) {
-    const int kcol = e % kcn, zz = e / kcn;
-    const int kx = kx0 + kcol;
-    const int64_t fidx = (int64_t(zz) * ny + y) * nkx + kx;
-    double2 v[3];
-    for (int c = 0; c < 3; ++c) v[c] = cols[(size_t(c) * nz + zz) * kc + kcol];
-    double2 sh[3];
-    if (A.shat) {
-      for (int c = 0; c < 3; ++c) {
-        sh[c] = A.shat[(int64_t(design_of(l, A.group)) * 3 + c) * f.nf + fidx];
-        v[c] = c2(fma(-mean[c], sh[c].x, v[c].x), fma(-mean[c], sh[c].y, v[c].y));
+  if (MODE != kFzScale) {
+    // per frequency: projection correction, Green multiply, Parseval partials
+    double sums[4] = {0.0, 0.0, 0.0, 0.0};  // r.z, s.w of the three components
+    const unsigned mk = f.mnkx;
+    for (int e = threadIdx.x; e < nzc; e += T) {
+      const int col = e % C, zz = e / C;
+      if (col >= ncol) continue;
+      const int fk = f0 + col, kx = fk - int(__umulhi(unsigned(fk), mk)) * f.nkx;
+      const int64_t fidx = int64_t(zz) * pl + fk;
+      double g[6];
+#pragma unroll
+      for (int i = 0; i < 6; ++i) g[i] = A.sym[i * f.nf + fidx];
+      double2 v[3], sh[3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) v[c] = cols[c * nzc + e];
+      if (A.shat) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) sh[c] = A.shat[(int64_t(design_of(l, A.group)) * 3 + c) * f.nf + fidx];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) v[c] = c2(fma(-mean[c], sh[c].x, v[c].x), fma(-mean[c], sh[c].y, v[c].y));
       }
+      double2 w[3];
+      w[0] = c2(g[0] * v[0].x + g[3] * v[1].x + g[4] * v[2].x, g[0] * v[0].y + g[3] * v[1].y + g[4] * v[2].y);
+      w[1] = c2(g[3] * v[0].x + g[1] * v[1].x + g[5] * v[2].x, g[3] * v[0].y + g[1] * v[1].y + g[5] * v[2].y);
+      w[2] = c2(g[4] * v[0].x + g[5] * v[1].x + g[2] * v[2].x, g[4] * v[0].y + g[5] * v[1].y + g[2] * v[2].y);
+      const double wgt = (kx == 0 || (A.nx % 2 == 0 && kx == A.nx / 2)) ? 1.0 : 2.0;
+      double t = 0.0;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) t += v[c].x * w[c].x + v[c].y * w[c].y;
+      sums[0] = fma(wgt, t, sums[0]);
+      if (A.shat)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) sums[1 + c] = fma(wgt, sh[c].x * w[c].x + sh[c].y * w[c].y, sums[1 + c]);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) cols[c * nzc + e] = w[c];
     }
-    const double g0 = A.sym[fidx], g1 = A.sym[f.nf + fidx], g2 = A.sym[2 * f.nf + fidx];
-    const double g3 = A.sym[3 * f.nf + fidx], g4 = A.sym[4 * f.nf + fidx], g5 = A.sym[5 * f.nf + fidx];
-    double2 w[3];
-    w[0] = c2(g0 * v[0].x + g3 * v[1].x + g4 * v[2].x, g0 * v[0].y + g3 * v[1].y + g4 * v[2].y);
-    w[1] = c2(g3 * v[0].x + g1 * v[1].x + g5 * v[2].x, g3 * v[0].y + g1 * v[1].y + g5 * v[2].y);
-    w[2] = c2(g4 * v[0].x + g5 * v[1].x + g2 * v[2].x, g4 * v[0].y + g5 * v[1].y + g2 * v[2].y);
-    const double wgt = (kx == 0 || (A.nx % 2 == 0 && kx == A.nx / 2)) ? 1.0 : 2.0;
-    double t = 0.0;
-    for (int c = 0; c < 3; ++c) t += v[c].x * w[c].x + v[c].y * w[c].y;
-    rz = fma(wgt, t, rz);
-    if (A.shat)
-      for (int c = 0; c < 3; ++c) sw[c] = fma(wgt, sh[c].x * w[c].x + sh[c].y * w[c].y, sw[c]);
-    for (int c = 0; c < 3; ++c) cols[(size_t(c) * nz + zz) * kc + kcol] = w[c];
+    block_sums<4>(sums, red);
+    if (threadIdx.x == 0) {
+      double* pg = A.pg + (int64_t(l) * f.nkb * A.ny + blockIdx.x) * 4;
+      for (int i = 0; i < 4; ++i) pg[i] = sums[i];
+    }
+    __syncthreads();
+    for (int l0 = wave0; l0 < 3 * C; l0 += step) {
+      const int line = l0 + at.line;
+      line_fft<true>(cols + line / C * nzc + line % C, C, at.on && line < 3 * C, at.j0, a, tw, 1);
+    }
+    __syncthreads();
   }
-  __syncthreads();
-  lds_fft<true>(cols, zmap, f.fz, A.twz, 1);
-  for (int e = threadIdx.x; e < total; e += blockDim.x) {
-    const int kcol = e % kcn, cz = e / kcn;
-    const int c = cz / nz, zz = cz % nz;
-    S[((int64_t(c) * nz + zz) * ny + y) * nkx + kx0 + kcol] = cols[(size_t(c) * nz + zz) * kc + kcol];
-  }
-  const double trz = block_sum(rz, red);
-  double tsw[3];
-  for (int c = 0; c < 3; ++c) tsw[c] = block_sum(sw[c], red);
-  if (threadIdx.x == 0) {
-    pg[0] = trz;
-    pg[1] = tsw[0];
-    pg[2] = tsw[1];
-    pg[3] = tsw[2];
+  for (int e = threadIdx.x; e < 3 * nzc; e += T) {
+    const int col = e % C, row = e / C;
+    if (col < ncol) S[int64_t(row) * pl + col] = cols[e];
   }
 }
 
 // --------------------------------------------------------------- inverse xy
 template <int MODE>
 __global__ __launch_bounds__(512) void fxyi_kernel(FFTArgs A) {
-  extern __shared__ double2 plane[];
+  extern __shared__ double smem[];
   const FFTGeom& f = A.f;
-  const int z = blockIdx.x;
-  const int comps = f.comps;
-  const int c0 = comps == 3 ? 0 : blockIdx.y;
-  const int l = blockIdx.z;
-  const int nx = A.nx, ny = A.ny;
-  const int64_t plane_nodes = int64_t(nx) * ny;
-  const int64_t count = comps == 3 ? 3 * plane_nodes : plane_nodes;
+  int z, c;
+  if (!plane_of_block(A.nz, z, c)) return;
+  const int l = blockIdx.z, T = blockDim.x;
+  const int nx = A.nx, ny = A.ny, pn = nx * ny, rs = f.rs, ns = A.soa ? 1 : 3;
+  const int dl = design_of(l, A.group);
+  const int64_t p0 = int64_t(z) * pn;
+  const int64_t off = A.soa ? (int64_t(l) * 3 + c) * A.N + p0 : (int64_t(l) * A.N + p0) * 3 + c;
+  const int64_t soff = A.soa ? (int64_t(dl) * 3 + c) * A.N + p0 : (int64_t(dl) * A.N + p0) * 3 + c;
   // PCG: the displacement update u += alpha p of this iteration (alpha from the forward pass)
   const bool move = MODE == kFxyiPCG && A.p != nullptr && A.u != nullptr;
   const double alpha = move ? A.st.alpha[l] : 0.0;
+  const double* pp = A.p ? A.p + off : nullptr;
+  double* up = A.u ? A.u + off : nullptr;
   if (MODE == kFxyiPCG) {
-    if (threadIdx.x == 0 && z == 0 && blockIdx.y == 0) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) {
       A.st.active[l] = A.st.active_next[l];
       A.st.it[l] = A.st.it_next[l];
       A.st.bad[l] = A.st.bad_next[l];
     }
     if (!A.st.active_next[l]) {
       // a load stopped by this iteration's test still takes its last displacement update
-      if (move && A.st.stopped[l]) {
-        for (int64_t e = threadIdx.x; e < count; e += blockDim.x) {
-          const int64_t node = comps == 3 ? e / 3 : e;
-          const int c = comps == 3 ? int(e % 3) : c0;
-          const int64_t oi = vindex(A, l, c, int64_t(z) * plane_nodes + node);
-          A.u[oi] = fma(alpha, A.p[oi], A.u[oi]);
-        }
-      }
+      if (move && A.st.stopped[l])
+        for (int e = threadIdx.x; e < pn; e += T) up[e * ns] = fma(alpha, pp[e * ns], up[e * ns]);
       return;
     }
   }
+  double2* plane = reinterpret_cast<double2*>(smem + kRedDoubles);
+  double2 *twx = plane + ny * rs, *twy = twx + nx;
+  // 1. load the half spectrum of the plane
+  const double2* in = A.spec + ((int64_t(l) * 3 + c) * A.nz + z) * (ny * f.nkx);
+  const unsigned mk = f.mnkx;
+  const int total = ny * f.nkx, pad = rs - f.nkx;
+  for (int e = threadIdx.x; e < total; e += T) plane[e + (pad ? int(__umulhi(unsigned(e), mk)) * pad : 0)] = in[e];
+  plane_twiddles(A, twx);
   // PCG: the output is the next direction p = z + beta p (z alone right after init)
-  double mean[3] = {0.0, 0.0, 0.0};
-  double beta = 0.0;
+  double mean = 0.0, beta = 0.0;
   const bool update = MODE == kFxyiPCG && A.p != nullptr && !A.st.first[l];
   if (A.shat || update) {
-    // one pass: r.z (offset 0) and the s.w partials of the three components (offsets 1..3)
-    const int cnt = f.nkb * ny;
-    const int off[4] = {0, 1, 2, 3};
-    double sums[4];
-    wave_reduce_partials_n<4>(A.pg + int64_t(l) * cnt * 4, off, cnt, 4, sums);
-    if (A.shat)
-      for (int c = 0; c < 3; ++c) mean[c] = sums[1 + c] / double(A.N);
+    // one pass: r.z (offset 0) and this component's s.w partials (offset 1 + c)
+    const int at[2] = {0, 1 + c};
+    double sums[2];
+    wave_reduce_partials_n<2>(A.pg + int64_t(l) * f.nkb * ny * 4, at, A.zslots, 4, sums);
+    if (A.shat) mean = sums[1] / double(A.N);
     if (update) {
       const double rz = A.st.rz[l];
       beta = sums[0] / (rz != 0.0 ? rz : 1.0);
     }
   }
-  // 1. load the half spectrum of the plane
-  const double2* in = A.spec + ((int64_t(l) * 3 + c0) * A.nz + z) * int64_t(ny) * f.nkx;
-  const int64_t total = int64_t(comps) * ny * f.nkx;
-  for (int64_t e = threadIdx.x; e < total; e += blockDim.x) {
-    const int c = int(e / (int64_t(ny) * f.nkx));
-    const int rem = int(e % (int64_t(ny) * f.nkx));
-    const int y = rem / f.nkx, kx = rem % f.nkx;
-    plane[(size_t(c) * ny + y) * f.rs + kx] = in[int64_t(c) * A.nz * ny * f.nkx + rem];
-  }
   __syncthreads();
   // 2. inverse y transform
-  lds_fft<true>(plane, cols_map(comps, ny, f.nkx, f.rs), f.fy, A.twy, 1);
-  const int rows = comps * ny;
+  column_ffts<true>(plane, f.nkx, rs, f.py, twy);
+  __syncthreads();
+  // 3. rebuild the complex line of each real row and transform it, by the row's own lanes
   const bool even = (nx % 2) == 0;
-  // 3. rebuild the complex line of each real row
-  if (even) {
-    const int M = f.M, half = M / 2;
-    const int pairs = rows * (half + 1);
-    for (int b = threadIdx.x; b < pairs; b += blockDim.x) {
-      const int row = b / (half + 1), k = b % (half + 1);
-      double2* L = plane + size_t(row) * f.rs;
-      double2 xk = L[k], xm = L[M - k];
-      if (k == 0) {
-        xk.y = 0.0;
-        xm.y = 0.0;
+  {
+    const AxisPlan& a = f.px;
+    const LanePlace<false> at(a);
+    const int M = f.M, half = M / 2, step = (T >> 6) * a.lpw;
+    for (int l0 = (threadIdx.x >> 6) * a.lpw; l0 < ny; l0 += step) {
+      const int row = l0 + at.line;
+      const bool on = at.on && row < ny;
+      double2* L = plane + row * rs;
+      if (even && on) {
+        for (int k = at.j0; k <= half; k += a.G) {
+          double2 xk = L[k], xm = L[M - k];
+          if (k == 0) {
+            xk.y = 0.0;
+            xm.y = 0.0;
+          }
+          // Z[k] = (X[k] + conj(X[M-k])) + i (X[k] - conj(X[M-k])) conj(W^k)
+          const double2 wk = conjd(twx[k]);
+          const double2 e1 = c2(xk.x + xm.x, xk.y - xm.y);
+          const double2 o1 = cmul(c2(xk.x - xm.x, xk.y + xm.y), wk);
+          if (k != 0 && M - k != k) {
+            const double2 wm = conjd(twx[M - k]);
+            const double2 e2 = c2(xm.x + xk.x, xm.y - xk.y);
+            const double2 o2 = cmul(c2(xm.x - xk.x, xm.y + xk.y), wm);
+            L[M - k] = c2(e2.x - o2.y, e2.y + o2.x);
+          }
+          L[k] = c2(e1.x - o1.y, e1.y + o1.x);
+        }
+      } else if (on) {
+        // odd nx: Hermitian completion of the row
+        for (int k = f.nkx + at.j0; k < nx; k += a.G) L[k] = conjd(L[nx - k]);
+        if (at.j0 == 0) L[0].y = 0.0;
       }
-      // Z[k] = (X[k] + conj(X[M-k])) + i (X[k] - conj(X[M-k])) conj(W^k)
-      const double2 wk = conjd(A.twx[k]);
-      const double2 e1 = c2(xk.x + xm.x, xk.y - xm.y);
-      const double2 o1 = cmul(c2(xk.x - xm.x, xk.y + xm.y), wk);
-      const double2 zk = c2(e1.x - o1.y, e1.y + o1.x);
-      if (k != 0 && M - k != k) {
-        const double2 wm = conjd(A.twx[M - k]);
-        const double2 e2 = c2(xm.x + xk.x, xm.y - xk.y);
-        const double2 o2 = cmul(c2(xm.x - xk.x, xm.y + xk.y), wm);
-        L[M - k] = c2(e2.x - o2.y, e2.y + o2.x);
-      }
-      L[k] = zk;
+      wave_fence();
+      line_fft<true>(L, 1, on, at.j0, a, twx, even ? 2 : 1);
     }
-  } else {
-    // odd nx: Hermitian completion of every row
-    const int fill = nx - f.nkx;
-    for (int b = threadIdx.x; b < rows * fill; b += blockDim.x) {
-      const int row = b / fill, k = f.nkx + b % fill;
-      double2* L = plane + size_t(row) * f.rs;
-      L[k] = conjd(L[nx - k]);
-    }
-    for (int b = threadIdx.x; b < rows; b += blockDim.x) plane[size_t(b) * f.rs].y = 0.0;
   }
   __syncthreads();
-  // 4. inverse x transform
-  lds_fft<true>(plane, rows_map(rows, f.rs), f.fx, A.twx, nx / f.M);
-  // 5. unpack, scale and project; PCG: next direction and displacement update
-  for (int64_t e = threadIdx.x; e < count; e += blockDim.x) {
-    const int64_t node = comps == 3 ? e / 3 : e;
-    const int c = comps == 3 ? int(e % 3) : c0;
-    const int x = int(node % nx), y = int(node / nx);
-    const double2* row = plane + (size_t(comps == 3 ? c : 0) * ny + y) * f.rs;
-    const double w = even ? reinterpret_cast<const double*>(row)[x] : row[x].x;
-    const int64_t gnode = int64_t(z) * plane_nodes + node;
-    const double v = A.s ? A.s[vindex(A, design_of(l, A.group), c, gnode)] * w - mean[c] : w;
-    const int64_t oi = vindex(A, l, c, gnode);
-    A.zout[oi] = update ? fma(beta, A.p[oi], v) : v;
-    if (move) A.u[oi] = fma(alpha, A.p[oi], A.u[oi]);
+  // 4. unpack, scale and project; PCG: next direction and displacement update
+  const double* sp = A.s ? A.s + soff : nullptr;
+  double* zp = A.zout + off;
+  const unsigned mx = f.mnx;
+  for (int e0 = threadIdx.x; e0 < pn; e0 += kPlaneUnroll * T) {
+    double vs[kPlaneUnroll], vp[kPlaneUnroll], vu[kPlaneUnroll];
+#pragma unroll
+    for (int i = 0; i < kPlaneUnroll; ++i) {
+      const int e = min(e0 + i * T, pn - 1) * ns;
+      vs[i] = sp ? sp[e] : 1.0;
+      vp[i] = update || move ? pp[e] : 0.0;
+      vu[i] = move ? up[e] : 0.0;
+    }
+#pragma unroll
+    for (int i = 0; i < kPlaneUnroll; ++i) {
+      const int e = e0 + i * T;
+      if (e < pn) {
+        const int y = int(__umulhi(unsigned(e), mx)), x = e - y * nx;
+        const double2* row = plane + y * rs;
+        const double w = even ? reinterpret_cast<const double*>(row)[x] : row[x].x;
+        const double v = sp ? vs[i] * w - mean : w;
+        zp[e * ns] = update ? fma(beta, vp[i], v) : v;
+        if (move) up[e * ns] = fma(alpha, vp[i], vu[i]);
+      }
+    }
   }
 }
 
@@ -566,49 +645,81 @@ int allow_lds(K kernel, size_t bytes) {
   PGJ_REQUIRE((A).f.runtime_ok, "grid (%d,%d,%d) has only the compile-time resident FFT path", (A).nz, (A).ny, \
               (A).nx)
 
-// With fewer plane blocks than CUs (few loads), the xy kernels take one
-// component per block, which triples the grid; the spectrum layout is the same.
-FFTArgs xy_args(const FFTArgs& A, int L) {
-  FFTArgs B = A;
-  if (A.f.comps == 3 && int64_t(A.nz) * L < 256) {
-    B.f.comps = 1;
-    B.f.lds_xy = (A.f.lds_xy - 64 * 8) / 3 + 64 * 8;
-  }
-  return B;
+// Threads of a block whose transforms carry `lines` lines of plan `a`: one round of wavefronts, 256 to 512 threads.
+inline int line_threads(const AxisPlan& a, int lines) {
+  const int waves = (lines + a.lpw - 1) / a.lpw;
+  return 64 * std::min(8, std::max(4, waves));
+}
+
+struct PlaneLaunch {
+  dim3 grid;
+  int threads;
+  size_t lds;  // below 148 KB: the supported planes hold at most 8192 + ny values (fft_geom)
+};
+
+inline PlaneLaunch plane_launch(const FFTArgs& A, int L) {
+  PlaneLaunch p;
+  p.grid = dim3(unsigned((A.nz + 7) / 8 * 24), 1, unsigned(L));
+  p.threads = std::max(line_threads(A.f.px, A.ny), line_threads(A.f.py, A.f.nkx));
+  p.lds = kRedDoubles * 8 + (size_t(A.ny) * A.f.rs + A.nx + A.ny) * 16;
+  return p;
 }
 
 template <int MODE>
-int launch_fxy(FFTArgs& A0, int L, hipStream_t s) {
-  PGJ_RUNTIME_FFT(A0);
-  FFTArgs A = xy_args(A0, L);
-  const FFTGeom& f = A.f;
-  dim3 grid(A.nz, f.comps == 3 ? 1 : 3, L);
-  if (int e = allow_lds(fxy_kernel<MODE>, f.lds_xy)) return e;
-  hipLaunchKernelGGL(fxy_kernel<MODE>, grid, dim3(f.threads_xy), f.lds_xy, s, A);
+int launch_fxy(FFTArgs& A, int L, hipStream_t s) {
+  PGJ_RUNTIME_FFT(A);
+  const PlaneLaunch p = plane_launch(A, L);
+  if (int e = allow_lds(fxy_kernel<MODE>, p.lds)) return e;
+  hipLaunchKernelGGL(fxy_kernel<MODE>, p.grid, dim3(p.threads), p.lds, s, A);
   PGJ_LAUNCHED("fxy_kernel");
+  return PGJ_OK;
+}
+
+template <int MODE, int C>
+int launch_fz_c(FFTArgs& A, int L, hipStream_t s) {
+  const int blocks = (A.ny * A.f.nkx + C - 1) / C;
+  PGJ_REQUIRE(A.zslots == blocks && blocks <= A.f.nkb * A.ny, "z pass blocks (%d) do not match the partial layout (%d)",
+              blocks, A.zslots);
+  const size_t lds = kRedDoubles * 8 + size_t(A.nz) * (3 * C + 1) * 16;
+  // a thread per element of the Green multiply, or what the transforms need
+  const int threads = std::max(line_threads(A.f.pz, 3 * C), std::min(512, (A.nz * C + 63) / 64 * 64));
+  if (int e = allow_lds(fz_kernel<MODE, C>, lds)) return e;
+  hipLaunchKernelGGL((fz_kernel<MODE, C>), dim3(blocks, 1, L), dim3(threads), lds, s, A);
+  PGJ_LAUNCHED("fz_kernel");
   return PGJ_OK;
 }
 
 template <int MODE>
 int launch_fz(FFTArgs& A, int L, hipStream_t s) {
   PGJ_RUNTIME_FFT(A);
-  const FFTGeom& f = A.f;
-  dim3 grid(f.nkb, A.ny, L);
-  hipLaunchKernelGGL(fz_kernel<MODE>, grid, dim3(f.threads_z), f.lds_z, s, A);
-  PGJ_LAUNCHED("fz_kernel");
-  return PGJ_OK;
+  switch (A.zkc) {
+    case 16: return launch_fz_c<MODE, 16>(A, L, s);
+    case 8: return launch_fz_c<MODE, 8>(A, L, s);
+    default: return launch_fz_c<MODE, 4>(A, L, s);
+  }
 }
 
 template <int MODE>
-int launch_fxyi(FFTArgs& A0, int L, hipStream_t s) {
-  PGJ_RUNTIME_FFT(A0);
-  FFTArgs A = xy_args(A0, L);
-  const FFTGeom& f = A.f;
-  dim3 grid(A.nz, f.comps == 3 ? 1 : 3, L);
-  if (int e = allow_lds(fxyi_kernel<MODE>, f.lds_xy)) return e;
-  hipLaunchKernelGGL(fxyi_kernel<MODE>, grid, dim3(f.threads_xy), f.lds_xy, s, A);
+int launch_fxyi(FFTArgs& A, int L, hipStream_t s) {
+  PGJ_RUNTIME_FFT(A);
+  const PlaneLaunch p = plane_launch(A, L);
+  if (int e = allow_lds(fxyi_kernel<MODE>, p.lds)) return e;
+  hipLaunchKernelGGL(fxyi_kernel<MODE>, p.grid, dim3(p.threads), p.lds, s, A);
   PGJ_LAUNCHED("fxyi_kernel");
   return PGJ_OK;
+}
+
+// 16 columns (two lines of every row) where that still gives a block per CU and the columns stay within 64 KB, 8 down to
+// 100 blocks, else 4. Preconditioner with 4 / 8 / 16 columns (us): 20^3 one load 20.3 / 20.9 / 21.9, 40^3 three loads
+// 35.5 / 33.1 / 33.5, 45x60x50 one 36.4 / 33.2 / 34.2, three 48.3 / 51.3 / 46.7, 60x50x54 six 97.9 / 94.5 / 89.7,
+// 98x35x80 three (73 KB at 16) 107 / 109 / 126.
+int runtime_chunk(const FFTGeom& f, int L) {
+  const int pl = f.ny * f.nkx;
+  int c = 16;
+  while (c > kMinChunk &&
+         (int64_t(pl + c - 1) / c * L < (c == 16 ? 256 : 100) || size_t(f.nz) * 3 * c * 16 > 64 * 1024))
+    c /= 2;
+  return c;
 }
 
 int launch_fxy_mode(FFTArgs& A, int L, int mode, hipStream_t s) {
@@ -708,6 +819,7 @@ extern "C" int pgj_scale_spectrum(const pgj_grid* g, const void* plan, const dou
   A.spec = static_cast<double2*>(s_hat);
   A.pr = reinterpret_cast<double*>(static_cast<char*>(ws) + pl.pr);
   A.pg = reinterpret_cast<double*>(static_cast<char*>(ws) + pl.pg);
+  zpass_choose(A, *g, 1);
   hipStream_t st = as_stream(stream);
   if (int e = launch_fxy<kFxyScale>(A, 1, st)) return e;
   return launch_fz<kFzScale>(A, 1, st);
@@ -738,12 +850,6 @@ extern "C" int pgj_precond_apply(const pgj_grid* g, int L, const void* plan, con
     if (int e = launch_fz_static(A, L, kFzPre, st)) return e;
     return launch_fxyi_static(A, L, st, kFxyiPre);
   }
-  const int kc = precond_kc(A.f, g->ny, L);
-  if (kc != A.f.kc) {
-    A.f.kc = kc;
-    A.f.nkb = (A.f.nkx + kc - 1) / kc;
-    A.f.lds_z = size_t(kc) * g->nz * 3 * 16 + 64 * 8;
-  }
   char* w = static_cast<char*>(ws);
   A.rin = r;
   A.s = s;
@@ -752,6 +858,7 @@ extern "C" int pgj_precond_apply(const pgj_grid* g, int L, const void* plan, con
   A.pr = reinterpret_cast<double*>(w + pl.pr);
   A.pg = reinterpret_cast<double*>(w + pl.pg);
   A.zout = z;
+  zpass_choose(A, *g, L);
   hipStream_t st = as_stream(stream);
   if (int e = launch_fxy<kFxyPre>(A, L, st)) return e;
   if (int e = launch_fz<kFzPre>(A, L, st)) return e;

@@ -40,18 +40,13 @@ struct FFTArgsT {
   StateView st;
   int soa;               // vectors (and s) are SoA (L, 3, N) instead of AoS (L, N, 3)
   int group;             // loads per design (s is (designs, 3N), s_hat (designs, 3, nf)); 0: shared
-  int zkc, zslots;       // cubes: kx chunk width of the z pass (0: register-resident) and its partial rows per
+  int zkc, zslots;       // columns per block of the z pass (0: register-resident cubes) and its partial rows per
                          // load, set by zpass_choose; the same for every launch that writes or reads one
                          // workspace's z partials
   const double* rin64;   // FP32 preconditioner apply on AoS vectors: FP64 input residual, rounded to T on load
   double* zout64;        // ... and FP64 output z (exact widening of the T result); both null otherwise
 };
 using FFTArgs = FFTArgsT<double>;
-
-// Index of component c of node `node` of load l in a vector (and of s with l = 0).
-__device__ __forceinline__ int64_t vindex(const FFTArgs& A, int l, int c, int64_t node) {
-  return A.soa ? (int64_t(l) * 3 + c) * A.N + node : (int64_t(l) * A.N + node) * 3 + c;
-}
 
 FFTArgs fft_args(const pgj_grid& g, const void* plan);
 int check_fft(const pgj_grid* g);
@@ -63,6 +58,8 @@ bool static_fft(const pgj_grid& g);
 // Whether the LDS z pass of a solve with L loads in all (its workspace's load count) and elements of es bytes
 // takes the wide kx chunks: where these fill the device with more than one round of blocks (64^3 FP64).
 bool zpass_wide(const pgj_grid& g, int L, int es);
+// Columns per block of the runtime z pass (16, 8 or 4) of a workspace of L loads.
+int runtime_chunk(const FFTGeom& f, int L);
 // Sets A.zkc and A.zslots for a workspace of L loads (FFTArgsT).
 template <typename T> void zpass_choose(FFTArgsT<T>& A, const pgj_grid& g, int L);
 template <typename T> int launch_fxy_static(FFTArgsT<T>& A, int L, int mode, hipStream_t s);

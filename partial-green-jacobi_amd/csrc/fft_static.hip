@@ -1047,8 +1047,8 @@ static int zkc_of(const pgj_grid& g, int L) {
 template <typename R>
 void zpass_choose(FFTArgsT<R>& A, const pgj_grid& g, int L) {
   if (!static_cube(g)) {
-    A.zkc = A.f.kc;
-    A.zslots = A.f.nkb * g.ny;
+    A.zkc = runtime_chunk(A.f, L);
+    A.zslots = (g.ny * A.f.nkx + A.zkc - 1) / A.zkc;
     return;
   }
   switch (g.nx) {

@@ -128,18 +128,82 @@ inline Factors factorize(int n) {
   return f;
 }
 
+// Radix plan of one axis for the runtime-shaped kernels (fft.hip): the fewest stages of radices 10..2, ties to the plan
+// with the largest smallest radix (40 = 8 x 5, 60 = 10 x 6, 75 = 5 x 5 x 3). A group of G lanes carries a line through
+// all its stages, so a wavefront holds 64 / G whole lines and a transform needs no block barrier.
+constexpr int kMaxAxis = 256;
+struct AxisPlan {
+  struct Stage {
+    int R, nb, Ns, tws;  // radix, butterflies n / R, product of the earlier radices, twiddle step n / (Ns R)
+    unsigned mNs;        // j / Ns = j mNs >> 16 for j < n
+  } st[4];
+  int n, count, G, lpw;  // lanes of a line, lines of a wavefront
+  unsigned mG, mL;       // lane / G and lane / lpw as products >> 16
+};
+
+inline unsigned magic16(int d) { return 65536u / unsigned(d) + 1; }  // q = x magic >> 16, exact for x d < 65536
+inline unsigned magic32(int d) { return unsigned((uint64_t(1) << 32) / unsigned(d) + 1); }  // q = x magic >> 32, d > 1
+
+// Stages of `left` with radices <= cap into r[at...]: the best plan found so far is (best, r).
+inline void axis_search(int left, int cap, int at, int lowest, int (&cur)[8], int& best, int& best_low, int (&r)[8]) {
+  if (left == 1) {
+    if (at < best || (at == best && lowest > best_low)) {
+      best = at;
+      best_low = lowest;
+      for (int i = 0; i < at; ++i) r[i] = cur[i];
+    }
+    return;
+  }
+  if (at == 8) return;
+  for (int R = cap; R >= 2; --R) {
+    if (left % R) continue;
+    cur[at] = R;
+    axis_search(left / R, R, at + 1, R, cur, best, best_low, r);
+  }
+}
+
+inline AxisPlan make_axis_plan(int n) {
+  AxisPlan a{};
+  a.n = n;
+  int cur[8], r[8] = {}, best = 9, low = 0;
+  axis_search(n, 10, 0, 99, cur, best, low, r);
+  a.count = best <= 4 ? best : -1;  // lengths up to 256 take at most three stages
+  a.G = 1;
+  int Ns = 1;
+  for (int s = 0; s < a.count; ++s) {
+    a.st[s] = AxisPlan::Stage{r[s], n / r[s], Ns, n / (Ns * r[s]), magic16(Ns)};
+    Ns *= r[s];
+    if (n / r[s] > a.G) a.G = n / r[s];
+  }
+  if (a.G > 64) a.G = 64;  // 243 = 9 x 9 x 3 alone: its last stage takes two butterflies per lane
+  a.lpw = 64 / a.G;
+  a.mG = magic16(a.G);
+  a.mL = magic16(a.lpw);
+  return a;
+}
+
+// Plans of every length up to kMaxAxis, made once (count -1 where a length has another prime factor).
+inline const AxisPlan& axis_plan(int n) {
+  struct Table {
+    AxisPlan p[kMaxAxis + 1];
+    Table() {
+      for (int i = 1; i <= kMaxAxis; ++i) p[i] = make_axis_plan(i);
+    }
+  };
+  static const Table t;
+  static const AxisPlan none{{}, 0, -1, 1, 64, 0, 0};
+  return n >= 1 && n <= kMaxAxis ? t.p[n] : none;
+}
+
 struct FFTGeom {
   int nz, ny, nx;
   int nkx;          // nx/2 + 1
   int M;            // complex length of the x transform: nx/2 (even nx) or nx (odd)
   int rs;           // row stride of a plane row in LDS (complex): max(nkx, M)
   int64_t nf;       // nz*ny*nkx
-  int comps;        // components per plane block in the xy kernels (3 or 1)
-  int kc;           // kx columns per block in the z kernel
-  int nkb;          // ceil(nkx/kc)
-  int threads_xy, threads_z;
-  size_t lds_xy, lds_z;
-  Factors fx, fy, fz;
+  int nkb;          // the workspace holds nkb * ny rows of z pass partials per load
+  AxisPlan px, py, pz;
+  unsigned mnx, mnkx;  // magic32 of nx and nkx
   int valid;        // some FFT path supports the grid
   int runtime_ok;   // the runtime-shaped kernels (fft.hip) support it
 };
@@ -166,6 +230,8 @@ inline bool stages_fit(const Factors& f, int lines, int threads) {
   return true;
 }
 
+constexpr int kMinChunk = 4;  // frequency columns per block of the runtime z pass: 4, 8 or 16
+
 inline FFTGeom fft_geom(const pgj_grid& g) {
   FFTGeom f{};
   f.nz = g.nz; f.ny = g.ny; f.nx = g.nx;
@@ -173,43 +239,37 @@ inline FFTGeom fft_geom(const pgj_grid& g) {
   f.M = (g.nx % 2 == 0) ? g.nx / 2 : g.nx;
   f.rs = f.nkx > f.M ? f.nkx : f.M;
   f.nf = int64_t(g.nz) * g.ny * f.nkx;
-  f.fx = factorize(f.M);
-  f.fy = factorize(g.ny);
-  f.fz = factorize(g.nz);
-  f.valid = f.fx.count >= 0 && f.fy.count >= 0 && f.fz.count >= 0 && g.nx >= 2 && g.ny >= 2 && g.nz >= 2 &&
-            g.nx <= 256 && g.ny <= 256 && g.nz <= 256;
+  const Factors fx = factorize(f.M), fy = factorize(g.ny), fz = factorize(g.nz);
+  f.valid = fx.count >= 0 && fy.count >= 0 && fz.count >= 0 && g.nx >= 2 && g.ny >= 2 && g.nz >= 2 &&
+            g.nx <= kMaxAxis && g.ny <= kMaxAxis && g.nz <= kMaxAxis;
   const size_t plane = size_t(g.ny) * f.rs * 16;
-  f.comps = (3 * plane + 64 <= kLdsLimit) ? 3 : 1;
+  const int comps = (3 * plane + 64 <= kLdsLimit) ? 3 : 1;
   if (plane + 64 > kLdsLimit) f.valid = 0;
-  f.lds_xy = f.comps * plane + 64 * 8;
-  f.threads_xy = 512;
-  // z kernel: kc columns x 3 comps x nz complex
   const size_t col = size_t(g.nz) * 3 * 16;
   int kc = 1;
   while (kc < f.nkx && size_t(kc + 1) * col + 64 * 8 <= 56 * 1024) ++kc;
-  if (g.nx == g.ny && g.ny == g.nz) {
-    // cubes: at least as many rows of per-block partials (nkb n) as any of the compile-time z passes has blocks
+  // grids whose planes and columns the block-wide in-place stages of this library once held in registers: the set of
+  // supported grids, kept as it was
+  if (f.valid)
+    f.valid = stages_fit(fx, comps * g.ny, 512) && stages_fit(fy, comps * f.nkx, 512) && stages_fit(fz, 3 * kc, 256);
+  f.mnx = magic32(g.nx > 1 ? g.nx : 2);
+  f.mnkx = magic32(f.nkx > 1 ? f.nkx : 2);
+  f.px = axis_plan(f.M);
+  f.py = axis_plan(g.ny);
+  f.pz = axis_plan(g.nz);
+  if (static_cube(g)) {
+    // at least as many rows of per-block partials (nkb n) as any of the compile-time z passes has blocks
     // (fft_static.hip, ZWidths and ZReg)
     switch (g.nx) {
       case 16: kc = 3; break;
-      case 24: kc = 4; break;
-      case 32: kc = 4; break;
-      case 48: kc = 4; break;
-      case 64: kc = 4; break;
       case 96: kc = 6; break;
       case 128: kc = 5; break;
-      default: break;
+      default: kc = 4; break;
     }
+  } else {
+    kc = kMinChunk;  // the runtime z pass has at most ceil(ny nkx / kMinChunk) blocks per load
   }
-  f.kc = kc;
   f.nkb = (f.nkx + kc - 1) / kc;
-  f.lds_z = size_t(kc) * col + 64 * 8;
-  f.threads_z = 256;
-  if (f.valid) {
-    const int rows = f.comps * g.ny;
-    f.valid = stages_fit(f.fx, rows, f.threads_xy) && stages_fit(f.fy, f.comps * f.nkx, f.threads_xy) &&
-              stages_fit(f.fz, 3 * f.kc, f.threads_z);
-  }
   f.runtime_ok = f.valid;
   if (static_cube(g)) f.valid = 1;
   return f;
@@ -241,26 +301,13 @@ struct PrecondLayout {
   size_t bytes;
 };
 
-// kx columns per block of the preconditioner apply's z pass: the geometry's
-// chunk, or narrower when the (load, ky, chunk) blocks would not cover 512
-// (few loads), which raises the block count of that pass.
-inline int precond_kc(const FFTGeom& f, int ny, int L) {
-  const int64_t rows = int64_t(L) * ny;
-  if (rows * f.nkb >= 512) return f.kc;
-  const int64_t want = std::min<int64_t>(f.nkx, (512 + rows - 1) / rows);
-  return std::max(1, int((f.nkx + want - 1) / want));
-}
-
 inline PrecondLayout precond_layout(const pgj_grid& g, int L, size_t cs = 16) {
   FFTGeom f = fft_geom(g);
   PrecondLayout p{};
   size_t off = 0;
-  // partial rows for the geometry's chunking and for the preconditioner apply's
-  const int kc = precond_kc(f, g.ny, L);
-  const int nkb = std::max(f.nkb, (f.nkx + kc - 1) / kc);
   p.spec = off; off = align256(off + size_t(L) * 3 * f.nf * cs);
   p.pr = off; off = align256(off + size_t(L) * g.nz * 6 * 8);
-  p.pg = off; off = align256(off + size_t(L) * nkb * g.ny * 4 * 8);
+  p.pg = off; off = align256(off + size_t(L) * f.nkb * g.ny * 4 * 8);
   p.bytes = off;
   return p;
 }

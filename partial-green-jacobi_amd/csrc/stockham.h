@@ -125,17 +125,82 @@ __device__ __forceinline__ void dft(C (&v)[R], const C* tw, int n, int step) {
     v[0] = cadd(v[0], s);
     v[1] = cadd(m, jd);
     v[2] = csub(m, jd);
-  } else {
-    C out[R];
+  } else if constexpr (R == 5 || R == 7) {
+    // pairs v_k +- v_{R-k}: output p is v_0 + sum_k cos(2 pi p k / R) (v_k + v_{R-k}) -+ i sum_k sin(...) (v_k - v_{R-k})
+    constexpr int H = R / 2;
+    constexpr T c5[3] = {T(1), T(0.30901699437494742410), T(-0.80901699437494742410)};
+    constexpr T s5[3] = {T(0), T(0.95105651629515357212), T(0.58778525229247312917)};
+    constexpr T c7[4] = {T(1), T(0.62348980185873353053), T(-0.22252093395631440429), T(-0.90096886790241912624)};
+    constexpr T s7[4] = {T(0), T(0.78183148246802980871), T(0.97492791218182360702), T(0.43388373911755812048)};
+    C t[H], d[H];
 #pragma unroll
-    for (int p = 0; p < R; ++p) {
-      C acc = v[0];
+    for (int k = 1; k <= H; ++k) {
+      t[k - 1] = cadd(v[k], v[R - k]);
+      d[k - 1] = csub(v[k], v[R - k]);
+    }
+    const C v0 = v[0];
+    C sum = v0;
 #pragma unroll
-      for (int q = 1; q < R; ++q) acc = cadd(acc, cmul(v[q], twiddle<INV>(tw, ((p * q) % R) * (n / R), step)));
-      out[p] = acc;
+    for (int k = 0; k < H; ++k) sum = cadd(sum, t[k]);
+    v[0] = sum;
+#pragma unroll
+    for (int p = 1; p <= H; ++p) {
+      C m = v0, s = c2(T(0), T(0));
+#pragma unroll
+      for (int k = 1; k <= H; ++k) {
+        const int a = (p * k) % R, b = a <= H ? a : R - a;
+        const T c = R == 5 ? c5[b < 3 ? b : 0] : c7[b];
+        const T sn = (a <= H ? T(1) : T(-1)) * (R == 5 ? s5[b < 3 ? b : 0] : s7[b]);
+        m = c2(fma(c, t[k - 1].x, m.x), fma(c, t[k - 1].y, m.y));
+        s = c2(fma(sn, d[k - 1].x, s.x), fma(sn, d[k - 1].y, s.y));
+      }
+      const C js = INV ? c2(-s.y, s.x) : c2(s.y, -s.x);  // -i s, conjugate for the inverse
+      v[p] = cadd(m, js);
+      v[R - p] = csub(m, js);
+    }
+  } else if constexpr (R == 9) {
+    // 3 x 3: x_{j + 3 r} for each j, twiddles W_9^(j p), then across j
+    constexpr T c9[5] = {T(1), T(0.76604444311897803520), T(0.17364817766693034885), T(-0.5), T(-0.93969262078590838405)};
+    constexpr T s9[5] = {T(0), T(0.64278760968653932632), T(0.98480775301220805937), T(0.86602540378443864676),
+                         T(0.34202014332566873304)};
+    C b[3][3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+#pragma unroll
+      for (int p = 0; p < 3; ++p) b[j][p] = v[j + 3 * p];
+      dft<3, INV>(b[j], tw, n, step);
+#pragma unroll
+      for (int p = 1; p < 3; ++p)
+        if (j > 0) b[j][p] = cmul(b[j][p], C(c2(c9[j * p], INV ? s9[j * p] : -s9[j * p])));
     }
 #pragma unroll
-    for (int p = 0; p < R; ++p) v[p] = out[p];
+    for (int p = 0; p < 3; ++p) {
+      C a[3] = {b[0][p], b[1][p], b[2][p]};
+      dft<3, INV>(a, tw, n, step);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) v[p + 3 * q] = a[q];
+    }
+  } else {
+    // R = 10 = 2 x 5: 2-point transforms of x_j, x_{j+5}, twiddles W_10^j on the differences, then 5-point ones over j
+    static_assert(R == 10, "radix");
+    constexpr T c10[5] = {T(1), T(0.80901699437494742410), T(0.30901699437494742410), T(-0.30901699437494742410),
+                          T(-0.80901699437494742410)};
+    constexpr T s10[5] = {T(0), T(0.58778525229247312917), T(0.95105651629515357212), T(0.95105651629515357212),
+                          T(0.58778525229247312917)};
+    C a[5], b[5];
+#pragma unroll
+    for (int j = 0; j < 5; ++j) {
+      a[j] = cadd(v[j], v[j + 5]);
+      b[j] = csub(v[j], v[j + 5]);
+      if (j > 0) b[j] = cmul(b[j], C(c2(c10[j], INV ? s10[j] : -s10[j])));
+    }
+    dft<5, INV>(a, tw, n, step);
+    dft<5, INV>(b, tw, n, step);
+#pragma unroll
+    for (int q = 0; q < 5; ++q) {
+      v[2 * q] = a[q];
+      v[2 * q + 1] = b[q];
+    }
   }
 }
 
