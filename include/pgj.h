@@ -449,6 +449,18 @@ int pgj_pcg_pre_step(int B, int64_t n, double* u, double* r, const double* p, co
  * pcg.py:495-508); minv_stride is 0 (one (n) diagonal for every batch) or n. */
 int pgj_pcg_post_step(int B, int64_t n, const double* r, double* z, const double* minv, int64_t minv_stride,
                       double* p, double* rz, double* ws, void* stream);
+/* count iterations of one load of the scalar operator (L = 1, AoS vectors of 3N
+ * FP64 values), each M^-1 r, the post-step, K p and the pre-step as above, with
+ * p.Ap and r.z formed inside the apply and the preconditioner. It follows a
+ * pgj_pcg_pre_step or another pgj_pcg_fi_iterate on the same ws. iteration is the number of the
+ * first one. sc, s_hat: the scale and its spectrum (both NULL: unscaled). fi_ws:
+ * pgj_pcg_fi_ws_bytes, precond_ws: pgj_precond_ws_bytes(g, 1). */
+size_t pgj_pcg_fi_ws_bytes(const pgj_grid* g);
+int pgj_pcg_fi_iterate(const pgj_grid* g, const double* a, const void* plan, const double* sc, const void* s_hat,
+                       double* u, double* r, double* p, double* Ap, double* z, double* rz, const double* rhs_norm,
+                       double* best_u, double* best_res, double* res, uint8_t* improved, int64_t* state, double tol,
+                       double near_tol, int64_t iteration, int count, int latched, double* ws, double* fi_ws,
+                       void* precond_ws, void* stream);
 /* The same four steps on FP32 vectors (u, r, p, Ap, z, best_u, minv); sums,
  * rz, rhs_norm, res and best_res stay FP64. The inner PCG of
  * solve_ir_batched (solver/src/runtime/fi/source/femlib/batched/ir.py:84-92)

@@ -237,7 +237,7 @@ __global__ __launch_bounds__(MAXT) void hex8_rowmarch(RowArgsT<T> A) {
 #pragma unroll
               for (int d = 0; d < 3; ++d) {
                 st(out, at(rb + xo + xi, d), accL[j][xi][d]);
-                if (MODE == kModePCG) pq = fma(double(nodeLo[j][xi][d]), double(accL[j][xi][d]), pq);
+                if (MODE != kModeApply) pq = fma(double(nodeLo[j][xi][d]), double(accL[j][xi][d]), pq);
               }
           }
         }
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(MAXT) void hex8_rowmarch(RowArgsT<T> A) {
           aU[j][xi] = aN[j][xi];
         }
     }
-    if (MODE == kModePCG) {
+    if (MODE != kModeApply) {
       const double total = block_sum(pq, reinterpret_cast<double*>(lds + 2 * slot_size));
       if (threadIdx.x == 0) A.ppq[int64_t(l) * A.ppq_stride + blockIdx.y * gridDim.x + rg] = total;
     }
@@ -373,7 +373,7 @@ __global__ __launch_bounds__(MAXT) void hex8_rowmarch(RowArgsT<T> A) {
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
               st(out, at(rb + xo + xi, d), accL[j][xi][d]);
-              if (MODE == kModePCG) pq = fma(double(nodeL[j][xi][d]), double(accL[j][xi][d]), pq);
+              if (MODE != kModeApply) pq = fma(double(nodeL[j][xi][d]), double(accL[j][xi][d]), pq);
             }
           }
         }
@@ -397,7 +397,7 @@ __global__ __launch_bounds__(MAXT) void hex8_rowmarch(RowArgsT<T> A) {
         }
       }
   }
-  if (MODE == kModePCG) {
+  if (MODE != kModeApply) {
     const double total = block_sum(pq, reinterpret_cast<double*>(lds + 2 * slot_size));
     if (threadIdx.x == 0) A.ppq[int64_t(l) * A.ppq_stride + blockIdx.y * gridDim.x + rg] = total;
   }
@@ -882,6 +882,8 @@ int launch_rowmarch(const pgj_grid& g, int L, int mode, RowArgsT<T>& A, hipStrea
   A.N = int64_t(g.nx) * g.ny * g.nz;
   A.cfg = rowmarch_config(g, L, int(sizeof(T)));
   A.coef = coef_of(g);
+  if constexpr (sizeof(T) == 8)
+    if (mode == kModeApplyDot) return launch_rowmarch_m<kModeApplyDot>(g, L, A, s);
   return mode == kModeApply ? launch_rowmarch_m<kModeApply>(g, L, A, s) : launch_rowmarch_m<kModePCG>(g, L, A, s);
 }
 template int launch_rowmarch<double>(const pgj_grid&, int, int, RowArgsT<double>&, hipStream_t);

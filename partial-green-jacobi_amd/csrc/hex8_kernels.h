@@ -7,7 +7,8 @@
 
 namespace pgj {
 
-enum { kModeApply = 0, kModePCG = 1 };
+// kModeApplyDot: the apply on AoS vectors with the u . K u partials of every block (one load).
+enum { kModeApply = 0, kModePCG = 1, kModeApplyDot = 2 };
 
 template <typename T>
 struct RowArgsT {
@@ -20,7 +21,7 @@ struct RowArgsT {
   T* out;                // apply: K u; PCG: q = K p
   const uint8_t* mask;   // apply: optional active mask
   StateView st;          // PCG: active mask
-  double* ppq;           // per-block p.q partials, per load stride ppq_stride
+  double* ppq;           // PCG, ApplyDot: per-block p.q (u.out) partials, per load stride ppq_stride
   int ppq_stride;
   int group;             // loads per design (a is (designs, N)); 0: one shared a
 };

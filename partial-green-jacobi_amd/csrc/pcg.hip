@@ -7,6 +7,8 @@
 // :636-669 (compiled pre/post steps), :677-727 (latch kernels, best copy).
 #include <cmath>
 
+#include "fft_kernels.h"
+#include "hex8_kernels.h"
 #include "layout.h"
 #include "pgj_internal.h"
 
@@ -49,11 +51,14 @@ __global__ void pcg_norms(int B, const double* part, int nblk, double* out) {
   }
 }
 
-// part[b][blk] = partial x_b . y_b; with minv, z = minv * x is stored and y is ignored (Jacobi r.z).
+// part[b][blk] = partial x_b . y_b; with minv, z = minv * x is stored and y is ignored (Jacobi r.z). With `rz`, its
+// value goes to `rz_old`, so that the pass after this one can replace rz while its blocks still read the old one.
 template <typename T>
 __global__ __launch_bounds__(kVecThreads) void pcg_dot(const T* x, const T* y, const T* minv, T* z, int64_t n,
-                                                       int64_t minv_stride, double* part) {
+                                                       int64_t minv_stride, double* part, const double* rz,
+                                                       double* rz_old) {
   __shared__ double red[kVecThreads / 64];
+  if (rz && blockIdx.x == 0 && threadIdx.x == 0) rz_old[blockIdx.y] = rz[blockIdx.y];
   const int64_t off = int64_t(blockIdx.y) * n;
   const int64_t moff = int64_t(blockIdx.y) * minv_stride;
   double s = 0.0;
@@ -82,14 +87,23 @@ __global__ void pcg_reduce(int B, const double* part, int nblk, double* out) {
 }
 
 // alpha = rz / max(pAp, eps), 0 where pAp is not finite or <= 0; u += alpha p;
-// r -= alpha Ap; rr_part = partial |r|^2 of the updated residual.
+// r -= alpha Ap; rr_part = partial |r|^2 of the updated residual. The best residuals and the stop iteration so far go
+// to `best_old` and `stop_old` for pcg_best, whose blocks read them while others already write the new ones; rz goes to
+// `rz_old` likewise, for pcg_update_p where no pcg_dot precedes it.
 template <typename T>
 __global__ __launch_bounds__(kVecThreads) void pcg_update_ur(T* u, T* r, const T* p, const T* Ap, int64_t n,
                                                              const double* pap_part, int nblk, const double* rz,
-                                                             double* rr_part) {
+                                                             double* rr_part, const double* best_res,
+                                                             const int64_t* state, double* best_old,
+                                                             int64_t* stop_old, double* rz_old) {
   __shared__ double red[kVecThreads / 64];
   __shared__ double s_alpha;
   const int b = blockIdx.y;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    best_old[b] = best_res[b];
+    rz_old[b] = rz[b];
+    if (b == 0) *stop_old = state[0];
+  }
   if (threadIdx.x < 64) {
     const double pap = wave_reduce_partials(pap_part + int64_t(b) * nblk, nblk, 1);
     if (threadIdx.x == 0) {
@@ -111,57 +125,53 @@ __global__ __launch_bounds__(kVecThreads) void pcg_update_ur(T* u, T* r, const T
   if (threadIdx.x == 0) rr_part[int64_t(b) * gridDim.x + blockIdx.x] = t;
 }
 
-// res = sqrt(|r|^2) / rhs_norm; improved = res < best_res (latched: and no stop
-// recorded yet); best_res updated. Latched: state[0] (stop iteration) is set to
-// `iteration` the first time every res < tol; state[1] to 1 the first time
-// every res < near_tol (near_tol > 0 only). One block.
-__global__ void pcg_finalize(int B, const double* rr_part, int nblk, const double* rhs_norm, double* res,
-                             double* best_res, uint8_t* improved, int64_t* state, double tol, double near_tol,
-                             int64_t iteration, int latched) {
-  const int wave = threadIdx.x >> 6, nw = blockDim.x >> 6, lane = threadIdx.x & 63;
-  const int64_t stopped = latched ? state[0] : 0;
-  int ok = 1, near = 1;
-  for (int b = wave; b < B; b += nw) {
-    const double rr = wave_reduce_partials(rr_part + int64_t(b) * nblk, nblk, 1);
-    const double rv = sqrt(rr) / rhs_norm[b];
-    const bool imp = rv < best_res[b] && stopped == 0;
-    ok &= rv < tol;
-    near &= rv < near_tol;
-    if (lane == 0) {
-      res[b] = rv;
-      improved[b] = imp;
-      if (imp) best_res[b] = rv;
-    }
+// res = sqrt(|r|^2) / rhs_norm; improved = res < best_res (latched: and no stop recorded yet); best_res updated and u
+// copied to best_u where improved. Latched: state[0] (stop iteration) is set to `iteration` the first time every
+// res < tol; state[1] to 1 the first time every res < near_tol (near_tol > 0 only), by the first block. Every block
+// forms its batch's residual from the partials (at most 1024, one pass of a wavefront), which costs it less than the
+// launch of its own that this test took before the copy: 2.9 of 24 us of vector kernels an iteration at 32^3.
+template <typename T>
+__global__ __launch_bounds__(kVecThreads) void pcg_best(const T* u, T* best_u, int64_t n, int B, const double* rr_part,
+                                                        int nblk, const double* rhs_norm, const double* best_old,
+                                                        const int64_t* stop_old, double* res, double* best_res,
+                                                        uint8_t* improved, int64_t* state, double tol, double near_tol,
+                                                        int64_t iteration, int latched) {
+  const int b = blockIdx.y, wave = threadIdx.x >> 6;
+  const int64_t stopped = latched ? *stop_old : 0;
+  const double rv = sqrt(wave_reduce_partials(rr_part + int64_t(b) * nblk, nblk, 1)) / rhs_norm[b];
+  const bool imp = rv < best_old[b] && stopped == 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    res[b] = rv;
+    improved[b] = imp;
+    if (imp) best_res[b] = rv;
+  }
+  if (imp) {
+    const int64_t off = int64_t(b) * n;
+    PGJ_GRID_LOOP(i, n) best_u[off + i] = u[off + i];
+  }
+  if (!latched || blockIdx.x != 0 || b != 0) return;
+  int ok = rv < tol, near = rv < near_tol;
+  for (int k = 1 + wave; k < B; k += kVecThreads / 64) {
+    const double v = sqrt(wave_reduce_partials(rr_part + int64_t(k) * nblk, nblk, 1)) / rhs_norm[k];
+    ok &= v < tol;
+    near &= v < near_tol;
   }
   const int all_ok = __syncthreads_and(ok);
   const int all_near = __syncthreads_and(near);
-  if (threadIdx.x == 0 && latched) {
+  if (threadIdx.x == 0) {
     if (stopped == 0 && all_ok) state[0] = iteration;
     if (near_tol > 0.0 && state[1] == 0 && all_near) state[1] = 1;
   }
 }
 
-template <typename T>
-__global__ __launch_bounds__(kVecThreads) void pcg_copy_best(const T* u, T* best_u, const uint8_t* improved,
-                                                             int64_t n) {
-  const int b = blockIdx.y;
-  if (!improved[b]) return;
-  const int64_t off = int64_t(b) * n;
-  PGJ_GRID_LOOP(i, n) best_u[off + i] = u[off + i];
-}
-
-// beta = rz_new / max(rz_old, eps); p = z + beta p (rz_old read here, replaced by pcg_reduce afterwards).
+// beta = rz_new / max(rz_old, eps); p = z + beta p; rz = rz_new.
 template <typename T>
 __global__ __launch_bounds__(kVecThreads) void pcg_update_p(const T* z, T* p, int64_t n, const double* rz_part,
-                                                            int nblk, const double* rz) {
-  __shared__ double s_beta;
+                                                            int nblk, int stride, const double* rz_old, double* rz) {
   const int b = blockIdx.y;
-  if (threadIdx.x < 64) {
-    const double rzn = wave_reduce_partials(rz_part + int64_t(b) * nblk, nblk, 1);
-    if (threadIdx.x == 0) s_beta = rzn / fmax(rz[b], kPcgEps);
-  }
-  __syncthreads();
-  const T beta = T(s_beta);
+  const double rzn = wave_reduce_partials(rz_part + int64_t(b) * nblk * stride, nblk, stride);
+  const T beta = T(rzn / fmax(rz_old[b], kPcgEps));
+  if (blockIdx.x == 0 && threadIdx.x == 0) rz[b] = rzn;
   const int64_t off = int64_t(b) * n;
   PGJ_GRID_LOOP(i, n) p[off + i] = fma(beta, p[off + i], z[off + i]);
 }
@@ -180,11 +190,28 @@ using namespace pgj;
 
 namespace {
 bool pcg_shape_ok(int B, int64_t n) { return B >= 1 && B <= 65535 && n >= 1 && n <= (int64_t(1) << 40); }
+
+// Workspace in doubles: partials of p.Ap, |r|^2 and r.z (B x nblk each), then the values a pass replaces while its blocks
+// read them: best residuals (B), r.z (B), stop iteration.
+struct PcgWs {
+  size_t pap, rr, rz, best_old, rz_old, stop_old, doubles;
+};
+PcgWs pcg_ws(int B, int64_t n) {
+  const size_t row = size_t(B) * vec_blocks(n);
+  PcgWs w{};
+  w.rr = row;
+  w.rz = 2 * row;
+  w.best_old = 3 * row;
+  w.rz_old = w.best_old + B;
+  w.stop_old = w.rz_old + B;
+  w.doubles = w.stop_old + 1;
+  return w;
+}
 }  // namespace
 
 extern "C" size_t pgj_pcg_ws_bytes(int B, int64_t n) {
   if (!pcg_shape_ok(B, n)) return 0;
-  return align256(size_t(B) * vec_blocks(n) * 8 * 3);
+  return align256(pcg_ws(B, n).doubles * 8);
 }
 
 namespace {
@@ -205,7 +232,8 @@ int pcg_init_t(int B, int64_t n, const T* r, const T* z, T* p, double* rz, doubl
   PGJ_REQUIRE(pcg_shape_ok(B, n) && r && z && p && rz && ws, "invalid pcg init arguments");
   hipStream_t s = as_stream(stream);
   const int nblk = vec_blocks(n);
-  hipLaunchKernelGGL(pcg_dot<T>, dim3(nblk, B), dim3(kVecThreads), 0, s, r, z, nullptr, nullptr, n, int64_t(0), ws);
+  hipLaunchKernelGGL(pcg_dot<T>, dim3(nblk, B), dim3(kVecThreads), 0, s, r, z, nullptr, nullptr, n, int64_t(0), ws,
+                     nullptr, nullptr);
   PGJ_LAUNCHED("pcg_dot");
   hipLaunchKernelGGL(pcg_reduce, batch_grid(B), dim3(256), 0, s, B, ws, nblk, rz);
   PGJ_LAUNCHED("pcg_reduce");
@@ -225,17 +253,18 @@ int pcg_pre_step_t(int B, int64_t n, T* u, T* r, const T* p, const T* Ap, const 
               "invalid pcg pre-step arguments");
   hipStream_t s = as_stream(stream);
   const int nblk = vec_blocks(n);
-  double* pap = ws;
-  double* rr = ws + size_t(B) * nblk;
-  hipLaunchKernelGGL(pcg_dot<T>, dim3(nblk, B), dim3(kVecThreads), 0, s, p, Ap, nullptr, nullptr, n, int64_t(0), pap);
+  const PcgWs w = pcg_ws(B, n);
+  double *pap = ws + w.pap, *rr = ws + w.rr, *best_old = ws + w.best_old;
+  int64_t* stop_old = reinterpret_cast<int64_t*>(ws + w.stop_old);
+  hipLaunchKernelGGL(pcg_dot<T>, dim3(nblk, B), dim3(kVecThreads), 0, s, p, Ap, nullptr, nullptr, n, int64_t(0), pap,
+                     nullptr, nullptr);
   PGJ_LAUNCHED("pcg_dot");
-  hipLaunchKernelGGL(pcg_update_ur<T>, dim3(nblk, B), dim3(kVecThreads), 0, s, u, r, p, Ap, n, pap, nblk, rz, rr);
+  hipLaunchKernelGGL(pcg_update_ur<T>, dim3(nblk, B), dim3(kVecThreads), 0, s, u, r, p, Ap, n, pap, nblk, rz, rr,
+                     best_res, state, best_old, stop_old, ws + w.rz_old);
   PGJ_LAUNCHED("pcg_update_ur");
-  hipLaunchKernelGGL(pcg_finalize, dim3(1), dim3(1024), 0, s, B, rr, nblk, rhs_norm, res, best_res, improved, state,
-                     tol, near_tol, iteration, latched);
-  PGJ_LAUNCHED("pcg_finalize");
-  hipLaunchKernelGGL(pcg_copy_best<T>, dim3(nblk, B), dim3(kVecThreads), 0, s, u, best_u, improved, n);
-  PGJ_LAUNCHED("pcg_copy_best");
+  hipLaunchKernelGGL(pcg_best<T>, dim3(nblk, B), dim3(kVecThreads), 0, s, u, best_u, n, B, rr, nblk, rhs_norm, best_old,
+                     stop_old, res, best_res, improved, state, tol, near_tol, iteration, latched);
+  PGJ_LAUNCHED("pcg_best");
   return PGJ_OK;
 }
 
@@ -246,13 +275,13 @@ int pcg_post_step_t(int B, int64_t n, const T* r, T* z, const T* minv, int64_t m
               "invalid pcg post-step arguments");
   hipStream_t s = as_stream(stream);
   const int nblk = vec_blocks(n);
-  double* part = ws + size_t(2) * B * nblk;
-  hipLaunchKernelGGL(pcg_dot<T>, dim3(nblk, B), dim3(kVecThreads), 0, s, r, z, minv, z, n, minv_stride, part);
+  const PcgWs w = pcg_ws(B, n);
+  double *part = ws + w.rz, *rz_old = ws + w.rz_old;
+  hipLaunchKernelGGL(pcg_dot<T>, dim3(nblk, B), dim3(kVecThreads), 0, s, r, z, minv, z, n, minv_stride, part, rz,
+                     rz_old);
   PGJ_LAUNCHED("pcg_dot");
-  hipLaunchKernelGGL(pcg_update_p<T>, dim3(nblk, B), dim3(kVecThreads), 0, s, z, p, n, part, nblk, rz);
+  hipLaunchKernelGGL(pcg_update_p<T>, dim3(nblk, B), dim3(kVecThreads), 0, s, z, p, n, part, nblk, 1, rz_old, rz);
   PGJ_LAUNCHED("pcg_update_p");
-  hipLaunchKernelGGL(pcg_reduce, batch_grid(B), dim3(256), 0, s, B, part, nblk, rz);
-  PGJ_LAUNCHED("pcg_reduce");
   return PGJ_OK;
 }
 }  // namespace
@@ -301,4 +330,62 @@ extern "C" int pgj_pcg32_pre_step(int B, int64_t n, float* u, float* r, const fl
 extern "C" int pgj_pcg32_post_step(int B, int64_t n, const float* r, float* z, const float* minv,
                                    int64_t minv_stride, float* p, double* rz, double* ws, void* stream) {
   return pcg_post_step_t(B, n, r, z, minv, minv_stride, p, rz, ws, stream);
+}
+
+// One load of the scalar operator with its Green preconditioner: what pgj_precond_apply, pgj_pcg_post_step, pgj_hex8_apply
+// and pgj_pcg_pre_step do, `count` times, from one call. p.Ap comes from the apply's own blocks and r.z from the z pass of
+// the preconditioner (Parseval), so seven launches an iteration take the place of nine, and no host work lies between
+// them: at 32^3 the loop over four entry points was bound by the host, 76 us an iteration for 45 us of kernels.
+extern "C" size_t pgj_pcg_fi_ws_bytes(const pgj_grid* g) {
+  return g ? align256(size_t(hex8_blocks_bound(*g)) * 8) : 0;
+}
+
+extern "C" int pgj_pcg_fi_iterate(const pgj_grid* g, const double* a, const void* plan, const double* sc,
+                                  const void* s_hat, double* u, double* r, double* p, double* Ap, double* z, double* rz,
+                                  const double* rhs_norm, double* best_u, double* best_res, double* res,
+                                  uint8_t* improved, int64_t* state, double tol, double near_tol, int64_t iteration,
+                                  int count, int latched, double* ws, double* fi_ws, void* precond_ws, void* stream) {
+  if (int e = check_grid(g)) return e;
+  if (int e = check_fft(g)) return e;
+  PGJ_REQUIRE(a && plan && u && r && p && Ap && z && rz && rhs_norm && best_u && best_res && res && improved && state &&
+                  ws && fi_ws && precond_ws && count >= 0 && (sc == nullptr) == (s_hat == nullptr),
+              "invalid pcg iterate arguments");
+  hipStream_t s = as_stream(stream);
+  const int64_t n = int64_t(g->nx) * g->ny * g->nz * 3;
+  const int nblk = vec_blocks(n);
+  const PcgWs w = pcg_ws(1, n);
+  double *rr = ws + w.rr, *best_old = ws + w.best_old, *rz_old = ws + w.rz_old;
+  int64_t* stop_old = reinterpret_cast<int64_t*>(ws + w.stop_old);
+  // the partials of r.z as the preconditioner's z pass leaves them
+  FFTArgs F = fft_args(*g, plan);
+  zpass_choose(F, *g, 1);
+  const double* rz_part = reinterpret_cast<const double*>(static_cast<char*>(precond_ws) + precond_layout(*g, 1).pg);
+  const bool march = rowmarch_config(*g, 1).valid;
+  for (int k = 0; k < count; ++k) {
+    if (int e = pgj_precond_apply(g, 1, plan, r, sc, s_hat, z, precond_ws, stream)) return e;
+    hipLaunchKernelGGL(pcg_update_p<double>, dim3(nblk, 1), dim3(kVecThreads), 0, s, z, p, n, rz_part, F.zslots, 4,
+                       rz_old, rz);
+    PGJ_LAUNCHED("pcg_update_p");
+    const double* pap = fi_ws;
+    int pblk = hex8_blocks_per_load(*g, 1);
+    if (march) {
+      RowArgs A{};
+      A.a = a; A.u = p; A.out = Ap; A.ppq = fi_ws; A.ppq_stride = pblk;
+      if (int e = launch_rowmarch(*g, 1, kModeApplyDot, A, s)) return e;
+    } else {
+      if (int e = pgj_hex8_apply(g, 1, a, p, nullptr, Ap, stream)) return e;
+      pap = ws + w.pap;
+      pblk = nblk;
+      hipLaunchKernelGGL(pcg_dot<double>, dim3(nblk, 1), dim3(kVecThreads), 0, s, p, Ap, nullptr, nullptr, n, int64_t(0),
+                         ws + w.pap, nullptr, nullptr);
+      PGJ_LAUNCHED("pcg_dot");
+    }
+    hipLaunchKernelGGL(pcg_update_ur<double>, dim3(nblk, 1), dim3(kVecThreads), 0, s, u, r, p, Ap, n, pap, pblk, rz, rr,
+                       best_res, state, best_old, stop_old, rz_old);
+    PGJ_LAUNCHED("pcg_update_ur");
+    hipLaunchKernelGGL(pcg_best<double>, dim3(nblk, 1), dim3(kVecThreads), 0, s, u, best_u, n, 1, rr, nblk, rhs_norm,
+                       best_old, stop_old, res, best_res, improved, state, tol, near_tol, iteration + k, latched);
+    PGJ_LAUNCHED("pcg_best");
+  }
+  return PGJ_OK;
 }

@@ -242,6 +242,27 @@ class Operator:
     def _unscaled_green(self, r):
         return self.green_precond(r)
 
+    def native_pcg_steps(self, work, u, r, p, ap, best_u, tol, near_tol, latched):
+        """``steps(iteration, count)``: that many iterations of ``solve_pcg_batched`` in one library call, or None where
+        this operator's apply or preconditioner is not the one this class and ``set_alpha`` attach."""
+        own = self.__dict__
+        precond = own.get('apply_precond')
+        if type(self) is not Operator or self.dtype != torch.float64 or type(precond) is not AttachedGreen \
+                or precond.op is not self or any(name in own for name in ('apply', 'green_precond', '_apply_call')):
+            return None
+        z = torch.empty_like(r)
+        fi_ws = torch.empty(_lib.lib().pgj_pcg_fi_ws_bytes(self.grid) // 8, dtype=torch.float64, device=self.device)
+
+        def steps(iteration, count):
+            s, shat = precond.fields()
+            _lib.call('pgj_pcg_fi_iterate', self.grid, _lib.ptr(self._material_field), _lib.ptr(self._plan),
+                      _lib.ptr(s), _lib.ptr(shat), _lib.ptr(u), _lib.ptr(r), _lib.ptr(p), _lib.ptr(ap), _lib.ptr(z),
+                      _lib.ptr(work.rz), _lib.ptr(work.rhs_norm), _lib.ptr(best_u), _lib.ptr(work.best_res),
+                      _lib.ptr(work.res), _lib.ptr(work.improved), _lib.ptr(work.state), float(tol), float(near_tol),
+                      iteration, count, int(latched), _lib.ptr(work.ws), _lib.ptr(fi_ws),
+                      _lib.ptr(self._workspace(1)), _lib.stream())
+        return steps
+
 
 def build(rho, lam=LAMBDA_STUDY2, mu=MU_STUDY2, device='cuda', dtype=torch.float64):
     """Operator + FP64 FI Green with alpha = 0 attached (``adaptive_green_scaling/study.py:61-77``)."""
@@ -271,17 +292,33 @@ def scale(op, alpha):
     return s
 
 
+class AttachedGreen:
+    """``op.apply_precond`` as ``set_alpha`` attaches it: r -> P s G s P r with the operator's current scale, or
+    P G P r."""
+
+    __slots__ = ('op', 'scaled')
+
+    def __init__(self, op, scaled):
+        self.op, self.scaled = op, scaled
+
+    def fields(self):
+        return (self.op._scale, self.op._scale_hat) if self.scaled else (None, None)
+
+    def __call__(self, r):
+        return self.op.green_precond(r, *self.fields())
+
+
 def set_alpha(op, alpha):
     """Attach M_alpha^-1 r = P(s G(s P r)) as ``op.apply_precond`` (``adaptive_green_scaling/study.py:91-101``)."""
     if alpha == 0:
         op._scale = op._scale_hat = None
-        op.apply_precond = lambda r: op.green_precond(r)
+        op.apply_precond = AttachedGreen(op, False)
     else:
         if op._log_diagonal is None:
             q = diagonal(op).log()
             op._log_diagonal = q - q.mean()   # the attribute the reference attaches (study.py:96-98)
         s = scale(op, alpha)
         op._scale, op._scale_hat = s, op.scale_spectrum(s)
-        op.apply_precond = lambda r: op.green_precond(r, op._scale, op._scale_hat)
+        op.apply_precond = AttachedGreen(op, True)
     op._alpha = float(alpha)
     return op

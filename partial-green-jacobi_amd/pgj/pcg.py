@@ -183,12 +183,31 @@ def solve_pcg_batched(op, rhs, *, tol=1e-6, max_iter=2000, verbose=False, log_ev
     recycle_stride = max(int(recycle_stride), 1)
     tag = {'eager': '', 'compiled': '', 'triton': ':Triton', 'cuda': ':CUDA'}[update_mode]
 
+    # an operator that knows this loop runs the iterations up to the next host check in one call
+    steps = native = None
+    if B == 1 and dt == torch.float64 and not jacobi and recycle is None and not verbose:
+        native = getattr(op, 'native_pcg_steps', None)
+
     n_iter_final = max_iter
-    for it in range(max_iter):
-        ap = _vector(op.apply(p), (B, n), 'op.apply(p)', dt)
-        if recycle is not None and it % recycle_stride == 0:
-            recycle(it, p.clone(), ap)
-        work.pre_step(u, r, p, ap, best_u, tol, near_tol, it + 1, latched)
+    it = 0
+    while it < max_iter:
+        if steps is None or it == 0:
+            if it > 0:
+                if jacobi:
+                    work.post_step(r, z, p, minv)
+                else:
+                    z = _vector(apply_m_inv(r), (B, n), 'apply_precond(r)', dt)
+                    work.post_step(r, z, p)
+            ap = _vector(op.apply(p), (B, n), 'op.apply(p)', dt)
+            if recycle is not None and it % recycle_stride == 0:
+                recycle(it, p.clone(), ap)
+            work.pre_step(u, r, p, ap, best_u, tol, near_tol, it + 1, latched)
+            if it == 0 and native is not None:
+                steps = native(work, u, r, p, torch.empty_like(ap), best_u, tol, near_tol, latched)
+        else:
+            count = min(host_check_stride - it % host_check_stride, max_iter - it)
+            steps(it + 1, count)
+            it += count - 1
 
         if verbose and ((it + 1) % log_every == 0 or it == 0):
             print(f'    [PCG-batched{tag}] iter {it + 1:5d}  max_res={work.res.max().item():.3e}  '
@@ -212,13 +231,7 @@ def solve_pcg_batched(op, rhs, *, tol=1e-6, max_iter=2000, verbose=False, log_ev
             else:
                 out = (work.best_res if latched else work.res).clone()
             return best_u, logical, out
-        if (it + 1) == max_iter:
-            break
-        if jacobi:
-            work.post_step(r, z, p, minv)
-        else:
-            z = _vector(apply_m_inv(r), (B, n), 'apply_precond(r)', dt)
-            work.post_step(r, z, p)
+        it += 1
 
     if verbose:
         print(f'    [PCG-batched{tag}] max_iter={max_iter} reached, max_res={work.res.max().item():.3e}')
