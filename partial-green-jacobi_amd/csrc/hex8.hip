@@ -116,7 +116,10 @@ __global__ __launch_bounds__(MAXT) void hex8_rowmarch(RowArgsT<T> A) {
   const int src_left = (xl + c.nl - 1) % c.nl;  // lane holding x - 1
   if constexpr (PLANE) {
     T nodeU[R + 1][XPL][3];
-    T nodeLo[R][XPL][3];             // bottom-plane nodes of the owned rows (p.q)
+    // bottom-plane nodes of the owned rows for p.q: held, or (two FP64 x per lane) read again from the cache, because
+    // the registers they take would spill
+    constexpr bool RELOAD = XPL == 2 && sizeof(T) == 8;
+    T nodeLo[R][XPL][3];
     T PL[R][XPL][3][4];              // in-plane modes of the bottom plane, per element column
     T CM[R][XPL][3][4];              // modal forces on the bottom plane from the layer below
     T accL[R + 1][XPL][3];
@@ -237,7 +240,10 @@ __global__ __launch_bounds__(MAXT) void hex8_rowmarch(RowArgsT<T> A) {
 #pragma unroll
               for (int d = 0; d < 3; ++d) {
                 st(out, at(rb + xo + xi, d), accL[j][xi][d]);
-                if (MODE != kModeApply) pq = fma(double(nodeLo[j][xi][d]), double(accL[j][xi][d]), pq);
+                if (MODE != kModeApply) {
+                  const T own = RELOAD ? ld(in, at(rb + xo + xi, d)) : nodeLo[j][xi][d];
+                  pq = fma(double(own), double(accL[j][xi][d]), pq);
+                }
               }
           }
         }

@@ -41,6 +41,33 @@ bool tuned_shape(const pgj_grid& g, int L, int es, int* R, int* W, int* ZC, int*
 // library's choice); set by pgj_fft_set_plan (the autotuner) and read at every launch of that pass.
 int fft_plan(int n, int es, int pass);
 
+// Row waves and planes per block of the FP64 plane-carry march with two x per lane (246 VGPRs: two waves per SIMD, so a
+// CU holds one block of 4 row waves + halo or two of 2 + halo; either way a round of blocks covers 1024 rows). A block
+// takes ZC + 1 layers, so the shape with the fewest rounds (ZC + 1) wins; 4 row waves repeat less of the halo, but pay only
+// over 16 planes or more and with a last round that is 3/4 full (a CU holds no second block of them). PCG pass, three loads (one load), 4 x 16 /
+// 4 x 32 / 2 x 8 / 2 x 4 row waves x planes: 96^3 78 / 74 / 81 / 82 (- / - / 39 / 36) us, 128^3 128 / 150 / 150 / -
+// (44 / - / 50 / -); the node march took 92 (41) and 160 (51) at its best shapes, 100 (42) and 161 (58) by its rule. The apply by this rule against the node march by
+// the old one, one / three / six loads: 66^3 22 / 48 / 92 against 27 / 58 / 111, 100^3 34 / 92 / 176 against
+// 43 / 111 / 217, 128^3 45 / 131 / 248 against 58 / 166 / 329 us.
+inline void pair64_shape(int ny, int nz, int L, int* W, int* ZC) {
+  int64_t best = -1;
+  for (int w : {4, 2, 1}) {
+    if (ny % w) continue;
+    const int64_t resident = 256 * (8 / (w + 1));
+    for (int z = 32; z >= 1; z /= 2) {
+      if (nz % z) continue;
+      const int64_t blocks = int64_t(ny / w) * (nz / z) * L, rounds = (blocks + resident - 1) / resident;
+      if (w == 4 && (z < 16 || 4 * (blocks - (rounds - 1) * resident) < 3 * resident)) continue;
+      const int64_t cost = rounds * (z + 1) * (w == 1 ? 4 : 3);  // one row wave per block repeats every row
+      if (best < 0 || cost < best) {
+        best = cost;
+        *W = w;
+        *ZC = z;
+      }
+    }
+  }
+}
+
 // Shape preferences (R, W, ZC) for L loads per launch. ZC (planes marched by
 // one block) is the largest of 16, 8, 4, 2, 1 dividing nz that still gives
 // at least 192 blocks: longer marches re-read fewer halo planes, but the
@@ -54,9 +81,12 @@ inline RowMarch rowmarch_config(const pgj_grid& g, int L, int es = 8) {
   c.nl = nx / c.xpl;
   // Default shape (measured on the PCG pass over 32^3..128^3, 1 and 6 loads):
   // the plane-carry march with two row waves (four for FP32 with one x per
-  // lane), except FP64 with two x per lane, which runs the node march.
+  // lane), except FP64 with two x per lane and voxels that are not cubes, whose
+  // plane-carry march would spill: that runs the node march.
+  const bool pair64 = es == 8 && c.xpl == 2 && g.hx == g.hy && g.hy == g.hz;
   int want_r = 1, want_w = (es == 4 && c.xpl == 1) ? 4 : 2, want_z = 0;
-  int want_plane = (es == 4 || c.xpl == 1) ? 1 : 0;
+  int want_plane = (es == 4 || c.xpl == 1 || pair64) ? 1 : 0;
+  if (pair64) pair64_shape(ny, nz, L, &want_w, &want_z);
   {
     int r = 0, w = 0, z = 0, p = 0;
     if (tuned_shape(g, L, es, &r, &w, &z, &p)) {
