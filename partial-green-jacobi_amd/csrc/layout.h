@@ -87,6 +87,17 @@ inline RowMarch rowmarch_config(const pgj_grid& g, int L, int es = 8) {
   int want_r = 1, want_w = (es == 4 && c.xpl == 1) ? 4 : 2, want_z = 0;
   int want_plane = (es == 4 || c.xpl == 1 || pair64) ? 1 : 0;
   if (pair64) pair64_shape(ny, nz, L, &want_w, &want_z);
+  // Launches of few blocks are one block's chain of layers long: one plane per block (two layers instead of three) while
+  // every block has a CU of its own, with the fewest row waves that allow it. FP64 stops at two row waves, whose four
+  // would only match the two-plane march. PCG pass by this rule against two planes: 16^3 one load 3.8 against 4.9 us,
+  // 20^3 4.2 / 4.9, 8^3 six loads 4.2 / 4.9; FP64 apply 16^3 3.4 / 4.3; FP32 apply 16^3 3.1 / 4.2, 32^3 3.6 / 4.3.
+  if (c.xpl == 1)
+    for (int w = 1; w <= (es == 8 ? 2 : 4); w *= 2)
+      if (ny % w == 0 && int64_t(ny / w) * nz * L <= 256) {
+        want_w = w;
+        want_z = 1;
+        break;
+      }
   {
     int r = 0, w = 0, z = 0, p = 0;
     if (tuned_shape(g, L, es, &r, &w, &z, &p)) {
