@@ -457,7 +457,7 @@ int pgj_pcg_post_step(int B, int64_t n, const double* r, double* z, const double
  * pgj_pcg_fi_ws_bytes, precond_ws: pgj_precond_ws_bytes(g, 1). */
 size_t pgj_pcg_fi_ws_bytes(const pgj_grid* g);
 int pgj_pcg_fi_iterate(const pgj_grid* g, const double* a, const void* plan, const double* sc, const void* s_hat,
-                       double* u, double* r, double* p, double* Ap, double* z, double* rz, const double* rhs_norm,
+                       double* u, double* r, double* p, double* Ap, double* rz, const double* rhs_norm,
                        double* best_u, double* best_res, double* res, uint8_t* improved, int64_t* state, double tol,
                        double near_tol, int64_t iteration, int count, int latched, double* ws, double* fi_ws,
                        void* precond_ws, void* stream);

@@ -410,7 +410,8 @@ __global__ __launch_bounds__(512) void fxyi_kernel(FFTArgs A) {
   // PCG: the displacement update u += alpha p of this iteration (alpha from the forward pass)
   const bool move = MODE == kFxyiPCG && A.p != nullptr && A.u != nullptr;
   const double alpha = move ? A.st.alpha[l] : 0.0;
-  const double* pp = A.p ? A.p + off : nullptr;
+  constexpr bool dir = MODE == kFxyiDir;
+  const double* pp = dir ? A.pdir + off : A.p ? A.p + off : nullptr;
   double* up = A.u ? A.u + off : nullptr;
   if (MODE == kFxyiPCG) {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
@@ -435,14 +436,17 @@ __global__ __launch_bounds__(512) void fxyi_kernel(FFTArgs A) {
   plane_twiddles(A, twx);
   // PCG: the output is the next direction p = z + beta p (z alone right after init)
   double mean = 0.0, beta = 0.0;
-  const bool update = MODE == kFxyiPCG && A.p != nullptr && !A.st.first[l];
+  const bool update = dir || (MODE == kFxyiPCG && A.p != nullptr && !A.st.first[l]);
   if (A.shat || update) {
     // one pass: r.z (offset 0) and this component's s.w partials (offset 1 + c)
     const int at[2] = {0, 1 + c};
     double sums[2];
     wave_reduce_partials_n<2>(A.pg + int64_t(l) * f.nkb * ny * 4, at, A.zslots, 4, sums);
     if (A.shat) mean = sums[1] / double(A.N);
-    if (update) {
+    if (dir) {
+      beta = sums[0] / fmax(*A.rz_old, 1e-30);
+      if (threadIdx.x == 0 && blockIdx.x == 0) *A.rz_out = sums[0];
+    } else if (update) {
       const double rz = A.st.rz[l];
       beta = sums[0] / (rz != 0.0 ? rz : 1.0);
     }
@@ -492,7 +496,7 @@ __global__ __launch_bounds__(512) void fxyi_kernel(FFTArgs A) {
   __syncthreads();
   // 4. unpack, scale and project; PCG: next direction and displacement update
   const double* sp = A.s ? A.s + soff : nullptr;
-  double* zp = A.zout + off;
+  double* zp = (dir ? A.pdir : A.zout) + off;
   const unsigned mx = f.mnx;
   for (int e0 = threadIdx.x; e0 < pn; e0 += kPlaneUnroll * T) {
     double vs[kPlaneUnroll], vp[kPlaneUnroll], vu[kPlaneUnroll];
@@ -825,18 +829,22 @@ extern "C" int pgj_scale_spectrum(const pgj_grid* g, const void* plan, const dou
   return launch_fz<kFzScale>(A, 1, st);
 }
 
-extern "C" int pgj_precond_apply(const pgj_grid* g, int L, const void* plan, const double* r, const double* s,
-                                 const void* s_hat, double* z, void* ws, void* stream) {
-  if (int e = check_fft(g)) return e;
-  PGJ_REQUIRE(L >= 1 && L <= 65535 && plan && r && z && ws, "invalid preconditioner arguments");
-  PGJ_REQUIRE((s == nullptr) == (s_hat == nullptr), "s and s_hat must be given together");
+namespace pgj {
+
+// z, or with `dir` (L = 1) the fields pdir, rz_old and rz_out of it.
+static int precond_passes(const pgj_grid* g, int L, const void* plan, const double* r, const double* s, const void* s_hat,
+                          double* z, const FFTArgs* dir, void* ws, hipStream_t st) {
   FFTArgs A = fft_args(*g, plan);
+  if (dir) {
+    A.pdir = dir->pdir;
+    A.rz_old = dir->rz_old;
+    A.rz_out = dir->rz_out;
+  }
   PrecondLayout pl = precond_layout(*g, L);
   if (static_fft(*g)) {
     // the compile-time passes read r and s and write z in their (L, 3N) node-interleaved layout; r is read by
     // the forward pass only, so z may alias it
     char* w = static_cast<char*>(ws);
-    hipStream_t st = as_stream(stream);
     A.rin = r;
     A.s = s;
     A.shat = static_cast<const double2*>(s_hat);
@@ -848,7 +856,7 @@ extern "C" int pgj_precond_apply(const pgj_grid* g, int L, const void* plan, con
     zpass_choose(A, *g, L);
     if (int e = launch_fxy_static(A, L, kFxyPre, st)) return e;
     if (int e = launch_fz_static(A, L, kFzPre, st)) return e;
-    return launch_fxyi_static(A, L, st, kFxyiPre);
+    return launch_fxyi_static(A, L, st, dir ? kFxyiDir : kFxyiPre);
   }
   char* w = static_cast<char*>(ws);
   A.rin = r;
@@ -859,8 +867,26 @@ extern "C" int pgj_precond_apply(const pgj_grid* g, int L, const void* plan, con
   A.pg = reinterpret_cast<double*>(w + pl.pg);
   A.zout = z;
   zpass_choose(A, *g, L);
-  hipStream_t st = as_stream(stream);
   if (int e = launch_fxy<kFxyPre>(A, L, st)) return e;
   if (int e = launch_fz<kFzPre>(A, L, st)) return e;
-  return launch_fxyi<kFxyiPre>(A, L, st);
+  return dir ? launch_fxyi<kFxyiDir>(A, L, st) : launch_fxyi<kFxyiPre>(A, L, st);
+}
+
+int precond_direction(const pgj_grid& g, const void* plan, const double* r, const double* s, const void* s_hat, double* p,
+                      const double* rz_old, double* rz, void* ws, hipStream_t stream) {
+  FFTArgs dir{};
+  dir.pdir = p;
+  dir.rz_old = rz_old;
+  dir.rz_out = rz;
+  return precond_passes(&g, 1, plan, r, s, s_hat, nullptr, &dir, ws, stream);
+}
+
+}  // namespace pgj
+
+extern "C" int pgj_precond_apply(const pgj_grid* g, int L, const void* plan, const double* r, const double* s,
+                                 const void* s_hat, double* z, void* ws, void* stream) {
+  if (int e = check_fft(g)) return e;
+  PGJ_REQUIRE(L >= 1 && L <= 65535 && plan && r && z && ws, "invalid preconditioner arguments");
+  PGJ_REQUIRE((s == nullptr) == (s_hat == nullptr), "s and s_hat must be given together");
+  return precond_passes(g, L, plan, r, s, s_hat, z, nullptr, ws, as_stream(stream));
 }

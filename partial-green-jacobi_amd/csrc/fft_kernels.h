@@ -9,7 +9,9 @@ namespace pgj {
 // ------------------------------------------------------------------ arguments
 enum { kFxyScale = 0, kFxyPre = 1, kFxyPCG = 2 };
 enum { kFzScale = 0, kFzPre = 1, kFzInit = 2, kFzPCG = 3 };
-enum { kFxyiPre = 0, kFxyiPCG = 1 };
+// kFxyiDir: the preconditioner apply that writes the next direction (FFTArgsT::pdir) in place of z, FP64 only. Its own
+// instances: the registers of the direction's loads cost the plain apply 5 % (64^3, one load 35.4 -> 37.1 us).
+enum { kFxyiPre = 0, kFxyiPCG = 1, kFxyiDir = 2 };
 
 // Arguments of the FFT/Green kernels; T is the vector precision (FP64 plain
 // path, FP32 inner solver of the mixed-precision form). Partial sums and the
@@ -45,9 +47,15 @@ struct FFTArgsT {
                          // workspace's z partials
   const double* rin64;   // FP32 preconditioner apply on AoS vectors: FP64 input residual, rounded to T on load
   double* zout64;        // ... and FP64 output z (exact widening of the T result); both null otherwise
+  double* pdir;          // FP64 preconditioner apply on AoS vectors: p = z + rz / max(rz_old, 1e-30) p takes the place
+  const double* rz_old;  // of z, rz (r.z of the z pass) goes to rz_out; one load, all null otherwise
+  double* rz_out;
 };
 using FFTArgs = FFTArgsT<double>;
 
+// r -> p = M^-1 r + beta p of one load (FFTArgsT::pdir); ws as for pgj_precond_apply.
+int precond_direction(const pgj_grid& g, const void* plan, const double* r, const double* s, const void* s_hat, double* p,
+                      const double* rz_old, double* rz, void* ws, hipStream_t stream);
 FFTArgs fft_args(const pgj_grid& g, const void* plan);
 int check_fft(const pgj_grid* g);
 int launch_fxy_mode(FFTArgs& A, int L, int mode, hipStream_t s);

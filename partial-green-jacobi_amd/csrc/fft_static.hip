@@ -734,7 +734,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(EU))) void f
 }
 
 // --------------------------------------------------------------- inverse xy
-// MODE kFxyiPre: the preconditioner apply alone (z = P(s w), no PCG state).
+// MODE kFxyiPre: the preconditioner apply alone (z = P(s w), no PCG state); kFxyiDir: p = z + beta p in its place.
 template <int N, int MODE, typename R, int PLAN = 0>
 __global__ __launch_bounds__(Cube<N>::TXY) __attribute__((amdgpu_waves_per_eu(Cube<N>::template occ_xy<R>())))
 void fxyi_static(FFTArgsT<R> A) {
@@ -779,7 +779,9 @@ void fxyi_static(FFTArgsT<R> A) {
   // per-load partials are laid out with the geometry's chunk count (slices of a set are offset by it)
   const double* pgl = A.pg + int64_t(l) * A.f.nkb * N * 4;
   // the output is the next direction p = z + beta p (z alone right after init or without a direction input)
-  const bool update = PCG && A.p != nullptr && !A.st.first[l];
+  // (dir: the preconditioner apply that writes the direction in the drop-in layout)
+  constexpr bool dir = MODE == kFxyiDir;
+  const bool update = dir || (PCG && A.p != nullptr && !A.st.first[l]);
   double mean = 0.0, beta = 0.0;
   if (A.shat || update) {
     // one pass: r.z (offset 0) and this component's s.w (offset 1 + c) partials
@@ -796,7 +798,10 @@ void fxyi_static(FFTArgsT<R> A) {
       wave_reduce_partials_n<2>(pgl, off, NSLOT, 4, sums);
     }
     if (A.shat) mean = sums[1] / double(NN);
-    if (update) {
+    if (dir) {
+      beta = sums[0] / fmax(*A.rz_old, 1e-30);
+      if (threadIdx.x == 0 && z == 0 && c == 0) *A.rz_out = sums[0];
+    } else if (update) {
       const double rz = A.st.rz[l];
       beta = sums[0] / (rz != 0.0 ? rz : 1.0);
     }
@@ -816,10 +821,11 @@ void fxyi_static(FFTArgsT<R> A) {
   X* __restrict__ zp = reinterpret_cast<X*>(A.zout + off);
   const bool scaled = A.s != nullptr;
   // the preconditioner pass also reads s and writes z in the drop-in layout (A.soa == 0): xyz triples per node
-  const bool aos = MODE == kFxyiPre && !A.soa;
+  const bool aos = !PCG && !A.soa;
   const int64_t aoff = int64_t(z) * C::PLANE * 3 + c;
   const R* __restrict__ s_aos = aos && scaled ? A.s + int64_t(design_of(l, A.group)) * 3 * NN + aoff : nullptr;
-  R* __restrict__ z_aos = aos && A.zout ? A.zout + int64_t(l) * 3 * NN + aoff : nullptr;
+  R* __restrict__ out_aos = dir ? reinterpret_cast<R*>(A.pdir) : A.zout;
+  R* __restrict__ z_aos = aos && out_aos ? out_aos + int64_t(l) * 3 * NN + aoff : nullptr;
   // FP32 apply of FP64 vectors: z is written in FP64
   double* __restrict__ z64 = sizeof(R) == 4 && aos && A.zout64 ? A.zout64 + int64_t(l) * 3 * NN + aoff : nullptr;
   const R m = R(mean), tb = R(beta);
@@ -843,7 +849,13 @@ void fxyi_static(FFTArgsT<R> A) {
         }
       }
     }
-    if (update || move) {
+    if (dir) {
+#pragma unroll
+      for (int i = 0; i < C::CH; ++i) {
+        const R* q = z_aos + 6 * int64_t(pair_of<N>(i0 + i < C::ITER ? i0 + i : C::ITER - 1));
+        vp[i] = c2(q[0], q[3]);
+      }
+    } else if (update || move) {
 #pragma unroll
       for (int i = 0; i < C::CH; ++i) vp[i] = pp[pair_of<N>(i0 + i < C::ITER ? i0 + i : C::ITER - 1)];
     }
@@ -1077,6 +1089,14 @@ template <int N, typename R>
 int fxyi_static_n(FFTArgsT<R>& A, int L, int mode, hipStream_t s) {
   using C = Cube<N>;
   const size_t lds = C::lds_xy(sizeof(cplx<R>));
+  if constexpr (sizeof(R) == 8) {
+    if (mode == kFxyiDir) {
+      if (int e = allow_lds_static(fxyi_static<N, kFxyiDir, R, default_plan<N>()>, lds)) return e;
+      hipLaunchKernelGGL((fxyi_static<N, kFxyiDir, R, default_plan<N>()>), dim3(N, 3, L), dim3(C::TXY), lds, s, A);
+      PGJ_LAUNCHED("fxyi_static");
+      return PGJ_OK;
+    }
+  }
   if (mode == kFxyiPre) {
     if (int e = allow_lds_static(fxyi_static<N, kFxyiPre, R, default_plan<N>()>, lds)) return e;
     hipLaunchKernelGGL((fxyi_static<N, kFxyiPre, R, default_plan<N>()>), dim3(N, 3, L), dim3(C::TXY), lds, s, A);

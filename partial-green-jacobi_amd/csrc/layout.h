@@ -273,13 +273,23 @@ inline bool stages_fit(const Factors& f, int lines, int threads) {
 
 constexpr int kMinChunk = 4;  // frequency columns per block of the runtime z pass: 4, 8 or 16
 
+// Rows of z pass partials per load are partial_chunks(g) ny: as many as any z pass of the grid has blocks (the compile-time
+// ones: fft_static.hip, ZWidths and ZReg; the runtime one at most ceil(ny nkx / kMinChunk)).
+inline int partial_chunks(const pgj_grid& g) {
+  int kc = kMinChunk;
+  if (static_cube(g)) kc = g.nx == 16 ? 3 : g.nx == 96 ? 6 : g.nx == 128 ? 5 : 4;
+  return (g.nx / 2 + 1 + kc - 1) / kc;
+}
+
+inline int64_t half_spectrum(const pgj_grid& g) { return int64_t(g.nz) * g.ny * (g.nx / 2 + 1); }
+
 inline FFTGeom fft_geom(const pgj_grid& g) {
   FFTGeom f{};
   f.nz = g.nz; f.ny = g.ny; f.nx = g.nx;
   f.nkx = g.nx / 2 + 1;
   f.M = (g.nx % 2 == 0) ? g.nx / 2 : g.nx;
   f.rs = f.nkx > f.M ? f.nkx : f.M;
-  f.nf = int64_t(g.nz) * g.ny * f.nkx;
+  f.nf = half_spectrum(g);
   const Factors fx = factorize(f.M), fy = factorize(g.ny), fz = factorize(g.nz);
   f.valid = fx.count >= 0 && fy.count >= 0 && fz.count >= 0 && g.nx >= 2 && g.ny >= 2 && g.nz >= 2 &&
             g.nx <= kMaxAxis && g.ny <= kMaxAxis && g.nz <= kMaxAxis;
@@ -298,19 +308,7 @@ inline FFTGeom fft_geom(const pgj_grid& g) {
   f.px = axis_plan(f.M);
   f.py = axis_plan(g.ny);
   f.pz = axis_plan(g.nz);
-  if (static_cube(g)) {
-    // at least as many rows of per-block partials (nkb n) as any of the compile-time z passes has blocks
-    // (fft_static.hip, ZWidths and ZReg)
-    switch (g.nx) {
-      case 16: kc = 3; break;
-      case 96: kc = 6; break;
-      case 128: kc = 5; break;
-      default: kc = 4; break;
-    }
-  } else {
-    kc = kMinChunk;  // the runtime z pass has at most ceil(ny nkx / kMinChunk) blocks per load
-  }
-  f.nkb = (f.nkx + kc - 1) / kc;
+  f.nkb = partial_chunks(g);
   f.runtime_ok = f.valid;
   if (static_cube(g)) f.valid = 1;
   return f;
@@ -323,13 +321,12 @@ struct PlanLayout {
 };
 
 inline PlanLayout plan_layout(const pgj_grid& g, size_t rs = 8) {
-  FFTGeom f = fft_geom(g);
   PlanLayout p{};
   size_t off = 0;
   p.tw_x = off; off = align256(off + size_t(g.nx) * 2 * rs);
   p.tw_y = off; off = align256(off + size_t(g.ny) * 2 * rs);
   p.tw_z = off; off = align256(off + size_t(g.nz) * 2 * rs);
-  p.sym = off; off = align256(off + size_t(6) * f.nf * rs);
+  p.sym = off; off = align256(off + size_t(6) * half_spectrum(g) * rs);
   p.bytes = off;
   return p;
 }
@@ -343,12 +340,11 @@ struct PrecondLayout {
 };
 
 inline PrecondLayout precond_layout(const pgj_grid& g, int L, size_t cs = 16) {
-  FFTGeom f = fft_geom(g);
   PrecondLayout p{};
   size_t off = 0;
-  p.spec = off; off = align256(off + size_t(L) * 3 * f.nf * cs);
+  p.spec = off; off = align256(off + size_t(L) * 3 * half_spectrum(g) * cs);
   p.pr = off; off = align256(off + size_t(L) * g.nz * 6 * 8);
-  p.pg = off; off = align256(off + size_t(L) * f.nkb * g.ny * 4 * 8);
+  p.pg = off; off = align256(off + size_t(L) * partial_chunks(g) * g.ny * 4 * 8);
   p.bytes = off;
   return p;
 }

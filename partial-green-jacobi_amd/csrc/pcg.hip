@@ -89,7 +89,7 @@ __global__ void pcg_reduce(int B, const double* part, int nblk, double* out) {
 // alpha = rz / max(pAp, eps), 0 where pAp is not finite or <= 0; u += alpha p;
 // r -= alpha Ap; rr_part = partial |r|^2 of the updated residual. The best residuals and the stop iteration so far go
 // to `best_old` and `stop_old` for pcg_best, whose blocks read them while others already write the new ones; rz goes to
-// `rz_old` likewise, for pcg_update_p where no pcg_dot precedes it.
+// `rz_old` likewise, for the steps of pgj_pcg_fi_iterate.
 template <typename T>
 __global__ __launch_bounds__(kVecThreads) void pcg_update_ur(T* u, T* r, const T* p, const T* Ap, int64_t n,
                                                              const double* pap_part, int nblk, const double* rz,
@@ -167,9 +167,9 @@ __global__ __launch_bounds__(kVecThreads) void pcg_best(const T* u, T* best_u, i
 // beta = rz_new / max(rz_old, eps); p = z + beta p; rz = rz_new.
 template <typename T>
 __global__ __launch_bounds__(kVecThreads) void pcg_update_p(const T* z, T* p, int64_t n, const double* rz_part,
-                                                            int nblk, int stride, const double* rz_old, double* rz) {
+                                                            int nblk, const double* rz_old, double* rz) {
   const int b = blockIdx.y;
-  const double rzn = wave_reduce_partials(rz_part + int64_t(b) * nblk * stride, nblk, stride);
+  const double rzn = wave_reduce_partials(rz_part + int64_t(b) * nblk, nblk, 1);
   const T beta = T(rzn / fmax(rz_old[b], kPcgEps));
   if (blockIdx.x == 0 && threadIdx.x == 0) rz[b] = rzn;
   const int64_t off = int64_t(b) * n;
@@ -280,7 +280,7 @@ int pcg_post_step_t(int B, int64_t n, const T* r, T* z, const T* minv, int64_t m
   hipLaunchKernelGGL(pcg_dot<T>, dim3(nblk, B), dim3(kVecThreads), 0, s, r, z, minv, z, n, minv_stride, part, rz,
                      rz_old);
   PGJ_LAUNCHED("pcg_dot");
-  hipLaunchKernelGGL(pcg_update_p<T>, dim3(nblk, B), dim3(kVecThreads), 0, s, z, p, n, part, nblk, 1, rz_old, rz);
+  hipLaunchKernelGGL(pcg_update_p<T>, dim3(nblk, B), dim3(kVecThreads), 0, s, z, p, n, part, nblk, rz_old, rz);
   PGJ_LAUNCHED("pcg_update_p");
   return PGJ_OK;
 }
@@ -333,21 +333,22 @@ extern "C" int pgj_pcg32_post_step(int B, int64_t n, const float* r, float* z, c
 }
 
 // One load of the scalar operator with its Green preconditioner: what pgj_precond_apply, pgj_pcg_post_step, pgj_hex8_apply
-// and pgj_pcg_pre_step do, `count` times, from one call. p.Ap comes from the apply's own blocks and r.z from the z pass of
-// the preconditioner (Parseval), so seven launches an iteration take the place of nine, and no host work lies between
-// them: at 32^3 the loop over four entry points was bound by the host, 76 us an iteration for 45 us of kernels.
+// and pgj_pcg_pre_step do, `count` times, from one call. p.Ap comes from the apply's own blocks, r.z from the z pass of
+// the preconditioner (Parseval), and the inverse pass writes p in place of z: six launches an iteration instead of nine,
+// with no host work between them. At 32^3 the loop over four entry points was bound by the host, 73 us an iteration for
+// 45 us of kernels; now 43.
 extern "C" size_t pgj_pcg_fi_ws_bytes(const pgj_grid* g) {
   return g ? align256(size_t(hex8_blocks_bound(*g)) * 8) : 0;
 }
 
 extern "C" int pgj_pcg_fi_iterate(const pgj_grid* g, const double* a, const void* plan, const double* sc,
-                                  const void* s_hat, double* u, double* r, double* p, double* Ap, double* z, double* rz,
+                                  const void* s_hat, double* u, double* r, double* p, double* Ap, double* rz,
                                   const double* rhs_norm, double* best_u, double* best_res, double* res,
                                   uint8_t* improved, int64_t* state, double tol, double near_tol, int64_t iteration,
                                   int count, int latched, double* ws, double* fi_ws, void* precond_ws, void* stream) {
   if (int e = check_grid(g)) return e;
   if (int e = check_fft(g)) return e;
-  PGJ_REQUIRE(a && plan && u && r && p && Ap && z && rz && rhs_norm && best_u && best_res && res && improved && state &&
+  PGJ_REQUIRE(a && plan && u && r && p && Ap && rz && rhs_norm && best_u && best_res && res && improved && state &&
                   ws && fi_ws && precond_ws && count >= 0 && (sc == nullptr) == (s_hat == nullptr),
               "invalid pcg iterate arguments");
   hipStream_t s = as_stream(stream);
@@ -356,22 +357,16 @@ extern "C" int pgj_pcg_fi_iterate(const pgj_grid* g, const double* a, const void
   const PcgWs w = pcg_ws(1, n);
   double *rr = ws + w.rr, *best_old = ws + w.best_old, *rz_old = ws + w.rz_old;
   int64_t* stop_old = reinterpret_cast<int64_t*>(ws + w.stop_old);
-  // the partials of r.z as the preconditioner's z pass leaves them
-  FFTArgs F = fft_args(*g, plan);
-  zpass_choose(F, *g, 1);
-  const double* rz_part = reinterpret_cast<const double*>(static_cast<char*>(precond_ws) + precond_layout(*g, 1).pg);
   const bool march = rowmarch_config(*g, 1).valid;
   for (int k = 0; k < count; ++k) {
-    if (int e = pgj_precond_apply(g, 1, plan, r, sc, s_hat, z, precond_ws, stream)) return e;
-    hipLaunchKernelGGL(pcg_update_p<double>, dim3(nblk, 1), dim3(kVecThreads), 0, s, z, p, n, rz_part, F.zslots, 4,
-                       rz_old, rz);
-    PGJ_LAUNCHED("pcg_update_p");
+    if (int e = precond_direction(*g, plan, r, sc, s_hat, p, rz_old, rz, precond_ws, s)) return e;
     const double* pap = fi_ws;
-    int pblk = hex8_blocks_per_load(*g, 1);
+    int pblk;
     if (march) {
       RowArgs A{};
-      A.a = a; A.u = p; A.out = Ap; A.ppq = fi_ws; A.ppq_stride = pblk;
+      A.a = a; A.u = p; A.out = Ap; A.ppq = fi_ws;
       if (int e = launch_rowmarch(*g, 1, kModeApplyDot, A, s)) return e;
+      pblk = A.cfg.by * A.cfg.bz;  // of the launch itself: a tuner may set another shape meanwhile
     } else {
       if (int e = pgj_hex8_apply(g, 1, a, p, nullptr, Ap, stream)) return e;
       pap = ws + w.pap;

@@ -74,13 +74,12 @@ template <typename T = double>
 ResidentBuffersT<T> resident_buffers(const pgj_grid& g, int L, void* ws, int l0 = 0) {
   ResidentBuffersT<T> b{};
   b.lay = resident_layout(g, L, sizeof(cplx<T>));
-  const FFTGeom f = fft_geom(g);
   char* w = static_cast<char*>(ws);
   b.ppq = reinterpret_cast<double*>(w + b.lay.ppq) + int64_t(l0) * hex8_blocks_bound(g);
   b.pcert = reinterpret_cast<double*>(w + b.lay.pcert) + int64_t(l0) * b.lay.nblk_cert * 4;
-  b.spec = reinterpret_cast<cplx<T>*>(w + b.lay.pre.spec) + int64_t(l0) * 3 * f.nf;
+  b.spec = reinterpret_cast<cplx<T>*>(w + b.lay.pre.spec) + int64_t(l0) * 3 * half_spectrum(g);
   b.pr = reinterpret_cast<double*>(w + b.lay.pre.pr) + int64_t(l0) * g.nz * 6;
-  b.pg = reinterpret_cast<double*>(w + b.lay.pre.pg) + int64_t(l0) * f.nkb * g.ny * 4;
+  b.pg = reinterpret_cast<double*>(w + b.lay.pre.pg) + int64_t(l0) * partial_chunks(g) * g.ny * 4;
   b.rscale = reinterpret_cast<double*>(w + b.lay.rscale) + l0;
   return b;
 }

@@ -150,7 +150,7 @@ SIGNATURES = {
     'pgj_pcg_post_step': (c_int, [c_int, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p,
                                   c_void_p, c_void_p]),
     'pgj_pcg_fi_ws_bytes': (c_size_t, [GP]),
-    'pgj_pcg_fi_iterate': (c_int, [GP] + [c_void_p] * 16 + [c_double, c_double, c_int64, c_int, c_int] + [c_void_p] * 4),
+    'pgj_pcg_fi_iterate': (c_int, [GP] + [c_void_p] * 15 + [c_double, c_double, c_int64, c_int, c_int] + [c_void_p] * 4),
     'pgj_pcg32_start': (c_int, [c_int, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     'pgj_pcg32_init': (c_int, [c_int, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     'pgj_pcg32_pre_step': (c_int, [c_int, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,

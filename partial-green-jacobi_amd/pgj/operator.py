@@ -250,13 +250,12 @@ class Operator:
         if type(self) is not Operator or self.dtype != torch.float64 or type(precond) is not AttachedGreen \
                 or precond.op is not self or any(name in own for name in ('apply', 'green_precond', '_apply_call')):
             return None
-        z = torch.empty_like(r)
         fi_ws = torch.empty(_lib.lib().pgj_pcg_fi_ws_bytes(self.grid) // 8, dtype=torch.float64, device=self.device)
 
         def steps(iteration, count):
             s, shat = precond.fields()
             _lib.call('pgj_pcg_fi_iterate', self.grid, _lib.ptr(self._material_field), _lib.ptr(self._plan),
-                      _lib.ptr(s), _lib.ptr(shat), _lib.ptr(u), _lib.ptr(r), _lib.ptr(p), _lib.ptr(ap), _lib.ptr(z),
+                      _lib.ptr(s), _lib.ptr(shat), _lib.ptr(u), _lib.ptr(r), _lib.ptr(p), _lib.ptr(ap),
                       _lib.ptr(work.rz), _lib.ptr(work.rhs_norm), _lib.ptr(best_u), _lib.ptr(work.best_res),
                       _lib.ptr(work.res), _lib.ptr(work.improved), _lib.ptr(work.state), float(tol), float(near_tol),
                       iteration, count, int(latched), _lib.ptr(work.ws), _lib.ptr(fi_ws),
