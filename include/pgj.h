@@ -426,7 +426,7 @@ int pgj_gauss_rounds(int n, const double* x, const double* ratio, const double* 
  * (solver/src/runtime/fi/source/femlib/batched/pcg.py:20-245): the fused
  * compiled steps (pcg.py:622-666, :741-745), the convergence latches
  * (pcg.py:677-712), the latched best copy (pcg.py:715-738) and the Triton/CUDA Jacobi vector
- * kernels (pcg.py:459-532). ws holds 3 B ceil(n/1024)-capped partial rows. */
+ * kernels (pcg.py:459-532). ws holds 3 B rows of at most 1024 partials. */
 size_t pgj_pcg_ws_bytes(int B, int64_t n);
 /* r = rhs - Ax (Ax NULL: r = rhs) and rhs_norm = max(|rhs_b|, 1e-30) (pcg.py:79-85). */
 int pgj_pcg_start(int B, int64_t n, const double* rhs, const double* Ax, double* r, double* rhs_norm, double* ws,

@@ -17,13 +17,16 @@ namespace pgj {
 constexpr int kVecThreads = 256;
 constexpr double kPcgEps = 1e-30;  // pcg.py:112 (eps clamp of pAp and rz)
 
+// One value per thread up to 256 K values: a pass over a small vector is one round trip to memory, and every further value
+// of a thread would add its own (four values: certified solve 32^3 3.17 ms, one: 3.10; generic composite C^H 48^3
+// 16.7 and 16.2 ms).
 inline int vec_blocks(int64_t n) {
-  const int64_t b = (n + kVecThreads * 4 - 1) / (kVecThreads * 4);
+  const int64_t b = (n + kVecThreads - 1) / kVecThreads;
   return int(b < 1024 ? b : 1024);
 }
 
 #define PGJ_GRID_LOOP(i, n) \
-  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < (n); i += int64_t(gridDim.x) * blockDim.x)
+  _Pragma("unroll 4") for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < (n); i += int64_t(gridDim.x) * blockDim.x)
 
 // r = rhs - Ax (Ax may be null: r = rhs); rhs_part[b][blk] = partial |rhs_b|^2.
 // Vectors are T (FP64 or FP32); sums, partials and per-batch scalars are FP64.
@@ -91,7 +94,9 @@ __global__ void pcg_reduce(int B, const double* part, int nblk, double* out) {
 // to `best_old` and `stop_old` for pcg_best, whose blocks read them while others already write the new ones; rz goes to
 // `rz_old` likewise, for the steps of pgj_pcg_fi_iterate.
 template <typename T>
-__global__ __launch_bounds__(kVecThreads) void pcg_update_ur(T* u, T* r, const T* p, const T* Ap, int64_t n,
+__global__ __launch_bounds__(kVecThreads) void pcg_update_ur(T* __restrict__ u, T* __restrict__ r,
+                                                             const T* __restrict__ p,
+                                                             const T* __restrict__ Ap, int64_t n,
                                                              const double* pap_part, int nblk, const double* rz,
                                                              double* rr_part, const double* best_res,
                                                              const int64_t* state, double* best_old,
@@ -131,7 +136,8 @@ __global__ __launch_bounds__(kVecThreads) void pcg_update_ur(T* u, T* r, const T
 // forms its batch's residual from the partials (at most 1024, one pass of a wavefront), which costs it less than the
 // launch of its own that this test took before the copy: 2.9 of 24 us of vector kernels an iteration at 32^3.
 template <typename T>
-__global__ __launch_bounds__(kVecThreads) void pcg_best(const T* u, T* best_u, int64_t n, int B, const double* rr_part,
+__global__ __launch_bounds__(kVecThreads) void pcg_best(const T* __restrict__ u, T* __restrict__ best_u,
+                                                        int64_t n, int B, const double* rr_part,
                                                         int nblk, const double* rhs_norm, const double* best_old,
                                                         const int64_t* stop_old, double* res, double* best_res,
                                                         uint8_t* improved, int64_t* state, double tol, double near_tol,
@@ -166,7 +172,7 @@ __global__ __launch_bounds__(kVecThreads) void pcg_best(const T* u, T* best_u, i
 
 // beta = rz_new / max(rz_old, eps); p = z + beta p; rz = rz_new.
 template <typename T>
-__global__ __launch_bounds__(kVecThreads) void pcg_update_p(const T* z, T* p, int64_t n, const double* rz_part,
+__global__ __launch_bounds__(kVecThreads) void pcg_update_p(const T* __restrict__ z, T* __restrict__ p, int64_t n, const double* rz_part,
                                                             int nblk, const double* rz_old, double* rz) {
   const int b = blockIdx.y;
   const double rzn = wave_reduce_partials(rz_part + int64_t(b) * nblk, nblk, 1);
