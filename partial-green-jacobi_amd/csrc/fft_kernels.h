@@ -43,8 +43,10 @@ struct FFTArgsT {
   int soa;               // vectors (and s) are SoA (L, 3, N) instead of AoS (L, N, 3)
   int group;             // loads per design (s is (designs, 3N), s_hat (designs, 3, nf)); 0: shared
   int zkc, zslots;       // columns per block of the z pass (0: register-resident cubes) and its partial rows per
-                         // load, set by zpass_choose; the same for every launch that writes or reads one
-                         // workspace's z partials
+                         // load, set by zpass_choose. The form follows the radix plan in force at the launch, so in
+                         // the PCG modes of the compile-time cubes the passes that sum the rows take their number
+                         // from StateView::zrows, where the z pass that wrote them left it: a plan set between the
+                         // two (an eager initialization and a captured iteration) changes speed only
   const double* rin64;   // FP32 preconditioner apply on AoS vectors: FP64 input residual, rounded to T on load
   double* zout64;        // ... and FP64 output z (exact widening of the T result); both null otherwise
   double* pdir;          // FP64 preconditioner apply on AoS vectors: p = z + rz / max(rz_old, 1e-30) p takes the place

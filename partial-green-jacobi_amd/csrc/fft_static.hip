@@ -174,6 +174,8 @@ void fxy_static(FFTArgsT<R> A) {
     const R* q = base + 6 * int64_t(h);
     return c2(q[0], q[3]);
   };
+  // rows of z partials to sum: as many as the pass that wrote them left, whatever form a pass launched now would take
+  const int zrows = MODE == kFxyPCG ? A.st.zrows[l] : 0;
   double alpha = 0.0;
 #pragma unroll
   for (int i0 = 0; i0 < C::ITER; i0 += C::CH) {
@@ -208,12 +210,12 @@ void fxy_static(FFTArgsT<R> A) {
       if (C::SHARED_SUMS) {
         double t[2] = {0.0, 0.0};
         for (int k = threadIdx.x; k < A.ppq_count; k += T) t[0] += ppq[k];
-        for (int k = threadIdx.x; k < A.zslots; k += T) t[1] += pg[4 * k];
+        for (int k = threadIdx.x; k < zrows; k += T) t[1] += pg[4 * k];
         block_sums<2>(t, red);
         pq = t[0];
         rz = t[1];
       } else {
-        wave_reduce_partials_2(ppq, A.ppq_count, 1, pg, A.zslots, 4, pq, rz);
+        wave_reduce_partials_2(ppq, A.ppq_count, 1, pg, zrows, 4, pq, rz);
       }
       const bool valid = isfinite(pq) && pq > 0.0 && isfinite(rz) && rz > 0.0;
       alpha = valid ? rz / pq : 0.0;
@@ -364,6 +366,7 @@ void fz_static(FFTArgsT<R> A) {
         A.st.bad_next[l] = A.st.bad[l];
         A.st.first[l] = 1;
         A.st.stopped[l] = 0;
+        A.st.zrows[l] = Z::BLOCKS;
       }
     } else {
       const bool active = A.st.active[l] != 0;
@@ -376,6 +379,7 @@ void fz_static(FFTArgsT<R> A) {
         A.st.it_next[l] = it;
         A.st.bad_next[l] = A.st.bad[l] || (active && !valid) || (active && !finite);
         A.st.stopped[l] = active && !act;
+        A.st.zrows[l] = Z::BLOCKS;
       }
     }
     if (!act) return;
@@ -590,6 +594,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(EU))) void f
         A.st.bad_next[l] = bad || (MODE == kFzPCG && !(valid && finite));
         A.st.stopped[l] = MODE == kFzPCG && !act;
         if (MODE == kFzInit) A.st.first[l] = 1;
+        A.st.zrows[l] = Z::BLOCKS;
       }
       if (!act) return;
     }
@@ -775,7 +780,7 @@ void fxyi_static(FFTArgsT<R> A) {
   in.load(spec + (int64_t(c) * N + z) * (N * C::M), [](int e) { return e; });
   nyq.load(spec + Spec<N>::MAIN + (int64_t(c) * N + z) * N, [](int e) { return e; });
   twl.load(A.twy, [](int e) { return e; });
-  const int NSLOT = A.zslots;
+  const int NSLOT = PCG ? A.st.zrows[l] : A.zslots;
   // per-load partials are laid out with the geometry's chunk count (slices of a set are offset by it)
   const double* pgl = A.pg + int64_t(l) * A.f.nkb * N * 4;
   // the output is the next direction p = z + beta p (z alone right after init or without a direction input)

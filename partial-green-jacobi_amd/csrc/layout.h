@@ -379,7 +379,7 @@ constexpr int kMaxResidentLoads = 4096;
 // Resident state: public blocks first (documented in pgj.h), then private.
 struct StateLayout {
   size_t rz, target2, norm, absolute, it, active, bad;
-  size_t it_next, active_next, bad_next, first, alpha, stopped, valid, cap;
+  size_t it_next, active_next, bad_next, first, alpha, stopped, valid, cap, zrows;
   size_t bytes;
 };
 
@@ -401,6 +401,7 @@ inline StateLayout state_layout(int L) {
   s.stopped = off; off += align8(size_t(L));
   s.valid = off; off += align8(size_t(L));
   s.cap = off; off += align8(size_t(L) * 8);
+  s.zrows = off; off += align8(size_t(L) * 4);
   s.bytes = align256(off);
   return s;
 }
@@ -422,6 +423,7 @@ struct StateView {
   uint8_t* stopped;   // active at the start of this iteration and stopped by its test
   uint8_t* valid;     // this iteration's p.q and r.z were finite and positive (forward pass)
   int64_t* cap;       // iteration cap of the load (set by the set-up)
+  int32_t* zrows;     // partial rows the load's last z pass wrote (compile-time cubes)
 };
 
 // View of loads [l0, ...) of a state block laid out for L loads.
@@ -444,6 +446,7 @@ inline StateView state_view(void* base, int L, int l0 = 0) {
   v.stopped = reinterpret_cast<uint8_t*>(b + s.stopped) + l0;
   v.valid = reinterpret_cast<uint8_t*>(b + s.valid) + l0;
   v.cap = reinterpret_cast<int64_t*>(b + s.cap) + l0;
+  v.zrows = reinterpret_cast<int32_t*>(b + s.zrows) + l0;
   return v;
 }
 
