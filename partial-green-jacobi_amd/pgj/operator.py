@@ -244,11 +244,14 @@ class Operator:
 
     def native_pcg_steps(self, work, u, r, p, ap, best_u, tol, near_tol, latched):
         """``steps(iteration, count)``: that many iterations of ``solve_pcg_batched`` in one library call, or None where
-        this operator's apply or preconditioner is not the one this class and ``set_alpha`` attach."""
+        this operator's apply or preconditioner is not the one this module and ``set_alpha`` attach: replaced on the
+        instance or on the class (a counting or profiling wrapper), it is called in every iteration."""
         own = self.__dict__
         precond = own.get('apply_precond')
         if type(self) is not Operator or self.dtype != torch.float64 or type(precond) is not AttachedGreen \
-                or precond.op is not self or any(name in own for name in ('apply', 'green_precond', '_apply_call')):
+                or precond.op is not self or any(name in own for name in _STEP_METHODS) \
+                or AttachedGreen.__call__ is not _ATTACHED_CALL \
+                or any(getattr(Operator, name) is not fn for name, fn in _STEP_METHODS.items()):
             return None
         fi_ws = torch.empty(_lib.lib().pgj_pcg_fi_ws_bytes(self.grid) // 8, dtype=torch.float64, device=self.device)
 
@@ -305,6 +308,12 @@ class AttachedGreen:
 
     def __call__(self, r):
         return self.op.green_precond(r, *self.fields())
+
+
+# what an iteration of solve_pcg_batched calls, as defined above
+_STEP_METHODS = {name: getattr(Operator, name) for name in ('apply', '_validate_apply_input', '_apply_call',
+                                                            'green_precond')}
+_ATTACHED_CALL = AttachedGreen.__call__
 
 
 def set_alpha(op, alpha):

@@ -186,7 +186,8 @@ def solve_pcg_batched(op, rhs, *, tol=1e-6, max_iter=2000, verbose=False, log_ev
     # an operator that knows this loop runs the iterations up to the next host check in one call
     steps = native = None
     if B == 1 and dt == torch.float64 and not jacobi and recycle is None and not verbose:
-        native = getattr(op, 'native_pcg_steps', None)
+        # (looked up on the class: a wrapper that hands other names on to an operator has its own apply)
+        native = getattr(type(op), 'native_pcg_steps', None)
 
     n_iter_final = max_iter
     it = 0
@@ -203,7 +204,7 @@ def solve_pcg_batched(op, rhs, *, tol=1e-6, max_iter=2000, verbose=False, log_ev
                 recycle(it, p.clone(), ap)
             work.pre_step(u, r, p, ap, best_u, tol, near_tol, it + 1, latched)
             if it == 0 and native is not None:
-                steps = native(work, u, r, p, torch.empty_like(ap), best_u, tol, near_tol, latched)
+                steps = native(op, work, u, r, p, torch.empty_like(ap), best_u, tol, near_tol, latched)
         else:
             count = min(host_check_stride - it % host_check_stride, max_iter - it)
             steps(it + 1, count)
