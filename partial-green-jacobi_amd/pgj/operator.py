@@ -307,7 +307,7 @@ class AttachedGreen:
         return (self.op._scale, self.op._scale_hat) if self.scaled else (None, None)
 
     def __call__(self, r):
-        return self.op.green_precond(r, *self.fields())
+        return self.op.green_precond(r, *self.fields()) if self.scaled else self.op.green_precond(r)
 
 
 # what an iteration of solve_pcg_batched calls, as defined above
