@@ -9,8 +9,33 @@ results and iteration counts equal those of the one-chunk-at-a-time loop.
 """
 import contextlib
 import gc
+import threading
 
 import torch
+
+
+class _CollectorHold:
+    """Keeps the cyclic garbage collector off while any thread is inside; the last one to leave restores it as the
+    first one found it (the collector has one switch for the whole process)."""
+
+    def __init__(self):
+        self.lock, self.depth, self.enabled = threading.Lock(), 0, False
+
+    def __enter__(self):
+        with self.lock:
+            if self.depth == 0:
+                self.enabled = gc.isenabled()
+                gc.disable()
+            self.depth += 1
+
+    def __exit__(self, *exc):
+        with self.lock:
+            self.depth -= 1
+            if self.depth == 0 and self.enabled:
+                gc.enable()
+
+
+_HOLD = _CollectorHold()
 
 
 @contextlib.contextmanager
@@ -19,14 +44,8 @@ def capturing(graph):
     in a reference cycle until the collector runs; if that happens between two launches of a capture, the destructors
     of its graphs and events call into the runtime, which an open capture refuses, and the exception they raise ends
     the process (seen as an abort with the collector on top of the stack of a capturing thread)."""
-    enabled = gc.isenabled()
-    gc.disable()
-    try:
-        with torch.cuda.graph(graph):
-            yield
-    finally:
-        if enabled:
-            gc.enable()
+    with _HOLD, torch.cuda.graph(graph):
+        yield
 
 
 class MaskPipeline:
