@@ -411,20 +411,27 @@ __global__ __launch_bounds__(MAXT) void hex8_rowmarch(RowArgsT<T> A) {
 }
 
 // The 24x24 element stiffness of C0 by its tensor-product form, independent of the modal form of the other kernels.
-// The integrals over the element factor into per-axis ones: stiffness (s s' / h), mass (h / 3 on equal, h / 6 on
-// different ends) and mixed (s / 2, whatever the other end), with s = -1 or +1 the node's end of the axis. So
-//   K_ii(n, m) = diag[i][n ^ m],  K_ij(n, m) = (lam s_i(n) s_j(m) + mu s_j(n) s_i(m)) off[k][bit k of n ^ m]
-// (i != j, k the third axis): 36 numbers, all held in scalar registers.
+// The integrals over the element factor into per-axis ones over two ends. With the displacements written as the node's
+// own value and differences along the axes to the other ends, each factor is one over both ends (`sum`) or one of the
+// other end alone: mass h / 2 and h / 6, stiffness 0 and -1 / h, derivative of the node's function s and s / 2, of the
+// other's 0 and -s / 2, with s = -1 or +1 the node's end. So K_ii and K_ij take, for the set of axes `o` along which a
+// quantity is a difference,
+//   diag[i][o],  -s_i s_j (lam [j in o] + mu [i in o]) / (2 or, with both, 4) mass_k   (i != j, k the third axis):
+// 39 numbers, all held in scalar registers. The node's own value (o empty) drops out exactly.
 struct RefStiffness {
   double diag[3][8];
-  double off_sum[3][2], off_diff[3][2];   // (lam + mu) and (lam - mu) times the mixed integral
+  double lam[3][2], mu[3][2], both[3][2];   // lam / 2, mu / 2 and (lam + mu) / 4 times the mass along k
 };
 
 // Certification apply. A thread owns the column of nodes (x, y) over ZC planes and marches them: it loads each plane's
-// 3 x 3 neighbours once and adds their 3x3 blocks to the forces of the four elements of the layer below (as its top
-// corners) and of the layer above (as its bottom corners) on the layer's two nodes of the column: 576 FMAs and 31 loads
-// per node, with nine fixed offsets per thread. The form before evaluated eight whole elements per node for 3 of their
-// 24 forces each, 2700 flops and 192 loads: 64^3, six loads, 205 us against 75, 128^3 1590 against 430.
+// 3 x 3 neighbours once, turns them into differences from the column's node, and adds their terms to the forces of the
+// four elements of the layer below and of the layer above on the layer's two nodes of the column: 456 FMAs and 31 loads
+// per node, with nine fixed offsets per thread. Bound by FP64 issue at two waves per SIMD. One load at 64^3 15 us, six 57,
+// 128^3 six 383; eight whole elements evaluated per node for 3 of their 24 forces each took 39, 195 and 1562.
+// The differences also keep the digits: products with whole displacements (17, 62 and 388 us) cancel the rigid part only
+// in the rounded sum. Relative error on a smooth field plus an offset of 0 and 3, at 32^3: 9.8e-16 and 9.7e-14, of the
+// modal row march 6.6e-16 and 5.2e-14, here 2.6e-16 and 2.5e-16; at 9 x 5 x 64 1.2e-15 and 9.4e-14, 2.8e-16 and 8.0e-15,
+// 2.7e-16 and 2.7e-16.
 // I: unsigned where the byte offsets of a vector fit 32 bits (uniform base + 32-bit offset), else int64_t.
 template <bool CERT, typename I>
 __global__ __launch_bounds__(256) void hex8_reference(RefArgs A, RefStiffness K, int ZC) {
@@ -443,36 +450,38 @@ __global__ __launch_bounds__(256) void hex8_reference(RefArgs A, RefStiffness K,
     const double* __restrict__ rhs = CERT ? A.rhs + int64_t(l) * 3 * A.N : nullptr;
     double* __restrict__ out = A.out + int64_t(l) * 3 * A.N;
     const I cs = A.soa ? I(A.N) : I(1), ns = A.soa ? I(1) : I(3);   // strides of components and nodes
-    double v[3][3][3];            // a plane's neighbours [y][x][component]
-    double bot[4][3], top[4][3];  // forces, for a = 1, of the layer's elements on its bottom and top node of the column
+    // a plane's values: the column's node, its differences to x - 1, x + 1, y - 1, y + 1, and the mixed differences of
+    // the four quadrants e (bit set: the minus side of the axis)
+    double q[9][3], zq[9][3];     // of this plane; of the plane below, then differences of the two
+    // forces, for a = 1, of the layer's elements on its bottom and top node of the column: the terms of single differences
+    // ([0], the largest) and of mixed ones ([1]) are summed apart, so that fewer sums round at the size of the force
+    double bot[2][4][3], top[2][4][3];
     double carry[3] = {0.0, 0.0, 0.0};
-    // contributions of the plane at the layer's z corner ZM to the layer's node at z corner ZN
-    auto add = [&](auto zm, auto zn, double (&f)[4][3]) {
-      constexpr int ZM = decltype(zm)::value, ZN = decltype(zn)::value;
+    // terms of the plane's values (SZ = 0) or of the differences along z (SZ = 1) on the layer's node at z corner ZN
+    auto add = [&](auto sz, auto zn, const double (&w)[9][3], double (&force)[2][4][3]) {
+      constexpr int SZ = decltype(sz)::value, ZN = decltype(zn)::value;
 #pragma unroll
-      for (int py = 0; py < 3; ++py)
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int px = 0; px < 3; ++px)
+        for (int sxy = 0; sxy < 4; ++sxy) {
+          if (SZ == 0 && sxy == 0) continue;
+          const int at = sxy == 0 ? 0 : sxy == 1 ? 2 - (e & 1) : sxy == 2 ? 4 - (e >> 1) : 5 + e;
+          const int o = sxy | SZ << 2, n = e | ZN << 2;   // n: the node is the corner of the element's bits
+          const bool flip = SZ == 1 && ZN == 1;           // the other end of the top node lies below
+          double (&f)[4][3] = force[(o & (o - 1)) != 0];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            // element e lies on the minus side of an axis where its bit is set; the node is its corner of those bits
-            const int ox = px - 1 + (e & 1), oy = py - 1 + (e >> 1);
-            if (ox < 0 || ox > 1 || oy < 0 || oy > 1) continue;
-            const int n = e | ZN << 2, m = ox | oy << 1 | ZM << 2, df = n ^ m;
+          for (int a = 0; a < 3; ++a) {
+            f[e][a] = fma(flip ? -K.diag[a][o] : K.diag[a][o], w[at][a], f[e][a]);
 #pragma unroll
-            for (int a = 0; a < 3; ++a) f[e][a] = fma(K.diag[a][df], v[py][px][a], f[e][a]);
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-              // the two axes (a, b) other than k; K_ab = lam s_a(n) s_b(m) + mu s_b(n) s_a(m): equal signs or opposite
-              const int a = (k + 1) % 3, b = (k + 2) % 3, kb = (df >> k) & 1;
-              const bool p = ((n >> a) & 1) == ((m >> b) & 1), q = ((n >> b) & 1) == ((m >> a) & 1);
-              const double same = p ? K.off_sum[k][kb] : -K.off_sum[k][kb];
-              const double kab = p == q ? same : (p ? K.off_diff[k][kb] : -K.off_diff[k][kb]);
-              const double kba = p == q ? same : (q ? K.off_diff[k][kb] : -K.off_diff[k][kb]);
-              f[e][a] = fma(kab, v[py][px][b], f[e][a]);
-              f[e][b] = fma(kba, v[py][px][a], f[e][b]);
+            for (int b = 0; b < 3; ++b) {
+              const int k = 3 - a - b;
+              if (b == a || !((o >> a | o >> b) & 1)) continue;
+              const int m = (o >> k) & 1;
+              const double c = !((o >> a) & 1) ? K.lam[k][m] : !((o >> b) & 1) ? K.mu[k][m] : K.both[k][m];
+              f[e][a] = fma((((n >> a ^ n >> b) & 1) != 0) != flip ? c : -c, w[at][b], f[e][a]);
             }
           }
+        }
     };
     using Z0 = std::integral_constant<int, 0>;
     using Z1 = std::integral_constant<int, 1>;
@@ -489,19 +498,41 @@ __global__ __launch_bounds__(256) void hex8_reference(RefArgs A, RefStiffness K,
 #pragma unroll
         for (int px = 0; px < 3; ++px)
 #pragma unroll
-          for (int d = 0; d < 3; ++d) v[py][px][d] = u[ns * (plane + at[py][px]) + cs * I(d)];
+          for (int d = 0; d < 3; ++d) {
+            const int to = px == 1 && py == 1 ? 0 : py == 1 ? (px == 0 ? 1 : 2) : px == 1 ? (py == 0 ? 3 : 4)
+                                                 : 5 + (px == 0 ? 1 : 0) + (py == 0 ? 2 : 0);
+            q[to][d] = u[ns * (plane + at[py][px]) + cs * I(d)];
+          }
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q[5 + e][d] -= q[4 - (e >> 1)][d];   // along x, in the rows y - 1 and y + 1
+#pragma unroll
+        for (int i = 1; i < 5; ++i) q[i][d] -= q[0][d];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q[5 + e][d] -= q[2 - (e & 1)][d];
+      }
       if (z >= z0) {
         double ae[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) ae[e] = mat[below + at[1 - (e >> 1)][1 - (e & 1)]];
-        add(Z1{}, Z0{}, bot);
-        add(Z1{}, Z1{}, top);
+#pragma unroll
+        for (int i = 0; i < 9; ++i)
+#pragma unroll
+          for (int d = 0; d < 3; ++d) zq[i][d] = q[i][d] - zq[i][d];
+        add(Z1{}, Z0{}, zq, bot);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int d = 0; d < 3; ++d) top[0][e][d] = top[1][e][d] = 0.0;
+        add(Z0{}, Z1{}, q, top);
+        add(Z1{}, Z1{}, zq, top);
         if (z > z0) {
 #pragma unroll
           for (int d = 0; d < 3; ++d) {
             double acc = carry[d];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc = fma(ae[e], bot[e][d], acc);
+            for (int e = 0; e < 4; ++e) acc = fma(ae[e], bot[0][e][d] + bot[1][e][d], acc);
             const I idx = ns * (below + at[1][1]) + cs * I(d);
             if (CERT) {
               const double r = rhs[idx] - acc;
@@ -516,15 +547,18 @@ __global__ __launch_bounds__(256) void hex8_reference(RefArgs A, RefStiffness K,
         for (int d = 0; d < 3; ++d) {
           carry[d] = 0.0;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) carry[d] = fma(ae[e], top[e][d], carry[d]);
+          for (int e = 0; e < 4; ++e) carry[d] = fma(ae[e], top[0][e][d] + top[1][e][d], carry[d]);
         }
       }
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int d = 0; d < 3; ++d) bot[e][d] = top[e][d] = 0.0;
-      add(Z0{}, Z0{}, bot);
-      add(Z0{}, Z1{}, top);
+        for (int d = 0; d < 3; ++d) bot[0][e][d] = bot[1][e][d] = 0.0;
+      add(Z0{}, Z0{}, q, bot);
+#pragma unroll
+      for (int i = 0; i < 9; ++i)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) zq[i][d] = q[i][d];
     }
   }
   if (CERT) {
@@ -895,27 +929,28 @@ int launch_rowmarch(const pgj_grid& g, int L, int mode, RowArgsT<T>& A, hipStrea
 template int launch_rowmarch<double>(const pgj_grid&, int, int, RowArgsT<double>&, hipStream_t);
 template int launch_rowmarch<float>(const pgj_grid&, int, int, RowArgsT<float>&, hipStream_t);
 
-// 36 numbers of the element stiffness (RefStiffness).
+// The numbers of the element stiffness (RefStiffness).
 static RefStiffness ref_stiffness(const pgj_grid& g) {
   RefStiffness K{};
   const double h[3] = {g.hx, g.hy, g.hz};
-  auto mass = [&](int axis, int differ) { return differ ? h[axis] / 6 : h[axis] / 3; };
-  for (int df = 0; df < 8; ++df) {
-    double grad[3];   // integral of the product of the two nodes' derivatives along one axis
+  auto mass = [&](int axis, int other) { return other ? h[axis] / 6 : h[axis] / 2; };
+  for (int o = 0; o < 8; ++o) {
+    double grad[3];   // of the two nodes' derivatives along one axis
     for (int j = 0; j < 3; ++j) {
-      grad[j] = ((df >> j) & 1 ? -1.0 : 1.0) / h[j];
+      grad[j] = (o >> j) & 1 ? -1.0 / h[j] : 0.0;
       for (int k = 0; k < 3; ++k)
-        if (k != j) grad[j] *= mass(k, (df >> k) & 1);
+        if (k != j) grad[j] *= mass(k, (o >> k) & 1);
     }
     for (int i = 0; i < 3; ++i) {
-      K.diag[i][df] = g.lam * grad[i];
-      for (int j = 0; j < 3; ++j) K.diag[i][df] += g.mu * (i == j ? 2.0 : 1.0) * grad[j];
+      K.diag[i][o] = g.lam * grad[i];
+      for (int j = 0; j < 3; ++j) K.diag[i][o] += g.mu * (i == j ? 2.0 : 1.0) * grad[j];
     }
   }
   for (int k = 0; k < 3; ++k)
-    for (int differ = 0; differ < 2; ++differ) {
-      K.off_sum[k][differ] = (g.lam + g.mu) * 0.25 * mass(k, differ);
-      K.off_diff[k][differ] = (g.lam - g.mu) * 0.25 * mass(k, differ);
+    for (int other = 0; other < 2; ++other) {
+      K.lam[k][other] = 0.5 * g.lam * mass(k, other);
+      K.mu[k][other] = 0.5 * g.mu * mass(k, other);
+      K.both[k][other] = 0.25 * (g.lam + g.mu) * mass(k, other);
     }
   return K;
 }
