@@ -131,15 +131,16 @@ int pgj_diagonal_scale(const pgj_grid* g, const double* a, double alpha, double*
 int pgj_hex8_set_shape(const pgj_grid* g, int L, int es, int R, int W, int ZC, int plane);
 /* Radix plan of one FFT pass of the resident PCG iteration on the cube g in
  * precision es (8: FP64, 4: FP32): pass 0 forward x/y, 1 z with the Green
- * multiply, 2 inverse y/x; plan 0 takes radix-4 stages first (64 = 4 x 4 x 4),
- * plan 1 radix-8 stages first (64 = 8 x 8); for the z pass at 64^3, plan 2
+ * multiply, 2 inverse y/x; plan 0 (or -1) is the library's choice for that
+ * length (radix 8 first from 24 on; the z pass in registers where 16 divides n),
+ * plan 1 takes radix-8 stages first (64 = 8 x 8), plan 3 radix-4 stages first
+ * (64 = 4 x 4 x 4), both with the z pass in LDS; for the z pass at 64^3, plan 2
  * keeps the transforms and the Green multiply in registers (one LDS exchange per
- * transform). plan -1 leaves the pass to the library's choice for that length
- * (radix 8 first from 24 on; the z pass in registers where 16 divides n). The
+ * transform). The
  * choice holds for every later launch of that pass on any n^3 grid of that
  * precision (a graph keeps the kernels of its capture; a solver reads the plan
- * when it sets up its launches). get_plan writes the three passes' plans, 0
- * where none is set.
+ * when it sets up its launches). get_plan writes the three passes' plans, which
+ * may be set back as they are.
  * Counterpart of the reference's variant sweep
  * (solver/src/hex8_modal/gpu_study.py:174-222) for the FFT radix schedule. */
 int pgj_fft_set_plan(const pgj_grid* g, int es, int pass, int plan);

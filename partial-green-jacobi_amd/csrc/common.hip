@@ -40,7 +40,7 @@ std::map<PlanKey, int> g_plans;
 int fft_plan(int n, int es, int pass) {
   std::lock_guard<std::mutex> lock(g_plan_mutex);
   auto it = g_plans.find(PlanKey(n, es, pass));
-  return it == g_plans.end() ? -1 : it->second;
+  return it == g_plans.end() ? 0 : it->second;
 }
 
 bool tuned_shape(const pgj_grid& g, int L, int es, int* R, int* W, int* ZC, int* plane) {
@@ -78,10 +78,10 @@ extern "C" int pgj_hex8_get_shape(const pgj_grid* g, int L, int es, int* out5) {
 
 extern "C" int pgj_fft_set_plan(const pgj_grid* g, int es, int pass, int plan) {
   PGJ_REQUIRE(g && g->nx == g->ny && g->ny == g->nz && (es == 4 || es == 8) && pass >= 0 && pass <= 2 &&
-                  (plan == -1 || plan == 0 || plan == 1 || (plan == 2 && pass == 1 && g->nx == 64)),
-              "FFT plan needs a cube, es in {4,8}, pass in 0..2 and plan in {-1,0,1} (plan 2: the z pass at 64^3)");
+                  (plan == -1 || plan == 0 || plan == 1 || plan == 3 || (plan == 2 && pass == 1 && g->nx == 64)),
+              "FFT plan needs a cube, es in {4,8}, pass in 0..2 and plan in {-1,0,1,3} (plan 2: the z pass at 64^3)");
   std::lock_guard<std::mutex> lock(pgj::g_plan_mutex);
-  if (plan < 0)
+  if (plan <= 0)
     pgj::g_plans.erase(pgj::PlanKey(g->nx, es, pass));
   else
     pgj::g_plans[pgj::PlanKey(g->nx, es, pass)] = plan;
@@ -90,7 +90,7 @@ extern "C" int pgj_fft_set_plan(const pgj_grid* g, int es, int pass, int plan) {
 
 extern "C" int pgj_fft_get_plan(const pgj_grid* g, int es, int* out3) {
   PGJ_REQUIRE(g && (es == 4 || es == 8) && out3, "invalid FFT plan query");
-  for (int pass = 0; pass < 3; ++pass) out3[pass] = std::max(0, pgj::fft_plan(g->nx, es, pass));
+  for (int pass = 0; pass < 3; ++pass) out3[pass] = pgj::fft_plan(g->nx, es, pass);
   return PGJ_OK;
 }
 

@@ -98,7 +98,7 @@ constexpr int default_plan() {
 template <int N, typename R>
 int plan_of(int pass) {
   const int plan = fft_plan(N, int(sizeof(R)), pass);
-  return plan < 0 ? default_plan<N>() : plan;
+  return plan == 1 ? 1 : plan == 3 ? 0 : default_plan<N>();
 }
 
 // Global -> LDS copy of COUNT values in two phases, so that independent work
@@ -1057,7 +1057,7 @@ template <int N, typename R>
 static int zkc_of(const pgj_grid& g, int L) {
   using W = ZWidths<N, R>;
   const int plan = fft_plan(N, int(sizeof(R)), 1);
-  if (zreg<N>() && (plan == 2 || (plan < 0 && !(N == 64 && sizeof(R) == 8 && L == 1)))) return 0;
+  if (zreg<N>() && (plan == 2 || (plan == 0 && !(N == 64 && sizeof(R) == 8 && L == 1)))) return 0;
   return W::wide != W::def && zpass_wide(g, L, int(sizeof(R))) ? W::wide : W::def;
 }
 

@@ -37,8 +37,8 @@ struct RowMarch {
 bool tuned_shape(const pgj_grid& g, int L, int es, int* R, int* W, int* ZC, int* plane);
 
 // Radix plan of the compile-time FFT pass `pass` (0 forward xy, 1 z with the Green multiply, 2 inverse xy) of
-// the PCG iteration on an n^3 cube in precision es: 0 (radix 4 first), 1 (radix 8 first), -1 (not set: the
-// library's choice); set by pgj_fft_set_plan (the autotuner) and read at every launch of that pass.
+// the PCG iteration on an n^3 cube in precision es: 0 (not set: the library's choice), 1 (radix 8 first), 2 (z at 64^3
+// in registers), 3 (radix 4 first); set by pgj_fft_set_plan (the autotuner) and read at every launch of that pass.
 int fft_plan(int n, int es, int pass);
 
 // Row waves and planes per block of the FP64 plane-carry march with two x per lane (246 VGPRs: two waves per SIMD, so a

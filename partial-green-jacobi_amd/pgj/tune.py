@@ -90,7 +90,7 @@ class heterogeneous:
 
 
 def fft_plans(grid, es):
-    """The radix plans in use for the three passes of a cube in precision es."""
+    """The plans of the three passes of a cube in precision es: 0 for the library's choice, else the one set."""
     out = (_lib.c_int * 3)()
     _lib.check(_lib.lib().pgj_fft_get_plan(grid, es, out))
     return tuple(out)
