@@ -5,6 +5,7 @@
 // z / r.z / beta / p update. Semantics follow
 // solver/src/runtime/fi/source/femlib/batched/pcg.py:75-245 (eager loop),
 // :636-669 (compiled pre/post steps), :677-727 (latch kernels, best copy).
+#include <algorithm>
 #include <cmath>
 
 #include "fft_kernels.h"
@@ -17,13 +18,20 @@ namespace pgj {
 constexpr int kVecThreads = 256;
 constexpr double kPcgEps = 1e-30;  // pcg.py:112 (eps clamp of pAp and rz)
 
-// One value per thread up to 256 K values: a pass over a small vector is one round trip to memory, and every further value
-// of a thread would add its own (four values: certified solve 32^3 3.17 ms, one: 3.10; generic composite C^H 48^3
-// 16.7 and 16.2 ms).
-inline int vec_blocks(int64_t n) {
-  const int64_t b = (n + kVecThreads - 1) / kVecThreads;
-  return int(b < 1024 ? b : 1024);
+// Blocks per batch, at most 1024. One value per thread while the launch has at most 2048 blocks (a round of them): a pass
+// over a small vector is one round trip to memory, and every further value of a thread would add its own (four values:
+// certified solve 32^3 3.17 ms, one: 3.10; generic composite C^H 48^3 16.7 and 16.2 ms). Four values in larger launches,
+// because every block of an update reads all partials of its batch, which came to more than its values (pre-step, one
+// value against four: 6 x 262144 37 / 24 us, 64 x 98304 114 / 72, 3 x 331776 20.9 / 20.2, and 6 x 98304 17.8 / 18.4).
+inline int vec_blocks(int B, int64_t n) {
+  const int64_t one = std::min<int64_t>((n + kVecThreads - 1) / kVecThreads, 1024);
+  if (B * one <= 2048) return int(one);
+  return int(std::min<int64_t>((n + 4 * kVecThreads - 1) / (4 * kVecThreads), 1024));
 }
+
+// Batches whose latches the first block of pcg_best forms itself, four reductions at a time; more of them take a launch
+// of their own, which costs 2.5 us (256 batches of 3000 values: the pre-step 37 us with the latches in the block, 19).
+constexpr int kLatchBatches = 32;
 
 #define PGJ_GRID_LOOP(i, n) \
   _Pragma("unroll 4") for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < (n); i += int64_t(gridDim.x) * blockDim.x)
@@ -132,7 +140,8 @@ __global__ __launch_bounds__(kVecThreads) void pcg_update_ur(T* __restrict__ u, 
 
 // res = sqrt(|r|^2) / rhs_norm; improved = res < best_res (latched: and no stop recorded yet); best_res updated and u
 // copied to best_u where improved. Latched: state[0] (stop iteration) is set to `iteration` the first time every
-// res < tol; state[1] to 1 the first time every res < near_tol (near_tol > 0 only), by the first block. Every block
+// res < tol; state[1] to 1 the first time every res < near_tol (near_tol > 0 only), by the first block for up to
+// kLatchBatches batches, else by pcg_latch. Every block
 // forms its batch's residual from the partials (at most 1024, one pass of a wavefront), which costs it less than the
 // launch of its own that this test took before the copy: 2.9 of 24 us of vector kernels an iteration at 32^3.
 template <typename T>
@@ -155,7 +164,7 @@ __global__ __launch_bounds__(kVecThreads) void pcg_best(const T* __restrict__ u,
     const int64_t off = int64_t(b) * n;
     PGJ_GRID_LOOP(i, n) best_u[off + i] = u[off + i];
   }
-  if (!latched || blockIdx.x != 0 || b != 0) return;
+  if (!latched || B > kLatchBatches || blockIdx.x != 0 || b != 0) return;
   int ok = rv < tol, near = rv < near_tol;
   for (int k = 1 + wave; k < B; k += kVecThreads / 64) {
     const double v = sqrt(wave_reduce_partials(rr_part + int64_t(k) * nblk, nblk, 1)) / rhs_norm[k];
@@ -166,6 +175,22 @@ __global__ __launch_bounds__(kVecThreads) void pcg_best(const T* __restrict__ u,
   const int all_near = __syncthreads_and(near);
   if (threadIdx.x == 0) {
     if (stopped == 0 && all_ok) state[0] = iteration;
+    if (near_tol > 0.0 && state[1] == 0 && all_near) state[1] = 1;
+  }
+}
+
+// The latches of more than kLatchBatches batches from the residuals that pcg_best left. One block.
+__global__ __launch_bounds__(1024) void pcg_latch(int B, const double* res, int64_t* state, double tol, double near_tol,
+                                                  int64_t iteration) {
+  int ok = 1, near = 1;
+  for (int b = threadIdx.x; b < B; b += 1024) {
+    ok &= res[b] < tol;
+    near &= res[b] < near_tol;
+  }
+  const int all_ok = __syncthreads_and(ok);
+  const int all_near = __syncthreads_and(near);
+  if (threadIdx.x == 0) {
+    if (state[0] == 0 && all_ok) state[0] = iteration;
     if (near_tol > 0.0 && state[1] == 0 && all_near) state[1] = 1;
   }
 }
@@ -203,7 +228,7 @@ struct PcgWs {
   size_t pap, rr, rz, best_old, rz_old, stop_old, doubles;
 };
 PcgWs pcg_ws(int B, int64_t n) {
-  const size_t row = size_t(B) * vec_blocks(n);
+  const size_t row = size_t(B) * vec_blocks(B, n);
   PcgWs w{};
   w.rr = row;
   w.rz = 2 * row;
@@ -225,7 +250,7 @@ template <typename T>
 int pcg_start_t(int B, int64_t n, const T* rhs, const T* Ax, T* r, double* rhs_norm, double* ws, void* stream) {
   PGJ_REQUIRE(pcg_shape_ok(B, n) && rhs && r && rhs_norm && ws, "invalid pcg start arguments");
   hipStream_t s = as_stream(stream);
-  const int nblk = vec_blocks(n);
+  const int nblk = vec_blocks(B, n);
   hipLaunchKernelGGL(pcg_start<T>, dim3(nblk, B), dim3(kVecThreads), 0, s, rhs, Ax, r, n, ws);
   PGJ_LAUNCHED("pcg_start");
   hipLaunchKernelGGL(pcg_norms, batch_grid(B), dim3(256), 0, s, B, ws, nblk, rhs_norm);
@@ -237,7 +262,7 @@ template <typename T>
 int pcg_init_t(int B, int64_t n, const T* r, const T* z, T* p, double* rz, double* ws, void* stream) {
   PGJ_REQUIRE(pcg_shape_ok(B, n) && r && z && p && rz && ws, "invalid pcg init arguments");
   hipStream_t s = as_stream(stream);
-  const int nblk = vec_blocks(n);
+  const int nblk = vec_blocks(B, n);
   hipLaunchKernelGGL(pcg_dot<T>, dim3(nblk, B), dim3(kVecThreads), 0, s, r, z, nullptr, nullptr, n, int64_t(0), ws,
                      nullptr, nullptr);
   PGJ_LAUNCHED("pcg_dot");
@@ -258,7 +283,7 @@ int pcg_pre_step_t(int B, int64_t n, T* u, T* r, const T* p, const T* Ap, const 
                   state && ws,
               "invalid pcg pre-step arguments");
   hipStream_t s = as_stream(stream);
-  const int nblk = vec_blocks(n);
+  const int nblk = vec_blocks(B, n);
   const PcgWs w = pcg_ws(B, n);
   double *pap = ws + w.pap, *rr = ws + w.rr, *best_old = ws + w.best_old;
   int64_t* stop_old = reinterpret_cast<int64_t*>(ws + w.stop_old);
@@ -271,6 +296,10 @@ int pcg_pre_step_t(int B, int64_t n, T* u, T* r, const T* p, const T* Ap, const 
   hipLaunchKernelGGL(pcg_best<T>, dim3(nblk, B), dim3(kVecThreads), 0, s, u, best_u, n, B, rr, nblk, rhs_norm, best_old,
                      stop_old, res, best_res, improved, state, tol, near_tol, iteration, latched);
   PGJ_LAUNCHED("pcg_best");
+  if (latched && B > kLatchBatches) {
+    hipLaunchKernelGGL(pcg_latch, dim3(1), dim3(1024), 0, s, B, res, state, tol, near_tol, iteration);
+    PGJ_LAUNCHED("pcg_latch");
+  }
   return PGJ_OK;
 }
 
@@ -280,7 +309,7 @@ int pcg_post_step_t(int B, int64_t n, const T* r, T* z, const T* minv, int64_t m
   PGJ_REQUIRE(pcg_shape_ok(B, n) && r && z && p && rz && ws && (minv_stride == 0 || minv_stride == n),
               "invalid pcg post-step arguments");
   hipStream_t s = as_stream(stream);
-  const int nblk = vec_blocks(n);
+  const int nblk = vec_blocks(B, n);
   const PcgWs w = pcg_ws(B, n);
   double *part = ws + w.rz, *rz_old = ws + w.rz_old;
   hipLaunchKernelGGL(pcg_dot<T>, dim3(nblk, B), dim3(kVecThreads), 0, s, r, z, minv, z, n, minv_stride, part, rz,
@@ -359,7 +388,7 @@ extern "C" int pgj_pcg_fi_iterate(const pgj_grid* g, const double* a, const void
               "invalid pcg iterate arguments");
   hipStream_t s = as_stream(stream);
   const int64_t n = int64_t(g->nx) * g->ny * g->nz * 3;
-  const int nblk = vec_blocks(n);
+  const int nblk = vec_blocks(1, n);
   const PcgWs w = pcg_ws(1, n);
   double *rr = ws + w.rr, *best_old = ws + w.best_old, *rz_old = ws + w.rz_old;
   int64_t* stop_old = reinterpret_cast<int64_t*>(ws + w.stop_old);
