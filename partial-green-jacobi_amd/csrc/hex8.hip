@@ -988,13 +988,14 @@ int launch_reference(const pgj_grid& g, int L, RefArgs& A, bool cert, hipStream_
   return cert ? launch_reference_t<true>(g, L, A, s) : launch_reference_t<false>(g, L, A, s);
 }
 
-// Above 256 partial rows per load (more than 40^3 nodes) the means are reduced once per load instead of once per
-// block: 128^3, six loads, 1071 us of which all but 110 were the blocks' own reductions of 8192 rows; 64^3 22.9 us.
-// Below, the second launch costs more than it saves.
+// Where a launch has more than 1400 blocks of loads with more than 256 partial rows each (more than 40^3 nodes), the means
+// are reduced once per load instead of once per block, whose reductions grow with the square of the rows. Projection of
+// one load, three, six, by the blocks / in a launch before them (us): 64^3 18.2 / 21.0, 29.9 / 25.0, 51.1 / 39.3, 45^3
+// 18.2 / 20.6, 18.3 / 20.8, 26.9 / 22.2, 80^3 28.7 / 21.4, 64.8 / 40.2, 121 / 68, 128^3 207 / 52, 621 / 135, 1270 / 319.
 int launch_subtract_mean(const pgj_grid& g, int L, double* v, double* part, int soa, hipStream_t s) {
   const int64_t N = int64_t(g.nx) * g.ny * g.nz;
   const int nblk = int((N + 255) / 256);
-  if (nblk > 256) {
+  if (nblk > 256 && int64_t(nblk) * L > 1400) {
     hipLaunchKernelGGL(component_means, dim3(L), dim3(256), 0, s, N, part, nblk);
     PGJ_LAUNCHED("component_means");
     hipLaunchKernelGGL(subtract_mean<true>, dim3(nblk, L), dim3(256), 0, s, v, N, part, nblk, soa);
