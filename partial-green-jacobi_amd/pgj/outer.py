@@ -88,7 +88,8 @@ class PaperOuter(_Fields):
 
     def physical(self):
         if self.fused:
-            _lib.call('pgj_cone_physical', self.n, _lib.ptr(self.x), *self._stencil(), _lib.ptr(self.hs), self.beta,
+            x = self.x.contiguous()
+            _lib.call('pgj_cone_physical', self.n, _lib.ptr(x), *self._stencil(), _lib.ptr(self.hs), self.beta,
                       self.eta, self.emin, _lib.ptr(self.t), _lib.ptr(self.ph), _lib.ptr(self.dp), _lib.ptr(self.a),
                       _lib.stream())
             return
