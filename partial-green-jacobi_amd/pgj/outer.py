@@ -66,12 +66,13 @@ class PaperOuter(_Fields):
         off, w = cone_stencil(rmin)
         self.offsets = torch.tensor(off, device=device).contiguous()
         self.weights = torch.tensor(w, dtype=torch.float64, device=device)
-        self._alloc(n, ['x', 'ph', 'dp', 'a', 'energy', 'new', 'g', 'dv', 'ratio', 't', 'hs', 'trial_ph',
-                        'trial_dp', 'trial_a', 'tmp'], device)
-        self.bounds = torch.zeros(4, dtype=torch.float64, device=device)
         lib = _lib.lib()
         self.reach = max(0, math.ceil(rmin) - 1)
         self.fused = self.reach <= lib.pgj_cone_max_reach()   # wider stencils: one launch per filter, projection, ...
+        self._alloc(n, ['x', 'ph', 'dp', 'a', 'energy', 'new', 'g', 'dv', 'ratio', 't', 'hs'], device)
+        if not self.fused:
+            self._alloc(n, ['trial_ph', 'trial_dp', 'trial_a', 'tmp'], device)
+        self.bounds = torch.zeros(4, dtype=torch.float64, device=device)
         self.rounds_ws = torch.empty(lib.pgj_cone_rounds_ws_bytes(n) // 8, dtype=torch.float64, device=device)
         self.root = torch.empty(2 * n ** 3 if self.fused else 0, dtype=torch.float64, device=device)
         self.raw_filter(torch.ones_like(self.x), self.hs)
@@ -186,12 +187,13 @@ class GaussianOuter(_Fields):
         if self.radius > 4 * n:
             raise ValueError('Gaussian radius exceeds the supported range')
         self.weights = torch.tensor(gaussian_weights(sigma, self.radius), dtype=torch.float64, device=device)
-        self._alloc(n, ['x', 'ph', 'dp', 'a', 'energy', 'new', 'g', 'dv', 'ratio', 'tmp1', 'tmp2', 't', 'trial_ph',
-                        'trial_dp', 'trial_a', 'gin'], device)
-        self.beta = 1.0
-        self.bounds = torch.zeros(2, dtype=torch.float64, device=device)
         lib = _lib.lib()
         self.fused = bool(lib.pgj_gauss_fused(n, self.radius))
+        self._alloc(n, ['x', 'ph', 'dp', 'a', 'energy', 'new', 'g', 'dv', 'ratio', 'tmp1', 'tmp2', 't', 'gin'], device)
+        if not self.fused:
+            self._alloc(n, ['trial_ph', 'trial_dp', 'trial_a'], device)
+        self.beta = 1.0
+        self.bounds = torch.zeros(2, dtype=torch.float64, device=device)
         self.rounds_ws = torch.empty(lib.pgj_gauss_rounds_ws_bytes(n) // 8, dtype=torch.float64, device=device)
         self.physical_graph = self.update_graph = None
 
