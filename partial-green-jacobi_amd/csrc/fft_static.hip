@@ -1047,12 +1047,13 @@ bool zpass_wide(const pgj_grid& g, int L, int es) {
 }
 
 // The z pass of a workspace: 0 = in registers (fz_reg), else the chunk width of the LDS pass. In registers by default
-// wherever the columns divide into its waves; the LDS pass by an explicit radix plan, for the ragged cube, and for one
-// FP64 load at 64^3, whose 264 waves leave most SIMDs idle on a long chain of their own. Graph-replayed launches of one,
-// three and six loads, LDS -> registers (us): 32^3 FP64 6.2 / 7.2 / 9.2 -> 6.4 / 6.5 / 7.0, 48^3 FP64 8.4 / 12.9 / 18.8 ->
-// 7.4 / 11.7 / 16.1, 64^3 FP64 11.9 / 20.5 / 30.6 -> 13.3 / 18.7 / 26.1, 64^3 FP32 9.5 / 15.4 / 23.8 -> 8.8 / 12.8 / 18.4,
-// 96^3 FP64 31.7 / 68.6 / 127 -> 28.2 / 60.9 / 114, 96^3 FP32 23.7 / 43 / 73 -> 23.3 / 34.4 / 63.8, 128^3 FP64
-// 61 / 151 / 295 -> 58 / 140 / 275, 128^3 FP32 49 / 99 / 175 -> 38 / 79 / 163.
+// wherever the columns divide into its waves; the LDS pass by an explicit radix plan (1 or 3), for the ragged cube, and for
+// one FP64 load at 64^3, whose 264 waves leave most SIMDs idle on a long chain of their own. That exception is a table of
+// one entry, not a criterion: the other lone loads are faster in registers but for 32^3 FP64, where the two differ by 3 %.
+// Graph-replayed launches of one, three and six loads, LDS -> registers (us): 32^3 FP64 6.2 / 7.2 / 9.2 -> 6.4 / 6.5 / 7.0,
+// 48^3 FP64 8.4 / 12.9 / 18.8 -> 7.4 / 11.7 / 16.1, 64^3 FP64 11.9 / 20.5 / 30.6 -> 13.3 / 18.7 / 26.1, 64^3 FP32
+// 9.5 / 15.4 / 23.8 -> 8.8 / 12.8 / 18.4, 96^3 FP64 31.7 / 68.6 / 127 -> 28.2 / 60.9 / 114, 96^3 FP32 23.7 / 43 / 73 ->
+// 23.3 / 34.4 / 63.8, 128^3 FP64 61 / 151 / 295 -> 58 / 140 / 275, 128^3 FP32 49 / 99 / 175 -> 38 / 79 / 163.
 template <int N, typename R>
 static int zkc_of(const pgj_grid& g, int L) {
   using W = ZWidths<N, R>;

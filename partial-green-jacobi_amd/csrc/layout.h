@@ -43,12 +43,13 @@ int fft_plan(int n, int es, int pass);
 
 // Row waves and planes per block of the FP64 plane-carry march with two x per lane (246 VGPRs: two waves per SIMD, so a
 // CU holds one block of 4 row waves + halo or two of 2 + halo; either way a round of blocks covers 1024 rows). A block
-// takes ZC + 1 layers, so the shape with the fewest rounds (ZC + 1) wins; 4 row waves repeat less of the halo, but pay only
-// over 16 planes or more and with a last round that is 3/4 full (a CU holds no second block of them). PCG pass, three loads (one load), 4 x 16 /
-// 4 x 32 / 2 x 8 / 2 x 4 row waves x planes: 96^3 78 / 74 / 81 / 82 (- / - / 39 / 36) us, 128^3 128 / 150 / 150 / -
-// (44 / - / 50 / -); the node march took 92 (41) and 160 (51) at its best shapes, 100 (42) and 161 (58) by its rule. The apply by this rule against the node march by
-// the old one, one / three / six loads: 66^3 22 / 48 / 92 against 27 / 58 / 111, 100^3 34 / 92 / 176 against
-// 43 / 111 / 217, 128^3 45 / 131 / 248 against 58 / 166 / 329 us.
+// takes ZC + 1 layers, so the shape with the fewest rounds (ZC + 1) wins; 4 row waves repeat less of the halo, but pay
+// only over 16 planes or more and with a last round that is 3/4 full (a CU holds no second block of them). The count of
+// CUs is the MI355X's 256. PCG pass, three loads (one load), 4 x 16 / 4 x 32 / 2 x 8 / 2 x 4 row waves x planes: 96^3
+// 78 / 74 / 81 / 82 (- / - / 39 / 36) us, 128^3 128 / 150 / 150 / - (44 / - / 50 / -); the node march took 92 (41) and
+// 160 (51) at its best shapes, 100 (42) and 161 (58) by its rule. The apply by this rule against the node march by the
+// old one, one / three / six loads: 66^3 22 / 48 / 92 against 27 / 58 / 111, 100^3 34 / 92 / 176 against 43 / 111 / 217,
+// 128^3 45 / 131 / 248 against 58 / 166 / 329 us.
 inline void pair64_shape(int ny, int nz, int L, int* W, int* ZC) {
   int64_t best = -1;
   for (int w : {4, 2, 1}) {
@@ -68,11 +69,11 @@ inline void pair64_shape(int ny, int nz, int L, int* W, int* ZC) {
   }
 }
 
-// Shape preferences (R, W, ZC) for L loads per launch. ZC (planes marched by
-// one block) is the largest of 16, 8, 4, 2, 1 dividing nz that still gives
-// at least 192 blocks: longer marches re-read fewer halo planes, but the
-// launch must keep most of the 256 CUs busy. A tuned shape replaces the
-// preferences.
+// Shape preferences (R, W, ZC) for L loads per launch. Where no rule below
+// sets it, ZC (planes marched by one block) is the largest of 16, 8, 4, 2
+// dividing nz that still gives 768 blocks, three per CU: longer marches
+// re-read fewer halo planes, but the launch must keep the CUs busy. A tuned
+// shape replaces the preferences.
 inline RowMarch rowmarch_config(const pgj_grid& g, int L, int es = 8) {
   RowMarch c{};
   const int nx = g.nx, ny = g.ny, nz = g.nz;
@@ -273,11 +274,13 @@ inline bool stages_fit(const Factors& f, int lines, int threads) {
 
 constexpr int kMinChunk = 4;  // frequency columns per block of the runtime z pass: 4, 8 or 16
 
-// Rows of z pass partials per load are partial_chunks(g) ny: as many as any z pass of the grid has blocks (the compile-time
-// ones: fft_static.hip, ZWidths and ZReg; the runtime one at most ceil(ny nkx / kMinChunk)).
+// Rows of z pass partials per load are partial_chunks(g) ny, at least as many as any z pass of the grid has blocks: the
+// compile-time LDS ones N / 2 / kc chunks of N rows and N / kc Nyquist blocks of kc columns or more (kc: the narrowest of
+// ZWidths in fft_static.hip), the register-resident ones half as many or fewer of 8 columns, the runtime one at most
+// ceil(ny nkx / kMinChunk).
 inline int partial_chunks(const pgj_grid& g) {
   int kc = kMinChunk;
-  if (static_cube(g)) kc = g.nx == 16 ? 3 : g.nx == 96 ? 6 : g.nx == 128 ? 5 : 4;
+  if (static_cube(g)) kc = g.nx == 96 ? 6 : g.nx == 128 ? 8 : 4;
   return (g.nx / 2 + 1 + kc - 1) / kc;
 }
 

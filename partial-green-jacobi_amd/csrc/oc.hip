@@ -8,7 +8,8 @@
 //    tanh projection, sqrt OC with fixed bisection count
 //    (exp/asg_gpu_resident_20261103/outer.cu:7-37, outer.py:26-44).
 // Floating-point contraction is disabled so products and sums round like the
-// reference's --fmad=false builds and numpy.
+// reference's --fmad=false builds and numpy, except where an fma is written out:
+// the taps of the fused cone passes, which round once per term instead of twice.
 #include <cmath>
 
 #include "layout.h"
@@ -510,7 +511,9 @@ __global__ void gauss_bisect_kernel(const double* vpart, int nblk, int64_t N, do
 // LDS with their y halo. Each line is summed in gauss_axis_kernel's order. A bisection round (candidate, three axis
 // passes, projection, bisection: six launches, bound by their issue from the host at 38 us a round) is two.
 constexpr int kGaussCols = 16;
-// Rows of a strip: 8 up to n = 48, where 16 leave a launch with a quarter block per CU (the loop at 32^3: 524 -> 490 us).
+// Rows of a strip: 8 up to n = 48, where 16 leave a launch with half a block per CU or less. The update with 8 and 16 rows
+// (us): 24^3 399 / 443, 32^3 432 / 472, 40^3 564 / 627, 48^3 666 / 650; above the line 56^3 779 / 837, 64^3 795 / 914,
+// 96^3 1932 / 2108, so the line could lie higher.
 __host__ __device__ inline int gauss_rows(int n) { return n <= 48 ? 8 : 16; }
 
 // Weighted symmetric sum at `i` of a periodic line of n values with stride `st` in LDS (radius <= n).
@@ -575,7 +578,8 @@ __global__ __launch_bounds__(256) void gauss_z_kernel(const double* x, const dou
     z[k * NN + p] = gauss_line(col + c, kGaussCols, k, n, w, radius);
 }
 
-// y and x passes of gauss_rows(n) rows of a z-plane (inv: 2^32 / n rounded up, for the division by n). VOLUME: the projected density's sum per block instead of the field.
+// y and x passes of gauss_rows(n) rows of a z-plane (inv: 2^32 / n rounded up, for the division by n). VOLUME: the
+// projected density's sum per block instead of the field.
 template <bool VOLUME>
 __global__ __launch_bounds__(256) void gauss_yx_kernel(const double* z, const double* w, int radius, int n,
                                                        unsigned inv, double beta, double* y, double* vpart) {
@@ -723,8 +727,8 @@ extern "C" int pgj_gauss_filter(int n, const double* x, const double* weights, i
   const int64_t N = int64_t(n) * n * n;
   hipStream_t s = as_stream(stream);
   if (pgj_gauss_fused(n, radius) && tmp1 != y) {   // y may alias x or tmp1, as before
-    hipLaunchKernelGGL(gauss_z_kernel<false>, dim3(gauss_columns(n)), dim3(256), size_t(n) * kGaussCols * 8, s, x, nullptr, 0.0, 0.0, nullptr, nullptr, 0, nullptr, weights, radius,
-                       n, nullptr, tmp1);
+    hipLaunchKernelGGL(gauss_z_kernel<false>, dim3(gauss_columns(n)), dim3(256), size_t(n) * kGaussCols * 8, s, x,
+                       nullptr, 0.0, 0.0, nullptr, nullptr, 0, nullptr, weights, radius, n, nullptr, tmp1);
     hipLaunchKernelGGL(gauss_yx_kernel<false>, dim3(gauss_strips(n), n), dim3(256), gauss_lds(n, radius), s, tmp1,
                        weights, radius, n, gauss_inv(n), 0.0, y, nullptr);
     PGJ_LAUNCHED("gauss_filter");

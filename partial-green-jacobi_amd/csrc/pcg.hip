@@ -33,8 +33,9 @@ inline int vec_blocks(int B, int64_t n) {
 // of their own, which costs 2.5 us (256 batches of 3000 values: the pre-step 37 us with the latches in the block, 19).
 constexpr int kLatchBatches = 32;
 
-#define PGJ_GRID_LOOP(i, n) \
-  _Pragma("unroll 4") for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < (n); i += int64_t(gridDim.x) * blockDim.x)
+#define PGJ_GRID_LOOP(i, n)                                                                      \
+  _Pragma("unroll 4") for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < (n); \
+                           i += int64_t(gridDim.x) * blockDim.x)
 
 // r = rhs - Ax (Ax may be null: r = rhs); rhs_part[b][blk] = partial |rhs_b|^2.
 // Vectors are T (FP64 or FP32); sums, partials and per-batch scalars are FP64.
@@ -197,8 +198,9 @@ __global__ __launch_bounds__(1024) void pcg_latch(int B, const double* res, int6
 
 // beta = rz_new / max(rz_old, eps); p = z + beta p; rz = rz_new.
 template <typename T>
-__global__ __launch_bounds__(kVecThreads) void pcg_update_p(const T* __restrict__ z, T* __restrict__ p, int64_t n, const double* rz_part,
-                                                            int nblk, const double* rz_old, double* rz) {
+__global__ __launch_bounds__(kVecThreads) void pcg_update_p(const T* __restrict__ z, T* __restrict__ p, int64_t n,
+                                                            const double* rz_part, int nblk, const double* rz_old,
+                                                            double* rz) {
   const int b = blockIdx.y;
   const double rzn = wave_reduce_partials(rz_part + int64_t(b) * nblk, nblk, 1);
   const T beta = T(rzn / fmax(rz_old[b], kPcgEps));
